@@ -200,7 +200,7 @@ __device__ inline double drag_pouliquen(const Params& p, double hn, double u, do
 }
 
 // DragClosure family (src/Closures.f90:365-558).
-__device__ inline double drag(const Params& p, double hn, double u, double v, double psi, double bx,
+__device__ __attribute__((noinline)) double drag(const Params& p, double hn, double u, double v, double psi, double bx,
                               double by, double gam) {
     switch (p.drag) {
     case KST_DRAG_CHEZY: return drag_chezy(p, u, v, bx, by);

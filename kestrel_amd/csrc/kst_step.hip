@@ -67,6 +67,10 @@ struct Ctrl {
     long long work[16];        // launches that did work, per kernel (KW_*)
     int cur;                   // mixed precision: u^n is in S0 (0) or S0b (1)
     double next_t;             // NextFluxSeriesTime of t, kept with t
+    // every vertex bt is +0 and stays so (no morphodynamics): bt of the cells
+    // and faces is 0 and a face's CorrectSlopes bed is its b0, and the stage
+    // kernels read neither
+    int flat;
     // CFL minima: first hydraulic operator stages 1..3, then the second
     // operator of a Strang step stages 1..3
     CflSlot slot[6];
@@ -229,7 +233,7 @@ __device__ __forceinline__ ConstArg<Ctrl>* ctrl_view(const DevT& d) {
 // Has the member names of Ctrl, so that step_dt and first_operator_ok take
 // it as they take the control block.
 struct CtrlSnap {
-    int status, n_active, mref, cur, ncand;
+    int status, n_active, mref, cur, ncand, flat;
     double t, tend, next_t, dt_retry;
     struct {
         unsigned long long bits;
@@ -240,6 +244,7 @@ template <class CtrlP>
 __device__ __forceinline__ CtrlSnap snap_ctrl(CtrlP c) {
     CtrlSnap s;
     s.status = c->status; s.n_active = c->n_active; s.mref = c->mref; s.cur = c->cur; s.ncand = c->ncand;
+    s.flat = c->flat;
     s.t = c->t; s.tend = c->tend; s.next_t = c->next_t; s.dt_retry = c->dt_retry;
 #pragma unroll
     for (int k = 0; k < 6; ++k) s.slot[k].bits = c->slot[k].bits;
@@ -336,8 +341,9 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
         if (rt == KST_LIMITER_MINMOD1) return lim<KST_LIMITER_MINMOD1>(rt, a, b);
         return (T)limiter(rt, (double)a, (double)b);
     } else if (LIM == KST_LIMITER_MINMOD2) {
-        const T th = T(1.3);
-        const T m = fmin(th * fabs(a), fmin(th * fabs(b), T(0.5) * fabs(a + b)));
+        // min(th |a|, th |b|) is th min(|a|, |b|) to the bit (rounding is
+        // monotonic)
+        const T m = fmin(T(1.3) * fmin(fabs(a), fabs(b)), T(0.5) * fabs(a + b));
         return (a * b <= T(0)) ? T(0) : copysign(m, a);
     } else if (LIM == KST_LIMITER_MINMOD1) {
         const T m = fmin(fabs(a), fabs(b));
@@ -349,34 +355,75 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
 
 // Working set of one sub-block.  With MIX the per-cell Hnpsi, u, v and the
 // fluxes other than the hydrostatic one (q = 4, in fx4/fy4) are float.
-// BY: the sub-block's height (B or B/2); the region is RW x (BY + 4) cells.
+// BY: the sub-block's height (B or B/4); the region is RW x (BY + 4) cells.
 // ONED: a 1D grid (one row of cells), which also keeps the conserved rhoHnv
 // for its x-face reconstruction.
-template <int NQ, bool MIX = false, int BY = B, bool ONED = false>
-struct SmemT {
+// The fluxes of a 16 x 16 sub-block take the place of what the face pass
+// reads (ALIAS: each thread holds its faces' fluxes over the barrier between
+// the two), which leaves room for four workgroups on a CU instead of three
+// (48 -> 26 KB a workgroup); the 16 x 4 shape keeps them apart, since its
+// launches never fill a CU and the extra barrier would lengthen each.
+template <int NQ, bool MIX, int BY, bool ONED>
+struct RegionT {
     using FT = typename std::conditional<MIX, float, double>::type;
-    static constexpr int by = BY;
-    static constexpr bool oned = ONED;
     static constexpr int NR = RW * (BY + 4);       // region cells
-    static constexpr int NFX = (B + 1) * BY;       // x-faces
-    static constexpr int NFY = B * (BY + 1);       // y-faces
     double w[NR];
     FT h[NR], u[NR], v[NR];
     double rho[NR];
     double rv[ONED ? NR : 1];  // 1D: the conserved rhoHnv
-    double wst[NR];          // w behind the ghost tiles' stored face values (their tileContainer w)
     double xbed[BY][B + 3];  // CorrectSlopes bed of x-faces -1..B+1 of each row (relative)
     double ybed[B][BY + 3];  // CorrectSlopes bed of y-faces -1..BY+1 of each column
     double xside[2][BY];     // the W / E tile's own bed at this tile's edge x-faces
     double yside[2][B];      // the S / N tile's own bed at this tile's edge y-faces
-    int gidx[NR];
-    uint8_t act[NR];
+};
+
+template <int NQ, bool MIX, int BY>
+struct FluxT {
+    using FT = typename std::conditional<MIX, float, double>::type;
+    static constexpr int NFX = (B + 1) * BY;       // x-faces
+    static constexpr int NFY = B * (BY + 1);       // y-faces
     FT fx[NQ][NFX];          // hw, hru, hrv, hh, g (, pu, pv with eddy viscosity)
     FT fy[NQ][NFY];
     double fx4[MIX ? NFX : 1], fy4[MIX ? NFY : 1];
+};
+
+template <class A, class C, bool ALIAS>
+struct PairT {
+    A r;
+    C f;
+};
+template <class A, class C>
+struct PairT<A, C, true> {
+    union {
+        A r;
+        C f;
+    };
+};
+
+template <int NQ_, bool MIX = false, int BY = B, bool ONED = false>
+struct SmemT : PairT<RegionT<NQ_, MIX, BY, ONED>, FluxT<NQ_, MIX, BY>, BY == B> {
+    using FT = typename std::conditional<MIX, float, double>::type;
+    static constexpr bool alias = BY == B;
+    static constexpr int by = BY;
+    static constexpr bool oned = ONED;
+    static constexpr int NQ = NQ_;
+    static constexpr int NFX = FluxT<NQ_, MIX, BY>::NFX, NFY = FluxT<NQ_, MIX, BY>::NFY;
+    // stage 2: the owned cells' u1 momenta, over the face pass
+    double mom[2][alias && !MIX ? B * BY : 1];
     double red[STAGE_NT / 64];
-    int tile, bx0, by0, bxa, bya, skip, cur, more;
+    int tile, bx0, by0, bxa, bya, skip, cur, more, flat;
+    int solids;              // some cell of the region has Hnpsi other than 0
+    int nact;                // bits 0..3: the W, E, S, N neighbour tile is active
     double dt, tstage, tgrid;
+};
+
+// One face's fluxes: hw, hru, hrv, hh, g (, pu, pv), in a thread's registers
+// until they go to LDS.  With MIX all but g are float.
+template <bool MIX>
+struct FaceFlux {
+    using FT = typename std::conditional<MIX, float, double>::type;
+    FT q[7];
+    double g;
 };
 
 __device__ __forceinline__ int rg(int rx, int ry) { return (ry + 2) * RW + (rx + 2); }
@@ -400,28 +447,57 @@ struct FaceTopo {
     double bp, g, b0, bt, np, nm;
 };
 
+// Element idx of an array whose address is uniform over the wave: base in
+// scalar registers, a 32-bit byte offset in a vector register (one
+// instruction instead of a 64-bit address computation per load; every array
+// of a handle that fits the device is shorter than 4 GB, checked in kst_create).
+__device__ __forceinline__ double ld(const double* base, unsigned idx) {
+    return *(const double*)((const char*)base + idx * 8u);
+}
+
 template <bool YDIR, bool CFL, class DevT>
 __device__ __forceinline__ FaceTopo load_face_topo_at(const DevT& d, const Params& p, int t, int bx0,
-                                                      int by0, int fi, int fj) {
+                                                      int by0, int fi, int fj, bool flat) {
     const int fpos = (YDIR ? by0 : bx0) + fi;
-    FaceTopo f;
-    int fidx;
+    FaceTopo f{};
     if (!YDIR) {
-        fidx = t * p.NFX + (by0 + fj) * (p.nx + 1) + fpos;
-        f.bp = d.T.xby[fidx]; f.g = d.T.xgam[fidx]; f.b0 = d.xb0[fidx]; f.bt = d.T.xbt[fidx];
+        const unsigned k = t * p.NFX + (by0 + fj) * (p.nx + 1) + fpos;
+        f.bp = ld(d.T.xby, k); f.g = ld(d.T.xgam, k);
+        if (!flat) { f.b0 = ld(d.xb0, k); f.bt = ld(d.T.xbt, k); }
+        if (CFL) { f.np = ld(d.T.xnp, k); f.nm = ld(d.T.xnm, k); }
     } else {
-        fidx = t * p.NFY + fpos * p.nx + (bx0 + fj);
-        f.bp = d.T.ybx[fidx]; f.g = d.T.ygam[fidx]; f.b0 = d.yb0[fidx]; f.bt = d.T.ybt[fidx];
+        const unsigned k = t * p.NFY + fpos * p.nx + (bx0 + fj);
+        f.bp = ld(d.T.ybx, k); f.g = ld(d.T.ygam, k);
+        if (!flat) { f.b0 = ld(d.yb0, k); f.bt = ld(d.T.ybt, k); }
+        if (CFL) { f.np = ld(d.T.ynp, k); f.nm = ld(d.T.ynm, k); }
     }
-    f.np = CFL ? (YDIR ? d.T.ynp : d.T.xnp)[fidx] : 0.0;
-    f.nm = CFL ? (YDIR ? d.T.ynm : d.T.xnm)[fidx] : 0.0;
     return f;
 }
 
-template <bool YDIR, bool CFL, typename Smem, class DevT>
-__device__ __forceinline__ FaceTopo load_face_topo(const DevT& d, const Params& p, const Smem& s,
-                                                   int fi, int fj) {
-    return load_face_topo_at<YDIR, CFL>(d, p, s.tile, s.bx0, s.by0, fi, fj);
+// What a face needs of its sub-block (uniform over the workgroup): the tile
+// and its position in it, whether the neighbour tiles are active, and whether
+// the bed is flat (Ctrl::flat).
+struct Block {
+    int t, bx0, by0, nact;
+    bool flat;
+    bool solids;             // some cell of the region has Hnpsi other than 0
+    const double* Un;        // u^n of the step (a ghost cell's stored w)
+};
+
+// A cell beside an edge face that lies in a non-active neighbour tile: its
+// stored w slope and tileContainer w (src/UpdateTiles.f90:669-750).
+struct GhostCell {
+    double slope, w;
+};
+template <bool YDIR, class DevT>
+__device__ __forceinline__ GhostCell ghost_cell(const DevT& d, const Params& p, const Block& b, bool high,
+                                                int fj) {
+    const int nn = YDIR ? p.ny : p.nx, K = high ? nn : -1;
+    int tc, ci, cj;
+    if (YDIR) map_cell(p, b.t, b.bx0 + fj, K, tc, ci, cj);
+    else map_cell(p, b.t, K, b.by0 + fj, tc, ci, cj);
+    const int gi = tc * p.NC + cj * p.nx + ci;
+    return {(YDIR ? d.gsy : d.gsx)[gi], b.Un[gi]};
 }
 
 // Fused work of one x- or y-face (CalculateLimitedDerivs + Reconstruct +
@@ -429,77 +505,88 @@ __device__ __forceinline__ FaceTopo load_face_topo(const DevT& d, const Params& 
 // Along the face normal the four cells are c[-2], L=c[-1], R=c[0], c[1];
 // fi is the face position along the normal, fj the row (x) / column (y).
 template <bool YDIR, bool VISC, int LIM, bool CFL, typename Smem, class DevT>
-__device__ __forceinline__ void face_flux(const DevT& d, const Params& p, Smem& s, int fi, int fj,
-                                          double& cfl_min, const FaceTopo& ft) {
+__device__ __forceinline__ void face_flux(const DevT& d, const Params& p, const Smem& sm, const Block& blk, int fi,
+                                          int fj, double& cfl_min, const FaceTopo& ft, FaceFlux<false>& F) {
+    const auto& s = sm.r;
     int iLL, iL, iR, iRR;
     if (!YDIR) { iLL = rg(fi - 2, fj); iL = rg(fi - 1, fj); iR = rg(fi, fj); iRR = rg(fi + 1, fj); }
     else       { iLL = rg(fj, fi - 2); iL = rg(fj, fi - 1); iR = rg(fj, fi); iRR = rg(fj, fi + 1); }
     const double dxr = YDIR ? p.dyr : p.dxr;
     const double dx = YDIR ? p.dy : p.dx;
-    const bool actL = s.act[iL], actR = s.act[iR];
     const int nn = YDIR ? p.ny : p.nx;
-    const int fpos = (YDIR ? s.by0 : s.bx0) + fi;     // face index within the tile, 0..nn
+    const int fpos = (YDIR ? blk.by0 : blk.bx0) + fi;     // face index within the tile, 0..nn
+    // a cell beyond the tile's edge is active if that neighbour tile is
+    const bool actL = fpos > 0 || (blk.nact & (YDIR ? 4 : 1));
+    const bool actR = fpos < nn || (blk.nact & (YDIR ? 8 : 2));
 
     // --- slopes (CalculateLimitedDerivs, src/HydraulicRHS.f90:181-386);
     // non-active tiles keep their stored w slope and zero slopes otherwise.
     const double wLL = s.w[iLL], wL = s.w[iL], wR = s.w[iR], wRR = s.w[iRR];
-    const double* gs = YDIR ? d.gsy : d.gsx;
-    const double sLw = actL ? dxr * lim<LIM>(p.limiter, wR - wL, wL - wLL) : gs[s.gidx[iL]];
-    const double sRw = actR ? dxr * lim<LIM>(p.limiter, wRR - wR, wR - wL) : gs[s.gidx[iR]];
-    const double hLL = s.h[iLL], hL = s.h[iL], hR = s.h[iR], hRR = s.h[iRR];
-    const double sLh = actL ? dxr * lim<LIM>(p.limiter, hR - hL, hL - hLL) : 0.0;
-    const double sRh = actR ? dxr * lim<LIM>(p.limiter, hRR - hR, hR - hL) : 0.0;
+    double sLw = dxr * lim<LIM>(p.limiter, wR - wL, wL - wLL);
+    double sRw = dxr * lim<LIM>(p.limiter, wRR - wR, wR - wL);
+    double wLc = wL, wRc = wR;
+    if (!actL) { const GhostCell g = ghost_cell<YDIR>(d, p, blk, false, fj); sLw = g.slope; wLc = g.w; }
+    if (!actR) { const GhostCell g = ghost_cell<YDIR>(d, p, blk, true, fj); sRw = g.slope; wRc = g.w; }
+    // the other fields' slopes are 0 there: 1/dx is
+    const double dxL = actL ? dxr : 0.0, dxR = actR ? dxr : 0.0;
+    // (s 0.5) dx is s (0.5 dx) to the bit
+    const double hdx = 0.5 * dx;
     const double uLL = s.u[iLL], uL = s.u[iL], uR = s.u[iR], uRR = s.u[iRR];
-    const double sLu = actL ? dxr * lim<LIM>(p.limiter, uR - uL, uL - uLL) : 0.0;
-    const double sRu = actR ? dxr * lim<LIM>(p.limiter, uRR - uR, uR - uL) : 0.0;
+    const double sLu = dxL * lim<LIM>(p.limiter, uR - uL, uL - uLL);
+    const double sRu = dxR * lim<LIM>(p.limiter, uRR - uR, uR - uL);
     const double vLL = s.v[iLL], vL = s.v[iL], vR = s.v[iR], vRR = s.v[iRR];
-    const double sLv = actL ? dxr * lim<LIM>(p.limiter, vR - vL, vL - vLL) : 0.0;
-    const double sRv = actR ? dxr * lim<LIM>(p.limiter, vRR - vR, vR - vL) : 0.0;
-    const double rLL = s.rho[iLL], rL = s.rho[iL], rR = s.rho[iR], rRR = s.rho[iRR];
-    const double sLr = actL ? dxr * lim<LIM>(p.limiter, rR - rL, rL - rLL) : 0.0;
-    const double sRr = actR ? dxr * lim<LIM>(p.limiter, rRR - rR, rR - rL) : 0.0;
+    const double sLv = dxL * lim<LIM>(p.limiter, vR - vL, vL - vLL);
+    const double sRv = dxR * lim<LIM>(p.limiter, vRR - vR, vR - vL);
+    // Hnpsi and the density: where no cell of the region carries solids (a
+    // uniform branch) Hnpsi is 0 and rho the water's everywhere, and so are
+    // their slopes and face values.  Hnpsi: inside the tile both faces of a
+    // cell are reset where one is negative; across the tile edge only the
+    // copy this tile holds is checked (CorrectSlopes).
+    double hFL = 0.0, hFR = 0.0, rFL = p.rhow, rFR = p.rhow;
+    if (blk.solids) {
+        const double hLL = s.h[iLL], hL = s.h[iL], hR = s.h[iR], hRR = s.h[iRR];
+        const double sLh = dxL * lim<LIM>(p.limiter, hR - hL, hL - hLL);
+        const double sRh = dxR * lim<LIM>(p.limiter, hRR - hR, hR - hL);
+        const double rLL = s.rho[iLL], rL = s.rho[iL], rR = s.rho[iR], rRR = s.rho[iRR];
+        const double sLr = dxL * lim<LIM>(p.limiter, rR - rL, rL - rLL);
+        const double sRr = dxR * lim<LIM>(p.limiter, rRR - rR, rR - rL);
+        hFL = hL + sLh * hdx;
+        hFR = hR - sRh * hdx;
+        const double hWL = hL - sLh * hdx, hER = hR + sRh * hdx;
+        if ((hFL < 0.0) || (fpos != 0 && hWL < 0.0)) hFL = hL;
+        if ((hFR < 0.0) || (fpos != nn && hER < 0.0)) hFR = hR;
+        rFL = rL + sLr * hdx;
+        rFR = rR - sRr * hdx;
+    }
 
     // --- MUSCL face values (Reconstruct, src/HydraulicRHS.f90:397-490)
-    const double wEL = wL + sLw * 0.5 * dx;   // L's east face
-    const double wWR = wR - sRw * 0.5 * dx;   // R's west face
+    const double wEL = wL + sLw * hdx;   // L's east face
+    const double wWR = wR - sRw * hdx;   // R's west face
 
     // beds of the faces of L and R (InterpolateB, src/HydraulicRHS.f90:741-753);
     // the face itself is entry fi + 1, except at a tile edge, where the cell
     // on the far side sees its own tile's copy of the shared vertices
     const double* bed = YDIR ? &s.ybed[fj][0] : &s.xbed[fj][0];
     const double bWL = bed[fi], bER = bed[fi + 2];
-    const double fbL = (fpos == 0) ? (YDIR ? s.yside[0][fj] : s.xside[0][fj]) : bed[fi + 1];
-    const double fbR = (fpos == nn) ? (YDIR ? s.yside[1][fj] : s.xside[1][fj]) : bed[fi + 1];
+    const double bF = bed[fi + 1];
+    double fbL = bF, fbR = bF;
+    if (!blk.flat) {
+        if (fpos == 0) fbL = YDIR ? s.yside[0][fj] : s.xside[0][fj];
+        if (fpos == nn) fbR = YDIR ? s.yside[1][fj] : s.xside[1][fj];
+    }
 
     // --- CorrectSlopes for w (src/HydraulicRHS.f90:560-736): each cell's
     // pair of face values is replaced by the bed slope if either is below bed.
     // A ghost cell is tested with the face values ReconstructwAtEdges stored
     // from its tileContainer w (src/UpdateTiles.f90:669-750).
-    const double wLc = s.wst[iL], wRc = s.wst[iR];
     double wFL = wEL, wFR = wWR;
-    if ((wLc + sLw * 0.5 * dx < fbL) || (wLc - sLw * 0.5 * dx < bWL)) wFL = wL + 0.5 * (fbL - bWL);
-    if ((wRc + sRw * 0.5 * dx < bER) || (wRc - sRw * 0.5 * dx < fbR)) wFR = wR + 0.5 * (fbR - bER);
-    // Hnpsi: inside the tile both faces of a cell are reset; across the
-    // tile edge only the copy this tile holds is checked.
-    double hFL = hL + sLh * 0.5 * dx, hFR = hR - sRh * 0.5 * dx;
-    if (fpos == 0) {
-        if (hFL < 0.0) hFL = hL;
-    } else {
-        const double hWL = hL - sLh * 0.5 * dx;
-        if ((hFL < 0.0) || (hWL < 0.0)) hFL = hL;
-    }
-    if (fpos == nn) {
-        if (hFR < 0.0) hFR = hR;
-    } else {
-        const double hER = hR + sRh * 0.5 * dx;
-        if ((hFR < 0.0) || (hER < 0.0)) hFR = hR;
-    }
-    const double uFL = uL + sLu * 0.5 * dx, uFR = uR - sRu * 0.5 * dx;
-    const double vFL = vL + sLv * 0.5 * dx, vFR = vR - sRv * 0.5 * dx;
-    const double rFL = rL + sLr * 0.5 * dx, rFR = rR - sRr * 0.5 * dx;
+    if ((wLc + sLw * hdx < fbL) || (wLc - sLw * hdx < bWL)) wFL = wL + 0.5 * (fbL - bWL);
+    if ((wRc + sRw * hdx < bER) || (wRc - sRw * hdx < fbR)) wFR = wR + 0.5 * (fbR - bER);
+    const double uFL = uL + sLu * hdx, uFR = uR - sRu * hdx;
+    const double vFL = vL + sLv * hdx, vFR = vR - sRv * hdx;
 
     // face topography of this tile
-    const double fbp = ft.bp, fg = ft.g, fb0 = ft.b0, fbt = ft.bt;
+    const double fbp = ft.bp, fg = ft.g, fb0 = blk.flat ? bF : ft.b0, fbt = ft.bt;
     // face Hn from the corrected w (src/HydraulicRHS.f90:492-517)
     const double HnL = compute_hn(wFL, fb0, fbt, fg);
     const double HnR = compute_hn(wFR, fb0, fbt, fg);
@@ -510,10 +597,10 @@ __device__ __forceinline__ void face_flux(const DevT& d, const Params& p, Smem& 
         // a 1D grid keeps the x-face reconstruction of the conserved rhoHnv
         // (rho Hn v is rebuilt in 2D only, src/HydraulicRHS.f90:536-551)
         const double qLL = s.rv[iLL], qL = s.rv[iL], qR = s.rv[iR], qRR = s.rv[iRR];
-        const double sLq = actL ? dxr * lim<LIM>(p.limiter, qR - qL, qL - qLL) : 0.0;
-        const double sRq = actR ? dxr * lim<LIM>(p.limiter, qRR - qR, qR - qL) : 0.0;
-        rvL = qL + sLq * 0.5 * dx;
-        rvR = qR - sRq * 0.5 * dx;
+        const double sLq = dxL * lim<LIM>(p.limiter, qR - qL, qL - qLL);
+        const double sRq = dxR * lim<LIM>(p.limiter, qRR - qR, qR - qL);
+        rvL = qL + sLq * hdx;
+        rvR = qR - sRq * hdx;
     } else {
         rvL = rFL * HnL * vFL;
         rvR = rFR * HnR * vFR;
@@ -535,15 +622,11 @@ __device__ __forceinline__ void face_flux(const DevT& d, const Params& p, Smem& 
     }
 
     // --- fluxes (src/HydraulicRHS.f90:1027-1067, src/Equations.f90:53-245)
-    double* F = YDIR ? &s.fy[0][0] : &s.fx[0][0];
-    constexpr int NFACE = YDIR ? Smem::NFY : Smem::NFX;
-    const int fslot = YDIR ? (fi * B + fj) : (fj * (B + 1) + fi);
     // zero flux where the wave speeds close (src/HydraulicRHS.f90:1028-1031);
     // computed without a branch so the two faces of a thread interleave
     const double dif = aPos - aNeg;
     const bool none = dif < 1e-10;
     const double cPw = HnR * unR * fg, cMw = HnL * unL * fg;
-    const double cPh = hFR * unR * fg, cMh = hFL * unL * fg;
     const double cPu = ruR * unR, cMu = ruL * unL;
     const double cPv = rvR * unR, cMv = rvL * unL;
     double hp = -fbt;
@@ -556,27 +639,31 @@ __device__ __forceinline__ void face_flux(const DevT& d, const Params& p, Smem& 
     double x = HnR * fg - HnL * fg;
     x = x * aPos * aNeg;
     x = x + (aPos * cMw - aNeg * cPw);
-    F[0 * NFACE + fslot] = none ? 0.0 : x / dif;
+    F.q[0] = none ? 0.0 : x / dif;
     x = ruR - ruL;
     x = x * aPos * aNeg;
     x = x + (aPos * cMu - aNeg * cPu);
-    F[1 * NFACE + fslot] = none ? 0.0 : x / dif;
+    F.q[1] = none ? 0.0 : x / dif;
     x = rvR - rvL;
     x = x * aPos * aNeg;
     x = x + (aPos * cMv - aNeg * cPv);
-    F[2 * NFACE + fslot] = none ? 0.0 : x / dif;
-    x = hFR * fg - hFL * fg;
-    x = x * aPos * aNeg;
-    x = x + (aPos * cMh - aNeg * cPh);
-    F[3 * NFACE + fslot] = none ? 0.0 : x / dif;
-    F[4 * NFACE + fslot] = none ? 0.0 : (aPos * hydM - aNeg * hydP) / dif;
+    F.q[2] = none ? 0.0 : x / dif;
+    F.q[3] = 0.0;
+    if (blk.solids) {
+        const double cPh = hFR * unR * fg, cMh = hFL * unL * fg;
+        x = hFR * fg - hFL * fg;
+        x = x * aPos * aNeg;
+        x = x + (aPos * cMh - aNeg * cPh);
+        F.q[3] = none ? 0.0 : x / dif;
+    }
+    F.g = none ? 0.0 : (aPos * hydM - aNeg * hydP) / dif;
     if (VISC) {
         const double pPu = (HnR < 0.0) ? 0.0 : p.nu * rFR * HnR * sRu;
         const double pPv = (HnR < 0.0) ? 0.0 : p.nu * rFR * HnR * sRv;
         const double pMu = (HnL < 0.0) ? 0.0 : p.nu * rFL * HnL * sLu;
         const double pMv = (HnL < 0.0) ? 0.0 : p.nu * rFL * HnL * sLv;
-        F[5 * NFACE + fslot] = none ? 0.0 : 0.5 * (pPu + pMu);
-        F[6 * NFACE + fslot] = none ? 0.0 : 0.5 * (pPv + pMv);
+        F.q[5] = none ? 0.0 : 0.5 * (pPu + pMu);
+        F.q[6] = none ? 0.0 : 0.5 * (pPv + pMv);
     }
 }
 
@@ -593,75 +680,75 @@ __device__ __forceinline__ float wave_root_f(const Params& p, float hn, float bp
 }
 
 template <bool YDIR, bool VISC, int LIM, bool CFL, typename Smem, class DevT>
-__device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, Smem& s, int fi, int fj,
-                                                double& cfl_min) {
+__device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, const Smem& sm, const Block& blk,
+                                                int fi, int fj, double& cfl_min, const FaceTopo& ft,
+                                                FaceFlux<true>& F) {
+    const auto& s = sm.r;
     int iLL, iL, iR, iRR;
     if (!YDIR) { iLL = rg(fi - 2, fj); iL = rg(fi - 1, fj); iR = rg(fi, fj); iRR = rg(fi + 1, fj); }
     else       { iLL = rg(fj, fi - 2); iL = rg(fj, fi - 1); iR = rg(fj, fi); iRR = rg(fj, fi + 1); }
     const double dxr = YDIR ? p.dyr : p.dxr;
     const double dx = YDIR ? p.dy : p.dx;
     const float dxrf = (float)dxr, hdx = (float)(0.5 * dx);
-    const bool actL = s.act[iL], actR = s.act[iR];
     const int nn = YDIR ? p.ny : p.nx;
-    const int fpos = (YDIR ? s.by0 : s.bx0) + fi;
+    const int fpos = (YDIR ? blk.by0 : blk.bx0) + fi;
+    const bool actL = fpos > 0 || (blk.nact & (YDIR ? 4 : 1));
+    const bool actR = fpos < nn || (blk.nact & (YDIR ? 8 : 2));
 
     // FP64: w slopes (non-active tiles keep their stored slope), density slopes
     const double wLL = s.w[iLL], wL = s.w[iL], wR = s.w[iR], wRR = s.w[iRR];
-    const double* gs = YDIR ? d.gsy : d.gsx;
-    const double sLw = actL ? dxr * lim<LIM>(p.limiter, wR - wL, wL - wLL) : gs[s.gidx[iL]];
-    const double sRw = actR ? dxr * lim<LIM>(p.limiter, wRR - wR, wR - wL) : gs[s.gidx[iR]];
-    const double rLL = s.rho[iLL], rL = s.rho[iL], rR = s.rho[iR], rRR = s.rho[iRR];
-    const double sLr = actL ? dxr * lim<LIM>(p.limiter, rR - rL, rL - rLL) : 0.0;
-    const double sRr = actR ? dxr * lim<LIM>(p.limiter, rRR - rR, rR - rL) : 0.0;
-    // FP32: Hnpsi, u, v slopes
-    const float hLL = s.h[iLL], hL = s.h[iL], hR = s.h[iR], hRR = s.h[iRR];
-    const float sLh = actL ? dxrf * lim<LIM>(p.limiter, hR - hL, hL - hLL) : 0.f;
-    const float sRh = actR ? dxrf * lim<LIM>(p.limiter, hRR - hR, hR - hL) : 0.f;
+    double sLw = dxr * lim<LIM>(p.limiter, wR - wL, wL - wLL);
+    double sRw = dxr * lim<LIM>(p.limiter, wRR - wR, wR - wL);
+    double wLc = wL, wRc = wR;
+    if (!actL) { const GhostCell g = ghost_cell<YDIR>(d, p, blk, false, fj); sLw = g.slope; wLc = g.w; }
+    if (!actR) { const GhostCell g = ghost_cell<YDIR>(d, p, blk, true, fj); sRw = g.slope; wRc = g.w; }
+    const double dxL = actL ? dxr : 0.0, dxR = actR ? dxr : 0.0;
+    const float dxLf = actL ? dxrf : 0.f, dxRf = actR ? dxrf : 0.f;
+    const double hdxd = 0.5 * dx;
+    // FP32: u, v slopes
     const float uLL = s.u[iLL], uL = s.u[iL], uR = s.u[iR], uRR = s.u[iRR];
-    const float sLu = actL ? dxrf * lim<LIM>(p.limiter, uR - uL, uL - uLL) : 0.f;
-    const float sRu = actR ? dxrf * lim<LIM>(p.limiter, uRR - uR, uR - uL) : 0.f;
+    const float sLu = dxLf * lim<LIM>(p.limiter, uR - uL, uL - uLL);
+    const float sRu = dxRf * lim<LIM>(p.limiter, uRR - uR, uR - uL);
     const float vLL = s.v[iLL], vL = s.v[iL], vR = s.v[iR], vRR = s.v[iRR];
-    const float sLv = actL ? dxrf * lim<LIM>(p.limiter, vR - vL, vL - vLL) : 0.f;
-    const float sRv = actR ? dxrf * lim<LIM>(p.limiter, vRR - vR, vR - vL) : 0.f;
+    const float sLv = dxLf * lim<LIM>(p.limiter, vR - vL, vL - vLL);
+    const float sRv = dxRf * lim<LIM>(p.limiter, vRR - vR, vR - vL);
+    // Hnpsi (FP32) and the density (FP64), as in face_flux
+    float hFL = 0.f, hFR = 0.f;
+    double rFL = p.rhow, rFR = p.rhow;
+    if (blk.solids) {
+        const double rLL = s.rho[iLL], rL = s.rho[iL], rR = s.rho[iR], rRR = s.rho[iRR];
+        const double sLr = dxL * lim<LIM>(p.limiter, rR - rL, rL - rLL);
+        const double sRr = dxR * lim<LIM>(p.limiter, rRR - rR, rR - rL);
+        const float hLL = s.h[iLL], hL = s.h[iL], hR = s.h[iR], hRR = s.h[iRR];
+        const float sLh = dxLf * lim<LIM>(p.limiter, hR - hL, hL - hLL);
+        const float sRh = dxRf * lim<LIM>(p.limiter, hRR - hR, hR - hL);
+        hFL = hL + sLh * hdx;
+        hFR = hR - sRh * hdx;
+        const float hWL = hL - sLh * hdx, hER = hR + sRh * hdx;
+        if ((hFL < 0.f) || (fpos != 0 && hWL < 0.f)) hFL = hL;
+        if ((hFR < 0.f) || (fpos != nn && hER < 0.f)) hFR = hR;
+        rFL = rL + sLr * hdxd;
+        rFR = rR - sRr * hdxd;
+    }
 
     // FP64: w face values, beds and CorrectSlopes (as face_flux)
-    const double wEL = wL + sLw * 0.5 * dx;
-    const double wWR = wR - sRw * 0.5 * dx;
+    const double wEL = wL + sLw * hdxd;
+    const double wWR = wR - sRw * hdxd;
     const double* bed = YDIR ? &s.ybed[fj][0] : &s.xbed[fj][0];
     const double bWL = bed[fi], bER = bed[fi + 2];
-    const double fbL = (fpos == 0) ? (YDIR ? s.yside[0][fj] : s.xside[0][fj]) : bed[fi + 1];
-    const double fbR = (fpos == nn) ? (YDIR ? s.yside[1][fj] : s.xside[1][fj]) : bed[fi + 1];
-    const double wLc = s.wst[iL], wRc = s.wst[iR];
+    const double bF = bed[fi + 1];
+    double fbL = bF, fbR = bF;
+    if (!blk.flat) {
+        if (fpos == 0) fbL = YDIR ? s.yside[0][fj] : s.xside[0][fj];
+        if (fpos == nn) fbR = YDIR ? s.yside[1][fj] : s.xside[1][fj];
+    }
     double wFL = wEL, wFR = wWR;
-    if ((wLc + sLw * 0.5 * dx < fbL) || (wLc - sLw * 0.5 * dx < bWL)) wFL = wL + 0.5 * (fbL - bWL);
-    if ((wRc + sRw * 0.5 * dx < bER) || (wRc - sRw * 0.5 * dx < fbR)) wFR = wR + 0.5 * (fbR - bER);
-    float hFL = hL + sLh * hdx, hFR = hR - sRh * hdx;
-    if (fpos == 0) {
-        if (hFL < 0.f) hFL = hL;
-    } else {
-        const float hWL = hL - sLh * hdx;
-        if ((hFL < 0.f) || (hWL < 0.f)) hFL = hL;
-    }
-    if (fpos == nn) {
-        if (hFR < 0.f) hFR = hR;
-    } else {
-        const float hER = hR + sRh * hdx;
-        if ((hFR < 0.f) || (hER < 0.f)) hFR = hR;
-    }
+    if ((wLc + sLw * hdxd < fbL) || (wLc - sLw * hdxd < bWL)) wFL = wL + 0.5 * (fbL - bWL);
+    if ((wRc + sRw * hdxd < bER) || (wRc - sRw * hdxd < fbR)) wFR = wR + 0.5 * (fbR - bER);
     const float uFL = uL + sLu * hdx, uFR = uR - sRu * hdx;
     const float vFL = vL + sLv * hdx, vFR = vR - sRv * hdx;
-    const double rFL = rL + sLr * 0.5 * dx, rFR = rR - sRr * 0.5 * dx;
 
-    const int t = s.tile;
-    int fidx;
-    double fbp, fg, fb0, fbt;
-    if (!YDIR) {
-        fidx = t * p.NFX + (s.by0 + fj) * (p.nx + 1) + fpos;
-        fbp = d.T.xby[fidx]; fg = d.T.xgam[fidx]; fb0 = d.xb0[fidx]; fbt = d.T.xbt[fidx];
-    } else {
-        fidx = t * p.NFY + fpos * p.nx + (s.bx0 + fj);
-        fbp = d.T.ybx[fidx]; fg = d.T.ygam[fidx]; fb0 = d.yb0[fidx]; fbt = d.T.ybt[fidx];
-    }
+    const double fbp = ft.bp, fg = ft.g, fb0 = blk.flat ? bF : ft.b0, fbt = ft.bt;
     const double HnL = compute_hn(wFL, fb0, fbt, fg);
     const double HnR = compute_hn(wFR, fb0, fbt, fg);
     const float HnLf = (float)HnL, HnRf = (float)HnR, fgf = (float)fg;
@@ -680,19 +767,16 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
     if (aNeg > 0.f) aNeg = 0.f;
     if (CFL) {
         if ((double)aPos > kEps)
-            cfl_min = fmin((double)((float)(YDIR ? d.T.ynp : d.T.xnp)[fidx] / aPos), cfl_min);
+            cfl_min = fmin((double)((float)ft.np / aPos), cfl_min);
         if ((double)fabsf(aNeg) > kEps)
-            cfl_min = fmin((double)((float)(YDIR ? d.T.ynm : d.T.xnm)[fidx] / fabsf(aNeg)), cfl_min);
+            cfl_min = fmin((double)((float)ft.nm / fabsf(aNeg)), cfl_min);
     }
 
-    float* F = YDIR ? &s.fy[0][0] : &s.fx[0][0];
-    constexpr int NFACE = YDIR ? Smem::NFY : Smem::NFX;
-    double* F4 = YDIR ? s.fy4 : s.fx4;
-    const int fslot = YDIR ? (fi * B + fj) : (fj * (B + 1) + fi);
     const float dif = aPos - aNeg;
     if (dif < 1e-10f) {
-        for (int q = 0; q < (VISC ? 7 : 5); ++q) F[q * NFACE + fslot] = 0.f;
-        F4[fslot] = 0.0;
+#pragma unroll
+        for (int q = 0; q < 7; ++q) F.q[q] = 0.f;
+        F.g = 0.0;
         return;
     }
     const float rd = __builtin_amdgcn_rcpf(dif);
@@ -701,10 +785,10 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
     const float cPu = ruR * unR, cMu = ruL * unL;
     const float cPv = rvR * unR, cMv = rvL * unL;
     const float ab = aPos * aNeg;
-    F[0 * NFACE + fslot] = ((HnRf * fgf - HnLf * fgf) * ab + (aPos * cMw - aNeg * cPw)) * rd;
-    F[1 * NFACE + fslot] = ((ruR - ruL) * ab + (aPos * cMu - aNeg * cPu)) * rd;
-    F[2 * NFACE + fslot] = ((rvR - rvL) * ab + (aPos * cMv - aNeg * cPv)) * rd;
-    F[3 * NFACE + fslot] = ((hFR * fgf - hFL * fgf) * ab + (aPos * cMh - aNeg * cPh)) * rd;
+    F.q[0] = ((HnRf * fgf - HnLf * fgf) * ab + (aPos * cMw - aNeg * cPw)) * rd;
+    F.q[1] = ((ruR - ruL) * ab + (aPos * cMu - aNeg * cPu)) * rd;
+    F.q[2] = ((rvR - rvL) * ab + (aPos * cMv - aNeg * cPv)) * rd;
+    F.q[3] = ((hFR * fgf - hFL * fgf) * ab + (aPos * cMh - aNeg * cPh)) * rd;
     // FP64 hydrostatic flux
     double hp = -fbt;
     hp = hp + (wFR - fb0);
@@ -713,7 +797,7 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
     hp = hp + (wFL - fb0);
     const double hydM = 0.5 * p.g * rFL * hp * hp;
     const double aP = aPos, aN = aNeg;
-    F4[fslot] = (aP * hydM - aN * hydP) / (aP - aN);
+    F.g = (aP * hydM - aN * hydP) / (aP - aN);
     if (VISC) {
         const float nu = (float)p.nu;
         float pPu, pPv, pMu, pMv;
@@ -721,18 +805,20 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
         else { pPu = nu * rFRf * HnRf * sRu; pPv = nu * rFRf * HnRf * sRv; }
         if (HnLf < 0.f) { pMu = 0.f; pMv = 0.f; }
         else { pMu = nu * rFLf * HnLf * sLu; pMv = nu * rFLf * HnLf * sLv; }
-        F[5 * NFACE + fslot] = 0.5f * (pPu + pMu);
-        F[6 * NFACE + fslot] = 0.5f * (pPv + pMv);
+        F.q[5] = 0.5f * (pPu + pMu);
+        F.q[6] = 0.5f * (pPv + pMv);
     }
 }
 
-// Block-wide minimum of a positive double into a control slot.
+// Block-wide minimum of a positive double into a control slot: each wave's
+// minimum to LDS before a barrier, then thread 0 takes the block's.
 template <typename Smem>
-__device__ void reduce_min_to(Smem& s, double v, unsigned long long* slot) {
+__device__ __forceinline__ void wave_min(Smem& s, double v) {
     for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) s.red[wv] = v;
-    __syncthreads();
+    if ((threadIdx.x & 63) == 0) s.red[threadIdx.x >> 6] = v;
+}
+template <typename Smem>
+__device__ __forceinline__ void block_min_to(const Smem& s, unsigned long long* slot) {
     if (threadIdx.x == 0) {
         double m = s.red[0];
         for (int i = 1; i < STAGE_NT / 64; ++i) m = fmin(m, s.red[i]);
@@ -763,13 +849,13 @@ __device__ __forceinline__ double ghost_bed(const DevT& d, const Params& p, int 
 template <bool YDIR, class DevT>
 __device__ __forceinline__ double face_bed(const DevT& d, const Params& p, int t, int K, int r) {
     if (!YDIR) {
-        if (K < 0) return d.T.xib[nb_tile(p, t, -1, 0) * p.NFX + r * (p.nx + 1) + (p.nx - 1)];
-        if (K > p.nx) return d.T.xib[nb_tile(p, t, 1, 0) * p.NFX + r * (p.nx + 1) + 1];
-        return d.T.xib[t * p.NFX + r * (p.nx + 1) + K];
+        if (K < 0) return ld(d.T.xib, nb_tile(p, t, -1, 0) * p.NFX + r * (p.nx + 1) + (p.nx - 1));
+        if (K > p.nx) return ld(d.T.xib, nb_tile(p, t, 1, 0) * p.NFX + r * (p.nx + 1) + 1);
+        return ld(d.T.xib, t * p.NFX + r * (p.nx + 1) + K);
     } else {
-        if (K < 0) return d.T.yib[nb_tile(p, t, 0, -1) * p.NFY + (p.ny - 1) * p.nx + r];
-        if (K > p.ny) return d.T.yib[nb_tile(p, t, 0, 1) * p.NFY + 1 * p.nx + r];
-        return d.T.yib[t * p.NFY + K * p.nx + r];
+        if (K < 0) return ld(d.T.yib, nb_tile(p, t, 0, -1) * p.NFY + (p.ny - 1) * p.nx + r);
+        if (K > p.ny) return ld(d.T.yib, nb_tile(p, t, 0, 1) * p.NFY + 1 * p.nx + r);
+        return ld(d.T.yib, t * p.NFY + K * p.nx + r);
     }
 }
 
@@ -778,15 +864,30 @@ __device__ __forceinline__ double face_bed(const DevT& d, const Params& p, int t
 // STAGE 3: RHS(u2); u3 -> S3.                   (src/TimeStepper.f90:447-498)
 // STAGE 4: RHS(u3); implicit drag -> Sout; maxima; activation flags.
 //                                               (src/TimeStepper.f90:501-524)
-// pre: the face's topography when it was loaded ahead (FP64 only).
+// pre: the face's topography when it was loaded ahead.
 template <bool YDIR, bool VISC, int LIM, bool CFL, bool MIX, typename Smem, class DevT>
-__device__ __forceinline__ void face_work(const DevT& d, const Params& p, Smem& s, int fi, int fj,
-                                          double& cfl_min, const FaceTopo* pre = nullptr) {
-    if constexpr (MIX) {
-        face_flux_mixed<YDIR, VISC, LIM, CFL>(d, p, s, fi, fj, cfl_min);
-    } else {
-        const FaceTopo ft = pre ? *pre : load_face_topo<YDIR, CFL>(d, p, s, fi, fj);
-        face_flux<YDIR, VISC, LIM, CFL>(d, p, s, fi, fj, cfl_min, ft);
+__device__ __forceinline__ void face_work(const DevT& d, const Params& p, const Smem& s, const Block& blk, int fi,
+                                          int fj, double& cfl_min, FaceFlux<MIX>& F,
+                                          const FaceTopo* pre = nullptr) {
+    const FaceTopo ft = pre ? *pre : load_face_topo_at<YDIR, CFL>(d, p, blk.t, blk.bx0, blk.by0, fi, fj, blk.flat);
+    if constexpr (MIX) face_flux_mixed<YDIR, VISC, LIM, CFL>(d, p, s, blk, fi, fj, cfl_min, ft, F);
+    else face_flux<YDIR, VISC, LIM, CFL>(d, p, s, blk, fi, fj, cfl_min, ft, F);
+}
+
+template <bool YDIR, bool MIX, typename Smem>
+__device__ __forceinline__ void put_flux(Smem& s, int fi, int fj, const FaceFlux<MIX>& F) {
+    const int i = YDIR ? (fi * B + fj) : (fj * (B + 1) + fi);
+#pragma unroll
+    for (int q = 0; q < Smem::NQ; ++q) {
+        if (q == 4) {
+            if (MIX) (YDIR ? s.f.fy4 : s.f.fx4)[i] = F.g;
+            else if (YDIR) s.f.fy[4][i] = F.g;
+            else s.f.fx[4][i] = F.g;
+        } else if (YDIR) {
+            s.f.fy[q][i] = F.q[q];
+        } else {
+            s.f.fx[q][i] = F.q[q];
+        }
     }
 }
 
@@ -794,9 +895,9 @@ __device__ __forceinline__ void face_work(const DevT& d, const Params& p, Smem& 
 template <bool MIX, bool YDIR, typename Smem>
 __device__ __forceinline__ double fluxv(const Smem& s, int q, int i) {
     if constexpr (MIX) {
-        if (q == 4) return YDIR ? s.fy4[i] : s.fx4[i];
+        if (q == 4) return YDIR ? s.f.fy4[i] : s.f.fx4[i];
     }
-    return YDIR ? (double)s.fy[q][i] : (double)s.fx[q][i];
+    return YDIR ? (double)s.f.fy[q][i] : (double)s.f.fx[q][i];
 }
 
 // With morphodynamics the same kernels evaluate both hydraulic operators of
@@ -885,6 +986,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         }
         s.dt = dt;
         s.cur = c->cur;
+        s.flat = c->flat;
         const double tb = d.second ? c->t + dt : c->t;   // grid%t of this operator
         s.tgrid = tb;
         s.tstage = (STAGE == 1) ? tb : (STAGE == 3 ? tb + 0.5 * dt : tb + dt);
@@ -909,16 +1011,33 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         }
         s.skip = skip;
         s.more = more;
+        s.solids = 0;
     }
     __syncthreads();
     // read as wave-uniform values, so that the block's loop over items is a
     // uniform loop (a loop the compiler must treat as divergent costs far more)
     if (__builtin_amdgcn_readfirstlane(s.skip)) return false;
     const bool more = __builtin_amdgcn_readfirstlane(s.more) != 0;
-    const int t = s.tile;
+    const int t = __builtin_amdgcn_readfirstlane(s.tile);
     const double dt = s.dt;
     const int FS = (int)d.FS;
-    const int bxa = s.bxa, bya = s.bya;
+    const int bxa = __builtin_amdgcn_readfirstlane(s.bxa), bya = __builtin_amdgcn_readfirstlane(s.bya);
+    const double* Un = (MIX && s.cur) ? d.S0b : d.S0;   // u^n of the step
+    Block blk;
+    blk.t = t;
+    blk.bx0 = __builtin_amdgcn_readfirstlane(s.bx0);
+    blk.by0 = __builtin_amdgcn_readfirstlane(s.by0);
+    blk.flat = __builtin_amdgcn_readfirstlane(s.flat) != 0;
+    blk.Un = Un;
+    // whether the neighbour tiles are active, for the face pass (wave 3: its
+    // halo cells come last)
+    if (tid >= 192 && tid < 196) {
+        const int q = tid - 192;   // W, E, S, N
+        const int k = (Smem::oned && q >= 2) ? t
+                                             : nb_tile(p, t, q == 0 ? -1 : (q == 1 ? 1 : 0), q == 2 ? -1 : (q == 3 ? 1 : 0));
+        const unsigned long long on = __ballot(k >= 0 && k < p.ntiles && d.tstate[k] == KST_TILE_ACTIVE);
+        if (q == 0) s.nact = (int)(on & 15ull);
+    }
 
     // ---- phase A: stage state + derived variables on the region ----------
     const int tx = tid % B, ty = tid / B;
@@ -926,8 +1045,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     double ow = 0, oru = 0, orv = 0, oh = 0, ohn = 0, ou = 0, ov = 0, opsi = 0, orho = 0;
     double ob0 = 0, obt = 0, og = 1;
     double pw = 0, pru = 0, prv = 0, ph = 0;   // u^n of the owned cell (stage 2; mixed: 2..4)
-    int oidx = 0;
-    const double* Un = (MIX && s.cur) ? d.S0b : d.S0;   // u^n of the step
+    unsigned oidx = 0;
     // threads 0..OWN-1: the owned cells; the 2-cell halo strips (4 strips of
     // 2 x 16 slots) by the next 128 threads in the same round when there are
     // enough, else by threads 128..255 in a second round (waves 0 and 1 take
@@ -948,10 +1066,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         bool yb;
         const int q = split_item(tid, NXB, NYB, &yb);
         if (q >= 0) {
-            if (!yb) bedv = face_bed<false>(d, p, t, s.bx0 + q % (B + 3) - 1, s.by0 + q / (B + 3));
-            else bedv = face_bed<true>(d, p, t, s.by0 + q % (BY + 3) - 1, s.bx0 + q / (BY + 3));
+            if (!yb) bedv = face_bed<false>(d, p, t, blk.bx0 + q % (B + 3) - 1, blk.by0 + q / (B + 3));
+            else bedv = face_bed<true>(d, p, t, blk.by0 + q % (BY + 3) - 1, blk.bx0 + q / (BY + 3));
         }
     }
+    bool solids = false;
     for (int round = 0; round < (one_round ? 1 : 2); ++round) {
         int rx, ry;
         bool valid;
@@ -968,11 +1087,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         }
         if (!valid) continue;
         int tc, ci, cj;
-        map_cell(p, t, s.bx0 + rx, s.by0 + ry, tc, ci, cj);
-        const int gi = tc * p.NC + cj * p.nx + ci;
+        map_cell(p, t, blk.bx0 + rx, blk.by0 + ry, tc, ci, cj);
+        const unsigned gi = tc * p.NC + cj * p.nx + ci;
         double w, ru, rv, h;
         if constexpr (MIX) {
-            w = Un[gi]; ru = Un[FS + gi]; rv = Un[2 * FS + gi]; h = Un[3 * FS + gi];
+            w = ld(Un, gi); ru = ld(Un + FS, gi); rv = ld(Un + 2 * (size_t)FS, gi); h = ld(Un + 3 * (size_t)FS, gi);
             if (round == 0) { pw = w; pru = ru; prv = rv; ph = h; }
             if (STAGE == 2) {
                 const float* Rf = (const float*)d.R;
@@ -990,11 +1109,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
                 h = h + (double)Sf[3 * FS + gi];
             }
         } else if (STAGE == 1 || STAGE == 2) {
-            w = d.Uw[gi]; ru = d.Uu[gi]; rv = d.Uv[gi]; h = d.Uh[gi];
+            w = ld(d.Uw, gi); ru = ld(d.Uu, gi); rv = ld(d.Uv, gi); h = ld(d.Uh, gi);
             if (STAGE == 2) {
                 if (round == 0) { pw = w; pru = ru; prv = rv; ph = h; }
-                const double ew = d.R[gi], eu = d.R[FS + gi], ev = d.R[2 * FS + gi];
-                const double eh = d.R[3 * FS + gi], im = d.R[4 * FS + gi];
+                const double ew = ld(d.R, gi), eu = ld(d.R + FS, gi), ev = ld(d.R + 2 * (size_t)FS, gi);
+                const double eh = ld(d.R + 3 * (size_t)FS, gi), im = ld(d.R + 4 * (size_t)FS, gi);
                 ru = (ru + dt * eu) / (1.0 - dt * im);
                 rv = (rv + dt * ev) / (1.0 - dt * im);
                 w = w + dt * ew;
@@ -1002,9 +1121,9 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             }
         } else {
             const double* S = (STAGE == 3) ? d.S2 : d.S3;
-            w = S[gi]; ru = S[FS + gi]; rv = S[2 * FS + gi]; h = S[3 * FS + gi];
+            w = ld(S, gi); ru = ld(S + FS, gi); rv = ld(S + 2 * (size_t)FS, gi); h = ld(S + 3 * (size_t)FS, gi);
         }
-        const double b0c = d.b0c[gi], btc = d.T.btc[gi], gam = d.T.cgam[gi];
+        const double b0c = ld(d.b0c, gi), btc = blk.flat ? 0.0 : ld(d.T.btc, gi), gam = ld(d.T.cgam, gi);
         const bool act = d.tstate[tc] == KST_TILE_ACTIVE;
         // ComputeDesingularisedVariables (src/HydraulicRHS.f90:762-878) runs
         // on active tiles only; ghost tiles keep SetDefaultTileData's zeros
@@ -1016,84 +1135,104 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             if (hpc < 0.0) hpc = 0.0;
             const double eps = p.hthr;
             const double den = hn * hn + dmax(hn * hn, eps * eps);
-            psi = dmin(2.0 * hn * hpc / den, p.max_pack);
-            rho = density(p, psi);
-            uu = 2.0 * hn * ru / (hn * hn + dmax(hn * hn, eps * eps)) / rho;
+            // (0 / den is 0: no division, and the water's density, without solids)
+            if (hpc != 0.0) {
+                psi = dmin(2.0 * hn * hpc / den, p.max_pack);
+                rho = density(p, psi);
+            }
+            uu = 2.0 * hn * ru / den / rho;
             // a 1D grid never derives v (src/HydraulicRHS.f90:870-874): it stays 0
-            if constexpr (!Smem::oned) vv = 2.0 * hn * rv / (hn * hn + dmax(hn * hn, eps * eps)) / rho;
+            if constexpr (!Smem::oned) vv = 2.0 * hn * rv / den / rho;
         } else if (p.bc == KST_BC_DIRICHLET && dirichlet_ghost(p, tc)) {
             hn = p.bc_hn; psi = p.bc_psi; rho = p.bc_rho; uu = p.bc_u; vv = p.bc_v;
         }
+        solids |= h != 0.0 || psi != 0.0;
         const int r = rg(rx, ry);
-        if constexpr (Smem::oned) s.rv[r] = rv;
-        s.w[r] = w; s.h[r] = h; s.u[r] = uu; s.v[r] = vv; s.rho[r] = rho;
-        s.wst[r] = act ? w : Un[gi];
-        s.gidx[r] = gi;
-        s.act[r] = act ? 1 : 0;
+        if constexpr (Smem::oned) s.r.rv[r] = rv;
+        s.r.w[r] = w; s.r.h[r] = h; s.r.u[r] = uu; s.r.v[r] = vv; s.r.rho[r] = rho;
         if (round == 0) {
             ow = w; oru = ru; orv = rv; oh = h; ohn = hn; ou = uu; ov = vv; opsi = psi; orho = rho;
             ob0 = b0c; obt = btc; og = gam; oidx = gi;
         }
     }
+    if (__ballot(solids) != 0 && (tid & 63) == 0) s.solids = 1;
+    constexpr bool STASH = Smem::alias && !MIX && STAGE == 2;
+    if (STASH && own) { s.mom[0][tid] = oru; s.mom[1][tid] = orv; }
+    // DragClosure + ImplicitSourceTerms (src/Equations.f90:627-658) of the
+    // owned cell.  Here and not with the rest of its right-hand side: the
+    // closures are a call, and what lives over a call can use only half of
+    // the registers (in phase C that set the kernel's 158 VGPRs; here almost
+    // nothing lives)
+    double Im = 0.0;
+    if (own && ohn > p.hthr) {
+        const double bx = ld(d.T.cbx, oidx), by = ld(d.T.cby, oidx);
+        const double fric = drag(p, ohn, ou, ov, opsi, bx, by, og);
+        const double modu = sqrt(speed2(p.geometric, ou, ov, bx, by));
+        if (modu > 1.0e-8) {
+            const double hr = 1.0 / ohn;
+            Im = -(fric * hr / modu);
+        }
+    }
     // the small shape's loads of what phases B and C read: its face's
-    // topography, its cell's bed slopes and prefactors (and u^n in stage 3)
-    // (the cell's bed slopes and prefactors also in the first and last stage
-    // of the 16 x 16 shape, which have registers to spare for them)
+    // topography, its cell's bed slopes and prefactors (and u^n in stage 3);
+    // the 16 x 16 shape loads them as the face pass ends, so that they take
+    // no registers during it
     FaceTopo pft{};
     double pbx = 0, pby = 0, pgxu = 0, pgxv = 0, pgyv = 0, pw0 = 0, pu0 = 0, pv0 = 0, ph0 = 0;
-    const bool prec = pre || STAGE == 1 || STAGE == 4;
     if (pre) {
         bool yf;
         const int f = split_item(tid, Smem::NFX, Smem::NFY, &yf);
         if (f >= 0) {
-            if (!yf) pft = load_face_topo<false, STAGE != 4>(d, p, s, f % (B + 1), f / (B + 1));
-            else pft = load_face_topo<true, STAGE != 4>(d, p, s, f / B, f % B);
+            if (!yf) pft = load_face_topo_at<false, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f % (B + 1), f / (B + 1), blk.flat);
+            else pft = load_face_topo_at<true, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f / B, f % B, blk.flat);
         }
-        if (own && STAGE == 3) { pw0 = d.Uw[oidx]; pu0 = d.Uu[oidx]; pv0 = d.Uv[oidx]; ph0 = d.Uh[oidx]; }
-    }
-    if (prec && own) {
-        pbx = d.T.cbx[oidx]; pby = d.T.cby[oidx];
-        pgxu = d.T.pxu[oidx]; pgxv = d.T.pxv[oidx]; pgyv = d.T.pyv[oidx];
     }
     // the last stage's maxima update reads u^n and six maxima fields of the
-    // owned cell (each written only by its owner): loaded here too
+    // owned cell (each written only by its owner): loaded with them
     const bool trk = STAGE == 4 && p.track_maxima && !d.second;
     double mxv[6] = {0, 0, 0, 0, 0, 0}, mun[4] = {0, 0, 0, 0};
-    if (trk && own) {
+    auto load_cell = [&]() {
+        if (!own) return;
+        if (STAGE == 3 && !MIX) { pw0 = ld(d.Uw, oidx); pu0 = ld(d.Uu, oidx); pv0 = ld(d.Uv, oidx); ph0 = ld(d.Uh, oidx); }
+        pbx = ld(d.T.cbx, oidx); pby = ld(d.T.cby, oidx);
+        pgxu = ld(d.T.pxu, oidx); pgxv = ld(d.T.pxv, oidx); pgyv = ld(d.T.pyv, oidx);
+        if (trk) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) mxv[k] = d.maxima[2 * k * FS + oidx];   // fields 0, 2, ..., 10
+            for (int k = 0; k < 6; ++k) mxv[k] = ld(d.maxima + 2 * k * (size_t)FS, oidx);   // fields 0, 2, ..., 10
 #pragma unroll
-        for (int k = 0; k < 4; ++k) mun[k] = Un[k * FS + oidx];
-    }
+            for (int k = 0; k < 4; ++k) mun[k] = ld(Un + k * (size_t)FS, oidx);
+        }
+    };
+    if (!Smem::alias) load_cell();
     // face beds: rows of x-faces -1..bxa+1 and columns of y-faces -1..bya+1
     if (pre) {
         bool yb;
         const int q = split_item(tid, NXB, NYB, &yb);
         if (q >= 0) {
-            if (!yb) s.xbed[q / (B + 3)][q % (B + 3)] = bedv;
-            else s.ybed[q / (BY + 3)][q % (BY + 3)] = bedv;
+            if (!yb) s.r.xbed[q / (B + 3)][q % (B + 3)] = bedv;
+            else s.r.ybed[q / (BY + 3)][q % (BY + 3)] = bedv;
         }
     } else {
         for (int q = tid; q < B * (B + 3); q += STAGE_NT) {
             const int r = q / (B + 3), k = q % (B + 3) - 1;
-            if (r < bya && k <= bxa + 1) s.xbed[r][k + 1] = face_bed<false>(d, p, t, s.bx0 + k, s.by0 + r);
+            if (r < bya && k <= bxa + 1) s.r.xbed[r][k + 1] = face_bed<false>(d, p, t, blk.bx0 + k, blk.by0 + r);
             if (!Smem::oned && r < bxa && k <= bya + 1)
-                s.ybed[r][k + 1] = face_bed<true>(d, p, t, s.by0 + k, s.bx0 + r);
+                s.r.ybed[r][k + 1] = face_bed<true>(d, p, t, blk.by0 + k, blk.bx0 + r);
         }
     }
     // the neighbour tiles' own beds at the shared edge faces; in the last
     // stage a ghost neighbour's copy of the shared vertices is the one the
     // redistribution may have written (intermed3, src/Redistribute.f90:362-410)
-    if (tid < B) {
+    if (!blk.flat && tid < B) {
         // the sides that apply, whether the neighbour is a ghost (in the last
         // stage of a morphodynamic step), then the loads issued together and
         // stored after: one round trip rather than one per side
         const int r = tid;
         const bool ovl = STAGE == 4 && d.morpho;
-        const bool sx0 = r < bya && s.bx0 == 0, sx1 = r < bya && s.bx0 + bxa == p.nx;
-        const bool sy0 = !Smem::oned && r < bxa && s.by0 == 0;
-        const bool sy1 = !Smem::oned && r < bxa && s.by0 + bya == p.ny;
-        const int row = (s.by0 + r) * (p.nx + 1), col = s.bx0 + r;
+        const bool sx0 = r < bya && blk.bx0 == 0, sx1 = r < bya && blk.bx0 + bxa == p.nx;
+        const bool sy0 = !Smem::oned && r < bxa && blk.by0 == 0;
+        const bool sy1 = !Smem::oned && r < bxa && blk.by0 + bya == p.ny;
+        const int row = (blk.by0 + r) * (p.nx + 1), col = blk.bx0 + r;
         const int tW = nb_tile(p, t, -1, 0), tE = nb_tile(p, t, 1, 0);
         const int tS = Smem::oned ? t : nb_tile(p, t, 0, -1), tN = Smem::oned ? t : nb_tile(p, t, 0, 1);
         const bool gW = ovl && sx0 && d.tstate[tW] != KST_TILE_ACTIVE;
@@ -1102,64 +1241,89 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         const bool gN = ovl && sy1 && d.tstate[tN] != KST_TILE_ACTIVE;
         double vW = 0.0, vE = 0.0, vS = 0.0, vN = 0.0;
         if (sx0)
-            vW = gW ? ghost_bed<Smem::oned>(d, p, tW, p.nx, s.by0 + r, p.nx, s.by0 + r + 1)
+            vW = gW ? ghost_bed<Smem::oned>(d, p, tW, p.nx, blk.by0 + r, p.nx, blk.by0 + r + 1)
                     : d.T.xib[tW * p.NFX + row + p.nx];
         if (sx1)
-            vE = gE ? ghost_bed<Smem::oned>(d, p, tE, 0, s.by0 + r, 0, s.by0 + r + 1) : d.T.xib[tE * p.NFX + row];
+            vE = gE ? ghost_bed<Smem::oned>(d, p, tE, 0, blk.by0 + r, 0, blk.by0 + r + 1) : d.T.xib[tE * p.NFX + row];
         if (sy0)
             vS = gS ? ghost_bed(d, p, tS, col, p.ny, col + 1, p.ny) : d.T.yib[tS * p.NFY + p.ny * p.nx + col];
         if (sy1) vN = gN ? ghost_bed(d, p, tN, col, 0, col + 1, 0) : d.T.yib[tN * p.NFY + col];
-        if (sx0) s.xside[0][r] = vW;
-        if (sx1) s.xside[1][r] = vE;
-        if (sy0) s.yside[0][r] = vS;
-        if (sy1) s.yside[1][r] = vN;
+        if (sx0) s.r.xside[0][r] = vW;
+        if (sx1) s.r.xside[1][r] = vE;
+        if (sy0) s.r.yside[0][r] = vS;
+        if (sy1) s.r.yside[1][r] = vN;
     }
     __syncthreads();
 
+    blk.nact = __builtin_amdgcn_readfirstlane(s.nact);
+    blk.solids = __builtin_amdgcn_readfirstlane(s.solids) != 0;
+
     // ---- phase B: face fluxes --------------------------------------------
     double cflm = kHuge;
+    constexpr bool CFL = STAGE != 4;
     // x-faces: consecutive lanes walk along a row; y-faces: along a row too
-    if (bxa == B && bya == BY && BY == B && STAGE_NT == 256) {
-        // 272 x-faces and 272 y-faces: one of each per thread, the 16 extra
-        // x-faces on wave 0 and the 16 extra y-faces on wave 1
-        face_work<false, VISC, LIM, STAGE != 4, MIX>(d, p, s, tid % (B + 1), tid / (B + 1), cflm);
-        face_work<true, VISC, LIM, STAGE != 4, MIX>(d, p, s, tid / B, tid % B, cflm);
-        if (tid < 16) {
-            const int f = 256 + tid;
-            face_work<false, VISC, LIM, STAGE != 4, MIX>(d, p, s, f % (B + 1), f / (B + 1), cflm);
-        } else if (tid >= 64 && tid < 80) {
-            const int f = 256 + tid - 64;
-            face_work<true, VISC, LIM, STAGE != 4, MIX>(d, p, s, f / B, f % B, cflm);
+    if constexpr (Smem::alias) {
+        // up to 272 x-faces and 272 y-faces: one of each per thread, the last
+        // 16 x-faces on wave 0 and the last 16 y-faces on wave 1
+        FaceFlux<MIX> fx, fy, fe;
+        const int xi = tid % (B + 1), xj = tid / (B + 1), yi = tid / B, yj = tid % B;
+        const bool xon = xi <= bxa && xj < bya, yon = yj < bxa && yi <= bya;
+        if (xon) face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, xi, xj, cflm, fx);
+        if (yon) face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, yi, yj, cflm, fy);
+        const bool xe = tid < 16, ye = tid >= 64 && tid < 80;
+        const int ei = xe ? (256 + tid) % (B + 1) : B, ej = xe ? (256 + tid) / (B + 1) : tid - 64;
+        const bool eon = xe ? (ei <= bxa && ej < bya) : (ye && ej < bxa && bya == BY);
+        if (xe) {
+            if (eon) face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, ei, ej, cflm, fe);
+        } else if (ye) {
+            if (eon) face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, ei, ej, cflm, fe);
         }
+        if (!MIX && own) {
+            // the owned cell's variables from LDS and its topography again,
+            // rather than registers held over the face pass
+            const int r = rg(tx, ty);
+            ow = s.r.w[r]; oh = s.r.h[r]; ou = s.r.u[r]; ov = s.r.v[r]; orho = s.r.rho[r];
+            ob0 = ld(d.b0c, oidx); obt = blk.flat ? 0.0 : ld(d.T.btc, oidx); og = ld(d.T.cgam, oidx);
+            if (STASH) { oru = s.mom[0][tid]; orv = s.mom[1][tid]; }
+            if (STAGE == 2) { pw = ld(d.Uw, oidx); pru = ld(d.Uu, oidx); prv = ld(d.Uv, oidx); ph = ld(d.Uh, oidx); }
+            else if (STAGE >= 3) { const double* S = (STAGE == 3) ? d.S2 : d.S3; oru = ld(S + FS, oidx); orv = ld(S + 2 * (size_t)FS, oidx); }
+        }
+        load_cell();
+        if (CFL) wave_min(s, cflm);
+        __syncthreads();
+        if (xon) put_flux<false, MIX>(s, xi, xj, fx);
+        if (yon) put_flux<true, MIX>(s, yi, yj, fy);
+        if (xe && eon) put_flux<false, MIX>(s, ei, ej, fe);
+        if (ye && eon) put_flux<true, MIX>(s, ei, ej, fe);
     } else if (pre) {
         bool yf;
         const int f = split_item(tid, Smem::NFX, Smem::NFY, &yf);
+        FaceFlux<MIX> F;
         if (f >= 0) {
-            if (!yf) face_work<false, VISC, LIM, STAGE != 4, MIX>(d, p, s, f % (B + 1), f / (B + 1), cflm, &pft);
-            else face_work<true, VISC, LIM, STAGE != 4, MIX>(d, p, s, f / B, f % B, cflm, &pft);
-        }
-    } else if (bxa == B && bya == BY) {
-        // x- and y-faces as one list over the block
-        for (int f = tid; f < Smem::NFX + Smem::NFY; f += STAGE_NT) {
-            if (f < Smem::NFX) {
-                face_work<false, VISC, LIM, STAGE != 4, MIX>(d, p, s, f % (B + 1), f / (B + 1), cflm);
+            if (!yf) {
+                face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, f % (B + 1), f / (B + 1), cflm, F, &pft);
+                put_flux<false, MIX>(s, f % (B + 1), f / (B + 1), F);
             } else {
-                const int g = f - Smem::NFX;
-                face_work<true, VISC, LIM, STAGE != 4, MIX>(d, p, s, g / B, g % B, cflm);
+                face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, f / B, f % B, cflm, F, &pft);
+                put_flux<true, MIX>(s, f / B, f % B, F);
             }
         }
+        if (CFL) wave_min(s, cflm);
     } else {
-        for (int f = tid; f < (bxa + 1) * bya; f += STAGE_NT)
-            face_work<false, VISC, LIM, STAGE != 4, MIX>(d, p, s, f % (bxa + 1), f / (bxa + 1), cflm);
+        FaceFlux<MIX> F;
+        for (int f = tid; f < (bxa + 1) * bya; f += STAGE_NT) {
+            face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, f % (bxa + 1), f / (bxa + 1), cflm, F);
+            put_flux<false, MIX>(s, f % (bxa + 1), f / (bxa + 1), F);
+        }
         if constexpr (!Smem::oned)   // no y faces on a 1D grid (src/HydraulicRHS.f90:1075)
-            for (int f = tid; f < (bya + 1) * bxa; f += STAGE_NT)
-                face_work<true, VISC, LIM, STAGE != 4, MIX>(d, p, s, f / bxa, f % bxa, cflm);
+            for (int f = tid; f < (bya + 1) * bxa; f += STAGE_NT) {
+                face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, f / bxa, f % bxa, cflm, F);
+                put_flux<true, MIX>(s, f / bxa, f % bxa, F);
+            }
+        if (CFL) wave_min(s, cflm);
     }
-    if (STAGE != 4) {
-        reduce_min_to(s, cflm, &d.ctrl->slot[(d.second ? 3 : 0) + STAGE - 1].bits);
-    } else {
-        __syncthreads();
-    }
+    __syncthreads();
+    if (CFL) block_min_to(s, &d.ctrl->slot[(d.second ? 3 : 0) + STAGE - 1].bits);
 
     // ---- phase C: RHS of the owned cell and the stage update -------------
     if (!own) return more;
@@ -1167,10 +1331,14 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 #define FX(q, o) fluxv<MIX, false>(s, q, xs + (o))
 #define FY(q, o) fluxv<MIX, true>(s, q, ys + (o))
     const double gam = og;
-    const double bx = prec ? pbx : d.T.cbx[oidx], by = prec ? pby : d.T.cby[oidx];
+    const double bx = pbx, by = pby;
     // prefactors (1+by^2)/gam, -(bx by/gam), (1+bx^2)/gam are per-bed topography
-    const double gxu = prec ? pgxu : d.T.pxu[oidx], gxv = prec ? pgxv : d.T.pxv[oidx], gyu = gxv;
-    const double gyv = prec ? pgyv : d.T.pyv[oidx];
+    const double gxu = pgxu, gxv = pgxv, gyu = gxv;
+    const double gyv = pgyv;
+    if (Smem::alias && !MIX) {
+        ohn = compute_hn(ow, ob0, obt, gam);
+        if (ohn < 0.0) ohn = 0.0;
+    }
     // ConstructHydraulicRHS (src/HydraulicRHS.f90:1228-1271; on a 1D grid
     // :1276-1294, x fluxes only and the hydrostatic term divided by gamma)
     double stw, sth, stu, stv;
@@ -1219,7 +1387,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     if (p.n_sources > 0 && d.has_src[t]) {
         double Qt = 0.0, psiQt = 0.0;
         const int ti = t % p.ntx, tj = t / p.ntx;
-        const int i = s.bx0 + tx, j = s.by0 + ty;
+        const int i = blk.bx0 + tx, j = blk.by0 + ty;
         const double x = -0.5 * p.x_size + p.dx * (((ti + 1) - 1.0) * p.nx + ((i + 1) - 0.5));
         const double y = -0.5 * p.y_size + p.dy * (((tj + 1) - 1.0) * p.ny + ((j + 1) - 0.5));
         flux_sources(d, p, s.tstage, s.tgrid, x, y, Qt, psiQt);
@@ -1234,17 +1402,6 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     hpg = hpg / gam;
     const double Eu = stu + (0.0 - p.g * orho * hpg * bx);
     const double Ev = stv + (0.0 - p.g * orho * hpg * by);
-    // DragClosure + ImplicitSourceTerms (src/Equations.f90:627-658)
-    double Im = 0.0;
-    if (ohn > p.hthr) {
-        const double fric = drag(p, ohn, ou, ov, opsi, bx, by, gam);
-        const double modu = sqrt(speed2(p.geometric, ou, ov, bx, by));
-        if (modu > 1.0e-8) {
-            const double hr = 1.0 / ohn;
-            Im = -(fric * hr / modu);
-        }
-    }
-
     if (STAGE == 1) {
         if constexpr (MIX) {
             float* Rf = (float*)d.R;
@@ -1277,8 +1434,8 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         }
     } else if (STAGE == 3) {
         // third SSP substep (src/TimeStepper.f90:466-498)
-        const double w0 = MIX ? pw : (pre ? pw0 : d.Uw[oidx]), u0 = MIX ? pru : (pre ? pu0 : d.Uu[oidx]);
-        const double v0 = MIX ? prv : (pre ? pv0 : d.Uv[oidx]), h0 = MIX ? ph : (pre ? ph0 : d.Uh[oidx]);
+        const double w0 = MIX ? pw : pw0, u0 = MIX ? pru : pu0;
+        const double v0 = MIX ? prv : pv0, h0 = MIX ? ph : ph0;
         const double third = 1.0 / 3.0, twothird = 2.0 / 3.0;
         const double u3 = third * u0 + twothird * (oru + dt * Eu) / (1.0 - dt * Im);
         const double v3 = third * v0 + twothird * (orv + dt * Ev) / (1.0 - dt * Im);
@@ -1336,7 +1493,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         // activation flags from this state's Hn (CheckIfNearBoundaries,
         // src/TimeStepper.f90:946-1150): bit 0 N, 1 S, 2 E, 3 W
         if (d.last && ohn > p.hthr) {
-            const int i = s.bx0 + tx, j = s.by0 + ty, tb = p.tile_buffer;
+            const int i = blk.bx0 + tx, j = blk.by0 + ty, tb = p.tile_buffer;
             unsigned f = 0;
             if (j + 1 > p.ny - tb) f |= 1u;
             if (j + 1 <= tb) f |= 2u;
@@ -1350,8 +1507,17 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 
 // The grid is sized for the active set the host last saw (with room to
 // grow); a block whose share of the list holds more items takes them in turn.
+// The 16 x 16 shape is bound by latency and VALU issue: it is held to 128
+// VGPRs (4 waves a SIMD) by what phase B does not hold in registers -- the
+// drag closures are evaluated before it, the owned cell is read again after
+// it -- and, where a region carries no solids, by what it does not compute.
+// Plain 2048^2 (1.66 M active cells, clear water), stages 1..4: 154, 164,
+// 160, 166 us at 3 waves a SIMD with every array read, 127, 151, 134, 140 us
+// now (stage 2 spills 15 registers; at 3 waves without the spills it takes
+// 160 us).  Not reading the face and cell bt of a flat bed (8 of 31 words a
+// cell) by itself changed nothing at 3 waves.
 template <int STAGE, bool VISC, int LIM, bool MIX = false, int BY = B, bool ONED = false>
-__global__ __launch_bounds__(STAGE_NT) void stage_kernel(const Dev* __restrict__ d,
+__global__ __launch_bounds__(STAGE_NT, BY == B ? 4 : 1) void stage_kernel(const Dev* __restrict__ d,
                                                          const Params* __restrict__ p) {
     __shared__ SmemT<VISC ? 7 : 5, MIX, BY, ONED> s;
     for (int pass = 0; stage_body<STAGE, VISC, LIM, MIX>(const_arg(d), *p, s, -1, pass); ++pass)
@@ -2312,7 +2478,7 @@ __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt
 // contiguous eighth of it, so neighbouring sub-blocks share an L2.
 // second: the second hydraulic operator of the morphodynamic slots (dev2, off2)
 template <int STAGE, bool VISC, int LIM, bool MIX>
-__global__ __launch_bounds__(STAGE_NT) void batch_stage_kernel(Batch bt, int second) {
+__global__ __launch_bounds__(STAGE_NT, 4) void batch_stage_kernel(Batch bt, int second) {
     __shared__ SmemT<VISC ? 7 : 5, MIX> s;
     __shared__ int sh_slot;
     const int* off = second ? bt.off2 : bt.off;
@@ -2952,6 +3118,10 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
     // mixed precision covers the hydraulic operator only
     if (cfg->precision == KST_PREC_MIXED && cfg->morphodynamics) return KST_ERR_CONFIG;
     if (cfg->n_sources > 0 && !cfg->sources) return KST_ERR_CONFIG;
+    // 32-bit byte offsets into every per-tile array (a grid beyond them would
+    // need several times the device's memory)
+    const double per_tile = (double)(cfg->nx_per_tile + 1) * (cfg->ny_per_tile + 1) * 8.0;
+    if (per_tile * cfg->nx_tiles * cfg->ny_tiles >= 4294967296.0) return KST_ERR_CONFIG;
     kst_handle* h = new kst_handle();
     h->cfg = *cfg;
     h->cfg.sources = nullptr;
@@ -3162,6 +3332,7 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                 if (st[n] == KST_TILE_OFF) { st[n] = KST_TILE_GHOST; gh.push_back(n); }
             }
     }
+    bool flat = true;
     // vertex bt: each active tile takes its own copy of the global values
     // (ghost tiles keep bt = 0, as AllocateTopographicData leaves them),
     // then the topography of every set follows
@@ -3177,6 +3348,8 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                     for (int i = 0; i <= nx; ++i)
                         dst[j * NV1 + i] = btv[(size_t)(tj * ny + j) * (h->NX + 1) + ti * nx + i];
             }
+        // all +0 to the last bit
+        for (size_t q = 0; btv && flat && q < tv.size(); ++q) flat = tv[q] == 0.0 && !std::signbit(tv[q]);
         Topo* sets[4] = {&h->d.TA, &h->d.TB, &h->d.TM[0], &h->d.TM[1]};
         for (int q = 0; q < (h->d.morpho ? 4 : 1); ++q)
             HIPCHK(h, hipMemcpy(sets[q]->vbt, tv.data(), tv.size() * 8, hipMemcpyHostToDevice));
@@ -3287,6 +3460,7 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
     c.status = ST_DONE;
     c.n_active = (int)act.size();
     c.n_ghost = (int)gh.size();
+    c.flat = h->d.morpho ? 0 : (int)flat;
     int rc = write_ctrl(h, &c);
     if (rc) return rc;
     if (!gh.empty())
@@ -3570,6 +3744,11 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
     Ctrl c;
     int rc = read_ctrl(h, &c);
     if (rc) return rc;
+    if (c.flat) {   // the cells' bt may now differ from the vertices'
+        c.flat = 0;
+        rc = write_ctrl(h, &c);
+        if (rc) return rc;
+    }
     HIPCHK(h, hipMemset(h->d.eflags, 0, (size_t)h->ntiles * 4));
     if (c.n_active > 0)
         hipLaunchKernelGGL(init_flags_kernel, dim3(c.n_active), dim3(256), 0, h->stream, h->d, h->p);
