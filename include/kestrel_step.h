@@ -264,7 +264,8 @@ int kst_set_grid_cap(kst_handle* h, int tiles);
  * one CPU thread).  With enable != 0 the library times, before the first
  * launch on each new bucket of active-set sizes (active tiles rounded up to a
  * power of two), the first RK stage kernel in each candidate launch shape --
- * 16 x 16 sub-blocks on the default grid, on a grid of the blocks the device
+ * the wide sub-blocks (up to 256 cells in the shape that covers a tile in the
+ * fewest; 16 x 16 in tiles of 32) on the default grid, on a grid of the blocks the device
  * holds at once (blocks then take further sub-blocks in turn) or twice that,
  * and 16 x 4 sub-blocks (FP64) -- and launches that bucket in the fastest.
  * Choices are cached for the process per grid layout, operator and bucket,
@@ -275,7 +276,7 @@ int kst_set_grid_cap(kst_handle* h, int tiles);
  * choices. */
 int kst_autotune(kst_handle* h, int enable);
 /* The choices made so far, at most max: per bucket, whether 16 x 4
- * sub-blocks were chosen, the grid limit of the 16 x 16 shape (0: default
+ * sub-blocks were chosen, the grid limit of the wide shape (0: default
  * grid) and the stage-1 launch time in microseconds of the four candidates
  * in the order above (0: not tried).  Returns the number written. */
 int kst_autotune_choices(const kst_handle* h, int max, int32_t* bucket, int32_t* small,

@@ -41,7 +41,17 @@ struct Params {
     double bc_hn, bc_u, bc_v, bc_psi, bc_rho;
     // a 1D grid (isOneD: nYtiles * nYpertile = 1, src/DomainSettings.f90:216-220)
     int oned;
+    // the wide stage kernels' sub-block (wide_shape): width and height,
+    // sub-blocks per tile along x and in all, and the factors that divide by
+    // sw, sw + 1, sw + 3 and sh + 3 (small_div)
+    int sw, sh, sbx, spt;
+    unsigned dsw, dsw1, dsw3, dsh3;
 };
+
+// x / d for x < 1024 and d <= 64: a multiplication by ceil(2^16 / d) (its
+// excess over 2^16 / d is below 1, which x d < 2^16 keeps out of the result).
+__host__ __device__ __forceinline__ unsigned div_factor(int d) { return (65536u + d - 1) / d; }
+__host__ __device__ __forceinline__ int small_div(int x, unsigned f) { return (int)(((unsigned)x * f) >> 16); }
 
 __device__ __forceinline__ double dmin(double a, double b) { return (a < b) ? a : b; }
 __device__ __forceinline__ double dmax(double a, double b) { return (a > b) ? a : b; }

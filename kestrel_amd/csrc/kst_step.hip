@@ -16,6 +16,7 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -355,7 +356,9 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
 
 // Working set of one sub-block.  With MIX the per-cell Hnpsi, u, v and the
 // fluxes other than the hydrostatic one (q = 4, in fx4/fy4) are float.
-// BY: the sub-block's height (B or B/4); the region is RW x (BY + 4) cells.
+// BY = B: the wide shape, up to 256 cells in the proportions that suit the
+// tile (Params::sw x sh, wide_shape; the arrays are sized for the largest);
+// BY = B/4: 16 x 4.  The region is the sub-block and 2 cells on every side.
 // ONED: a 1D grid (one row of cells), which also keeps the conserved rhoHnv
 // for its x-face reconstruction.
 // The fluxes of a 16 x 16 sub-block take the place of what the face pass
@@ -363,25 +366,28 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
 // the two), which leaves room for four workgroups on a CU instead of three
 // (48 -> 26 KB a workgroup); the 16 x 4 shape keeps them apart, since its
 // launches never fill a CU and the extra barrier would lengthen each.
+constexpr int WIDE_REG = 432, WIDE_BED = 352, WIDE_EDGE = 32, WIDE_FACES = 288, WIDE_HALO = 160;
 template <int NQ, bool MIX, int BY, bool ONED>
 struct RegionT {
     using FT = typename std::conditional<MIX, float, double>::type;
-    static constexpr int NR = RW * (BY + 4);       // region cells
+    static constexpr int NR = BY == B ? WIDE_REG : RW * (BY + 4);       // region cells
+    static constexpr int NXB = BY == B ? WIDE_BED : BY * (B + 3), NYB = BY == B ? WIDE_BED : B * (BY + 3);
+    static constexpr int NS = BY == B ? WIDE_EDGE : B;
     double w[NR];
     FT h[NR], u[NR], v[NR];
     double rho[NR];
     double rv[ONED ? NR : 1];  // 1D: the conserved rhoHnv
-    double xbed[BY][B + 3];  // CorrectSlopes bed of x-faces -1..B+1 of each row (relative)
-    double ybed[B][BY + 3];  // CorrectSlopes bed of y-faces -1..BY+1 of each column
-    double xside[2][BY];     // the W / E tile's own bed at this tile's edge x-faces
-    double yside[2][B];      // the S / N tile's own bed at this tile's edge y-faces
+    double xbed[NXB];        // CorrectSlopes bed of x-faces -1..sw+1 of each row (relative)
+    double ybed[NYB];        // CorrectSlopes bed of y-faces -1..sh+1 of each column
+    double xside[2][NS];     // the W / E tile's own bed at this tile's edge x-faces
+    double yside[2][NS];     // the S / N tile's own bed at this tile's edge y-faces
 };
 
 template <int NQ, bool MIX, int BY>
 struct FluxT {
     using FT = typename std::conditional<MIX, float, double>::type;
-    static constexpr int NFX = (B + 1) * BY;       // x-faces
-    static constexpr int NFY = B * (BY + 1);       // y-faces
+    static constexpr int NFX = BY == B ? WIDE_FACES : (B + 1) * BY;       // x-faces
+    static constexpr int NFY = BY == B ? WIDE_FACES : B * (BY + 1);       // y-faces
     FT fx[NQ][NFX];          // hw, hru, hrv, hh, g (, pu, pv with eddy viscosity)
     FT fy[NQ][NFY];
     double fx4[MIX ? NFX : 1], fy4[MIX ? NFY : 1];
@@ -427,6 +433,7 @@ struct FaceFlux {
 };
 
 __device__ __forceinline__ int rg(int rx, int ry) { return (ry + 2) * RW + (rx + 2); }
+__device__ __forceinline__ int rgi(int rx, int ry, int rw) { return (ry + 2) * rw + (rx + 2); }
 
 // Map a cell given relative to tile t (i in [-2, nx+1], j in [-2, ny+1], not
 // both outside) to (tile, ci, cj).
@@ -479,6 +486,7 @@ __device__ __forceinline__ FaceTopo load_face_topo_at(const DevT& d, const Param
 // the bed is flat (Ctrl::flat).
 struct Block {
     int t, bx0, by0, nact;
+    int sw, sh;              // the sub-block's shape
     bool flat;
     bool solids;             // some cell of the region has Hnpsi other than 0
     const double* Un;        // u^n of the step (a ghost cell's stored w)
@@ -509,8 +517,9 @@ __device__ __forceinline__ void face_flux(const DevT& d, const Params& p, const 
                                           int fj, double& cfl_min, const FaceTopo& ft, FaceFlux<false>& F) {
     const auto& s = sm.r;
     int iLL, iL, iR, iRR;
-    if (!YDIR) { iLL = rg(fi - 2, fj); iL = rg(fi - 1, fj); iR = rg(fi, fj); iRR = rg(fi + 1, fj); }
-    else       { iLL = rg(fj, fi - 2); iL = rg(fj, fi - 1); iR = rg(fj, fi); iRR = rg(fj, fi + 1); }
+    const int rw = blk.sw + 4, st = YDIR ? rw : 1;       // region stride along y, and along the normal
+    iR = YDIR ? rgi(fj, fi, rw) : rgi(fi, fj, rw);
+    iL = iR - st; iLL = iL - st; iRR = iR + st;
     const double dxr = YDIR ? p.dyr : p.dxr;
     const double dx = YDIR ? p.dy : p.dx;
     const int nn = YDIR ? p.ny : p.nx;
@@ -566,7 +575,7 @@ __device__ __forceinline__ void face_flux(const DevT& d, const Params& p, const 
     // beds of the faces of L and R (InterpolateB, src/HydraulicRHS.f90:741-753);
     // the face itself is entry fi + 1, except at a tile edge, where the cell
     // on the far side sees its own tile's copy of the shared vertices
-    const double* bed = YDIR ? &s.ybed[fj][0] : &s.xbed[fj][0];
+    const double* bed = YDIR ? &s.ybed[fj * (blk.sh + 3)] : &s.xbed[fj * (blk.sw + 3)];
     const double bWL = bed[fi], bER = bed[fi + 2];
     const double bF = bed[fi + 1];
     double fbL = bF, fbR = bF;
@@ -685,8 +694,9 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
                                                 FaceFlux<true>& F) {
     const auto& s = sm.r;
     int iLL, iL, iR, iRR;
-    if (!YDIR) { iLL = rg(fi - 2, fj); iL = rg(fi - 1, fj); iR = rg(fi, fj); iRR = rg(fi + 1, fj); }
-    else       { iLL = rg(fj, fi - 2); iL = rg(fj, fi - 1); iR = rg(fj, fi); iRR = rg(fj, fi + 1); }
+    const int rw = blk.sw + 4, st = YDIR ? rw : 1;       // region stride along y, and along the normal
+    iR = YDIR ? rgi(fj, fi, rw) : rgi(fi, fj, rw);
+    iL = iR - st; iLL = iL - st; iRR = iR + st;
     const double dxr = YDIR ? p.dyr : p.dxr;
     const double dx = YDIR ? p.dy : p.dx;
     const float dxrf = (float)dxr, hdx = (float)(0.5 * dx);
@@ -734,7 +744,7 @@ __device__ __forceinline__ void face_flux_mixed(const DevT& d, const Params& p, 
     // FP64: w face values, beds and CorrectSlopes (as face_flux)
     const double wEL = wL + sLw * hdxd;
     const double wWR = wR - sRw * hdxd;
-    const double* bed = YDIR ? &s.ybed[fj][0] : &s.xbed[fj][0];
+    const double* bed = YDIR ? &s.ybed[fj * (blk.sh + 3)] : &s.xbed[fj * (blk.sw + 3)];
     const double bWL = bed[fi], bER = bed[fi + 2];
     const double bF = bed[fi + 1];
     double fbL = bF, fbR = bF;
@@ -875,8 +885,8 @@ __device__ __forceinline__ void face_work(const DevT& d, const Params& p, const 
 }
 
 template <bool YDIR, bool MIX, typename Smem>
-__device__ __forceinline__ void put_flux(Smem& s, int fi, int fj, const FaceFlux<MIX>& F) {
-    const int i = YDIR ? (fi * B + fj) : (fj * (B + 1) + fi);
+__device__ __forceinline__ void put_flux(Smem& s, const Block& blk, int fi, int fj, const FaceFlux<MIX>& F) {
+    const int i = YDIR ? (fi * blk.sw + fj) : (fj * (blk.sw + 1) + fi);
 #pragma unroll
     for (int q = 0; q < Smem::NQ; ++q) {
         if (q == 4) {
@@ -961,7 +971,9 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     asm("" : "+v"(tidu) : "s"(pass));
     const int tid = (int)(tidu & (STAGE_NT - 1));
     if (tid == 0) {
-        const int sbx = (p.nx + B - 1) / B, sby = (p.ny + BY - 1) / BY, spt = sbx * sby;
+        const int sbx = Smem::alias ? p.sbx : (p.nx + B - 1) / B;
+        const int spt = Smem::alias ? p.spt : sbx * ((p.ny + BY - 1) / BY);
+        const int sw = Smem::alias ? p.sw : B, sh = Smem::alias ? p.sh : BY;
         constexpr bool SPEC = BY < B;
         int wspec = 0, tspec = 0;
         if (SPEC && witem < 0) {
@@ -1004,10 +1016,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         if (!skip) {
             s.tile = spec ? tspec : d.active[w / spt];
             const int sub = w % spt;
-            s.bx0 = (sub % sbx) * B;
-            s.by0 = (sub / sbx) * BY;
-            s.bxa = min(B, p.nx - s.bx0);
-            s.bya = min(BY, p.ny - s.by0);
+            s.bx0 = (sub % sbx) * sw;
+            s.by0 = (sub / sbx) * sh;
+            s.bxa = min(sw, p.nx - s.bx0);
+            s.bya = min(sh, p.ny - s.by0);
         }
         s.skip = skip;
         s.more = more;
@@ -1027,6 +1039,8 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     blk.t = t;
     blk.bx0 = __builtin_amdgcn_readfirstlane(s.bx0);
     blk.by0 = __builtin_amdgcn_readfirstlane(s.by0);
+    blk.sw = Smem::alias ? p.sw : B;
+    blk.sh = Smem::alias ? p.sh : BY;
     blk.flat = __builtin_amdgcn_readfirstlane(s.flat) != 0;
     blk.Un = Un;
     // whether the neighbour tiles are active, for the face pass (wave 3: its
@@ -1040,18 +1054,18 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     }
 
     // ---- phase A: stage state + derived variables on the region ----------
-    const int tx = tid % B, ty = tid / B;
+    const int sw = blk.sw, sh = blk.sh, rw = sw + 4;
+    const int ty = Smem::alias ? small_div(tid, p.dsw) : tid / B, tx = tid - ty * sw;
     const bool own = (tx < bxa) && (ty < bya);
     double ow = 0, oru = 0, orv = 0, oh = 0, ohn = 0, ou = 0, ov = 0, opsi = 0, orho = 0;
     double ob0 = 0, obt = 0, og = 1;
     double pw = 0, pru = 0, prv = 0, ph = 0;   // u^n of the owned cell (stage 2; mixed: 2..4)
     unsigned oidx = 0;
-    // threads 0..OWN-1: the owned cells; the 2-cell halo strips (4 strips of
-    // 2 x 16 slots) by the next 128 threads in the same round when there are
-    // enough, else by threads 128..255 in a second round (waves 0 and 1 take
-    // the extra faces of phase B instead)
-    constexpr int OWN = B * BY;
-    constexpr bool one_round = STAGE_NT >= OWN + 128;
+    // threads 0..OWN-1: the owned cells; the 2-cell halo strips by the next
+    // 128 threads in the same round (16 x 4), or from the last thread down in
+    // a second round (wide: waves 0 and 1 take the extra faces of phase B)
+    const int OWN = sw * sh;
+    constexpr bool one_round = STAGE_NT >= B * BY + 128;
     // A sub-block with at most one face per thread (the small shape) issues
     // its other global loads ahead of the state's so that they overlap: the
     // CorrectSlopes beds of its faces here (kept in a register until the
@@ -1074,16 +1088,30 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     for (int round = 0; round < (one_round ? 1 : 2); ++round) {
         int rx, ry;
         bool valid;
-        const int hq = one_round ? tid - OWN : tid - 128;
+        const int hq = one_round ? tid - OWN : STAGE_NT - 1 - tid;
         if (round == 0 && tid < OWN) {
             rx = tx; ry = ty; valid = own;
-        } else {
+        } else if constexpr (one_round) {
             if (hq < 0 || hq >= 128) break;
             const int strip = hq >> 5, k = hq & 31, dd = k >> 4, pos = k & 15;
             if (strip == 0) { rx = -2 + dd; ry = pos; valid = pos < bya; }
             else if (strip == 1) { rx = bxa + dd; ry = pos; valid = pos < bya; }
             else if (strip == 2) { rx = pos; ry = -2 + dd; valid = pos < bxa && !Smem::oned; }
             else { rx = pos; ry = bya + dd; valid = pos < bxa && !Smem::oned; }   // no rows beyond a 1D grid's
+        } else {
+            if (round == 0) continue;
+            if (hq >= 4 * (sw + sh)) break;
+            if (hq < 4 * sh) {       // W and E: two cells of each row
+                const int e = hq >= 2 * sh, k = hq - (e ? 2 * sh : 0);
+                ry = k >> 1;
+                rx = (e ? bxa : -2) + (k & 1);
+                valid = ry < bya;
+            } else {                 // S and N: two rows
+                const int k = hq - 4 * sh, l = small_div(k, p.dsw);
+                rx = k - l * sw;
+                ry = l < 2 ? l - 2 : bya + l - 2;
+                valid = rx < bxa;
+            }
         }
         if (!valid) continue;
         int tc, ci, cj;
@@ -1147,7 +1175,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             hn = p.bc_hn; psi = p.bc_psi; rho = p.bc_rho; uu = p.bc_u; vv = p.bc_v;
         }
         solids |= h != 0.0 || psi != 0.0;
-        const int r = rg(rx, ry);
+        const int r = rgi(rx, ry, rw);
         if constexpr (Smem::oned) s.r.rv[r] = rv;
         s.r.w[r] = w; s.r.h[r] = h; s.r.u[r] = uu; s.r.v[r] = vv; s.r.rho[r] = rho;
         if (round == 0) {
@@ -1209,21 +1237,24 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         bool yb;
         const int q = split_item(tid, NXB, NYB, &yb);
         if (q >= 0) {
-            if (!yb) s.r.xbed[q / (B + 3)][q % (B + 3)] = bedv;
-            else s.r.ybed[q / (BY + 3)][q % (BY + 3)] = bedv;
+            if (!yb) s.r.xbed[q] = bedv;
+            else s.r.ybed[q] = bedv;
         }
     } else {
-        for (int q = tid; q < B * (B + 3); q += STAGE_NT) {
-            const int r = q / (B + 3), k = q % (B + 3) - 1;
-            if (r < bya && k <= bxa + 1) s.r.xbed[r][k + 1] = face_bed<false>(d, p, t, blk.bx0 + k, blk.by0 + r);
-            if (!Smem::oned && r < bxa && k <= bya + 1)
-                s.r.ybed[r][k + 1] = face_bed<true>(d, p, t, blk.by0 + k, blk.bx0 + r);
+        const int nbx = sh * (sw + 3), nby = Smem::oned ? 0 : sw * (sh + 3);
+        for (int q = tid; q < nbx || q < nby; q += STAGE_NT) {
+            const int rX = Smem::alias ? small_div(q, p.dsw3) : q / (B + 3), kX = q - rX * (sw + 3) - 1;
+            if (rX < bya && kX <= bxa + 1) s.r.xbed[q] = face_bed<false>(d, p, t, blk.bx0 + kX, blk.by0 + rX);
+            if (!Smem::oned) {
+                const int rY = Smem::alias ? small_div(q, p.dsh3) : q / (BY + 3), kY = q - rY * (sh + 3) - 1;
+                if (rY < bxa && kY <= bya + 1) s.r.ybed[q] = face_bed<true>(d, p, t, blk.by0 + kY, blk.bx0 + rY);
+            }
         }
     }
     // the neighbour tiles' own beds at the shared edge faces; in the last
     // stage a ghost neighbour's copy of the shared vertices is the one the
     // redistribution may have written (intermed3, src/Redistribute.f90:362-410)
-    if (!blk.flat && tid < B) {
+    if (!blk.flat && tid < (Smem::alias ? WIDE_EDGE : B)) {
         // the sides that apply, whether the neighbour is a ghost (in the last
         // stage of a morphodynamic step), then the loads issued together and
         // stored after: one round trip rather than one per side
@@ -1263,16 +1294,17 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     constexpr bool CFL = STAGE != 4;
     // x-faces: consecutive lanes walk along a row; y-faces: along a row too
     if constexpr (Smem::alias) {
-        // up to 272 x-faces and 272 y-faces: one of each per thread, the last
-        // 16 x-faces on wave 0 and the last 16 y-faces on wave 1
+        // up to 288 x-faces and 288 y-faces: one of each per thread, the rest
+        // of the x-faces on wave 0 and of the y-faces on wave 1
         FaceFlux<MIX> fx, fy, fe;
-        const int xi = tid % (B + 1), xj = tid / (B + 1), yi = tid / B, yj = tid % B;
+        const int xj = small_div(tid, p.dsw1), xi = tid - xj * (sw + 1), yi = ty, yj = tx;
         const bool xon = xi <= bxa && xj < bya, yon = yj < bxa && yi <= bya;
         if (xon) face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, xi, xj, cflm, fx);
         if (yon) face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, yi, yj, cflm, fy);
-        const bool xe = tid < 16, ye = tid >= 64 && tid < 80;
-        const int ei = xe ? (256 + tid) % (B + 1) : B, ej = xe ? (256 + tid) / (B + 1) : tid - 64;
-        const bool eon = xe ? (ei <= bxa && ej < bya) : (ye && ej < bxa && bya == BY);
+        const bool xe = tid < 64, ye = tid >= 64 && tid < 128;
+        const int ef = STAGE_NT + (tid & 63), ed = small_div(ef, xe ? p.dsw1 : p.dsw);
+        const int ei = xe ? ef - ed * (sw + 1) : ed, ej = xe ? ed : ef - ed * sw;
+        const bool eon = xe ? (ei <= bxa && ej < bya) : (ye && ej < bxa && ei <= bya);
         if (xe) {
             if (eon) face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, ei, ej, cflm, fe);
         } else if (ye) {
@@ -1281,7 +1313,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         if (!MIX && own) {
             // the owned cell's variables from LDS and its topography again,
             // rather than registers held over the face pass
-            const int r = rg(tx, ty);
+            const int r = rgi(tx, ty, rw);
             ow = s.r.w[r]; oh = s.r.h[r]; ou = s.r.u[r]; ov = s.r.v[r]; orho = s.r.rho[r];
             ob0 = ld(d.b0c, oidx); obt = blk.flat ? 0.0 : ld(d.T.btc, oidx); og = ld(d.T.cgam, oidx);
             if (STASH) { oru = s.mom[0][tid]; orv = s.mom[1][tid]; }
@@ -1291,10 +1323,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         load_cell();
         if (CFL) wave_min(s, cflm);
         __syncthreads();
-        if (xon) put_flux<false, MIX>(s, xi, xj, fx);
-        if (yon) put_flux<true, MIX>(s, yi, yj, fy);
-        if (xe && eon) put_flux<false, MIX>(s, ei, ej, fe);
-        if (ye && eon) put_flux<true, MIX>(s, ei, ej, fe);
+        if (xon) put_flux<false, MIX>(s, blk, xi, xj, fx);
+        if (yon) put_flux<true, MIX>(s, blk, yi, yj, fy);
+        if (xe && eon) put_flux<false, MIX>(s, blk, ei, ej, fe);
+        if (ye && eon) put_flux<true, MIX>(s, blk, ei, ej, fe);
     } else if (pre) {
         bool yf;
         const int f = split_item(tid, Smem::NFX, Smem::NFY, &yf);
@@ -1302,10 +1334,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         if (f >= 0) {
             if (!yf) {
                 face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, f % (B + 1), f / (B + 1), cflm, F, &pft);
-                put_flux<false, MIX>(s, f % (B + 1), f / (B + 1), F);
+                put_flux<false, MIX>(s, blk, f % (B + 1), f / (B + 1), F);
             } else {
                 face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, f / B, f % B, cflm, F, &pft);
-                put_flux<true, MIX>(s, f / B, f % B, F);
+                put_flux<true, MIX>(s, blk, f / B, f % B, F);
             }
         }
         if (CFL) wave_min(s, cflm);
@@ -1313,12 +1345,12 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         FaceFlux<MIX> F;
         for (int f = tid; f < (bxa + 1) * bya; f += STAGE_NT) {
             face_work<false, VISC, LIM, CFL, MIX>(d, p, s, blk, f % (bxa + 1), f / (bxa + 1), cflm, F);
-            put_flux<false, MIX>(s, f % (bxa + 1), f / (bxa + 1), F);
+            put_flux<false, MIX>(s, blk, f % (bxa + 1), f / (bxa + 1), F);
         }
         if constexpr (!Smem::oned)   // no y faces on a 1D grid (src/HydraulicRHS.f90:1075)
             for (int f = tid; f < (bya + 1) * bxa; f += STAGE_NT) {
                 face_work<true, VISC, LIM, CFL, MIX>(d, p, s, blk, f / bxa, f % bxa, cflm, F);
-                put_flux<true, MIX>(s, f / bxa, f % bxa, F);
+                put_flux<true, MIX>(s, blk, f / bxa, f % bxa, F);
             }
         if (CFL) wave_min(s, cflm);
     }
@@ -1327,7 +1359,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 
     // ---- phase C: RHS of the owned cell and the stage update -------------
     if (!own) return more;
-    const int xs = ty * (B + 1) + tx, ys = ty * B + tx;
+    const int xs = ty * (sw + 1) + tx, ys = ty * sw + tx;
 #define FX(q, o) fluxv<MIX, false>(s, q, xs + (o))
 #define FY(q, o) fluxv<MIX, true>(s, q, ys + (o))
     const double gam = og;
@@ -1356,17 +1388,17 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         k3.add(VISC ? (FX(6, 1) - FX(6, 0)) : 0.0);
         stv = k3.s * p.dxr;
     } else {
-        stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam) + (FY(0, 0) - FY(0, B)) * p.dyr / (gam * gam);
-        sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, B)) * p.dyr / gam;
+        stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam) + (FY(0, 0) - FY(0, sw)) * p.dyr / (gam * gam);
+        sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, sw)) * p.dyr / gam;
         Kahan k1;
         k1.add(FX(1, 0) - FX(1, 1));
         k1.add((FX(4, 0) - FX(4, 1)) * gxu);
         k1.add(VISC ? (FX(5, 1) - FX(5, 0)) : 0.0);
         stu = k1.s * p.dxr;
         Kahan k2;
-        k2.add(FY(1, 0) - FY(1, B));
-        k2.add((FY(4, 0) - FY(4, B)) * gyu);
-        k2.add(VISC ? (FY(5, B) - FY(5, 0)) : 0.0);
+        k2.add(FY(1, 0) - FY(1, sw));
+        k2.add((FY(4, 0) - FY(4, sw)) * gyu);
+        k2.add(VISC ? (FY(5, sw) - FY(5, 0)) : 0.0);
         stu = stu + k2.s * p.dyr;
         Kahan k3;
         k3.add(FX(2, 0) - FX(2, 1));
@@ -1374,9 +1406,9 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         k3.add(VISC ? (FX(6, 1) - FX(6, 0)) : 0.0);
         stv = k3.s * p.dxr;
         Kahan k4;
-        k4.add(FY(2, 0) - FY(2, B));
-        k4.add((FY(4, 0) - FY(4, B)) * gyv);
-        k4.add(VISC ? (FY(6, B) - FY(6, 0)) : 0.0);
+        k4.add(FY(2, 0) - FY(2, sw));
+        k4.add((FY(4, 0) - FY(4, sw)) * gyv);
+        k4.add(VISC ? (FY(6, sw) - FY(6, 0)) : 0.0);
         stv = stv + k4.s * p.dyr;
     }
 #undef FX
@@ -2423,6 +2455,7 @@ struct Batch {
     const Dev* dev2;      // the second hydraulic operator of each slot (morphodynamic slots)
     int* off2;            // [nslot + 1] as off, morphodynamic slots only
     int* off3;            // [nslot + 1] (tile, part) items of the morphodynamic slots
+    int* off4;            // [nslot + 1] as off (the stage kernels' sub-blocks), morphodynamic slots only
 };
 
 constexpr int BATCH_PLAN_THREADS = 1024;
@@ -2437,11 +2470,12 @@ __global__ __launch_bounds__(ACT_NT) void batch_activate_kernel(Batch bt) {
 // Work list of the iteration: the running slots' active sub-blocks.
 // The iteration's work lists (exclusive prefix sums over the slots): off,
 // the running slots' sub-blocks; with morphodynamic slots (lists > 1) also
-// off2, theirs alone, and off3, their (tile, part) items.
+// theirs alone for the morphodynamic kernels (off2, 16 x 16) and the second
+// operator's stages (off4), and off3, their (tile, part) items.
 __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt, int lists) {
     __shared__ int sc[BATCH_PLAN_THREADS];
     for (int kind = 0; kind < lists; ++kind) {
-        int* off = kind == 0 ? bt.off : (kind == 1 ? bt.off2 : bt.off3);
+        int* off = kind == 0 ? bt.off : (kind == 1 ? bt.off2 : (kind == 2 ? bt.off3 : bt.off4));
         int carry = 0;
         for (int base = 0; base < bt.nslot; base += BATCH_PLAN_THREADS) {
             const int s = base + (int)threadIdx.x;
@@ -2452,7 +2486,8 @@ __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt
                 const Ctrl* c = d.ctrl;
                 const bool run = c->status == ST_NEW || c->status == ST_RETRY;
                 const int spt = ((p.nx + B - 1) / B) * ((p.ny + B - 1) / B);
-                if (kind == 0 && run) n = c->n_active * spt;
+                if (kind == 0 && run) n = c->n_active * p.spt;
+                if (kind == 3 && run && d.morpho) n = c->n_active * p.spt;
                 if (kind == 1 && run && d.morpho) n = c->n_active * spt;
                 if (kind == 2 && d.morpho) n = c->n_active * TILE_PARTS;
             }
@@ -2481,7 +2516,7 @@ template <int STAGE, bool VISC, int LIM, bool MIX>
 __global__ __launch_bounds__(STAGE_NT, 4) void batch_stage_kernel(Batch bt, int second) {
     __shared__ SmemT<VISC ? 7 : 5, MIX> s;
     __shared__ int sh_slot;
-    const int* off = second ? bt.off2 : bt.off;
+    const int* off = second ? bt.off4 : bt.off;
     const Dev* dev = second ? bt.dev2 : bt.dev;
     const int total = off[bt.nslot];
     const int m = gridDim.x / 8, x = blockIdx.x % 8;
@@ -2602,7 +2637,7 @@ struct kst_batch {
     Dev* d_dev2 = nullptr;         // each slot's second hydraulic operator
     Params* d_par = nullptr;
     int *d_on = nullptr, *d_off = nullptr, *d_status = nullptr;
-    int *d_off2 = nullptr, *d_off3 = nullptr;
+    int *d_off2 = nullptr, *d_off3 = nullptr, *d_off4 = nullptr;
     int visc = -1, mixed = -1;     // fixed by the first scenario attached
     int anylim = 0;                // a running scenario's limiter is not MinMod2
     int morpho = 0;                // a running scenario has morphodynamics
@@ -2688,6 +2723,33 @@ int refresh_topography(kst_handle* h) {
     return 0;
 }
 
+// The wide stage kernels' sub-block for tiles of nx x ny cells: of the shapes
+// whose cells, faces, halo and LDS arrays a 256-thread workgroup holds, one
+// that covers the tile in the fewest workgroups -- each costs about the same
+// whatever its share of cells -- and among those the one with the smallest
+// halo.  32 x 32 tiles: 16 x 16.  The 50 x 50 tiles of the reference's decks:
+// 25 x 10, ten workgroups a tile instead of sixteen of 16 x 16, seven of
+// which hold 2 columns or rows.
+void wide_shape(Params& p) {
+    int best = INT_MAX, halo = INT_MAX;
+    for (int w = 4; w <= std::min(p.nx, WIDE_EDGE); ++w)
+        for (int h = 4; h <= std::min(p.ny, WIDE_EDGE); ++h) {
+            if (w * h > STAGE_NT || (w + 1) * h > WIDE_FACES || w * (h + 1) > WIDE_FACES ||
+                (w + 4) * (h + 4) > WIDE_REG || h * (w + 3) > WIDE_BED || w * (h + 3) > WIDE_BED ||
+                4 * (w + h) > WIDE_HALO)
+                continue;
+            const int n = ((p.nx + w - 1) / w) * ((p.ny + h - 1) / h);
+            if (n < best || (n == best && w + h < halo)) { best = n; halo = w + h; p.sw = w; p.sh = h; }
+        }
+    if (p.oned) { p.sw = p.sh = 4; }   // 1D grids have no wide kernels
+    p.sbx = (p.nx + p.sw - 1) / p.sw;
+    p.spt = p.sbx * ((p.ny + p.sh - 1) / p.sh);
+    p.dsw = div_factor(p.sw);
+    p.dsw1 = div_factor(p.sw + 1);
+    p.dsw3 = div_factor(p.sw + 3);
+    p.dsh3 = div_factor(p.sh + 3);
+}
+
 void fill_params(kst_handle* h) {
     const kst_config& c = h->cfg;
     Params& p = h->p;
@@ -2721,6 +2783,7 @@ void fill_params(kst_handle* h) {
     p.bc_hn = c.bc_hn; p.bc_u = c.bc_u; p.bc_v = c.bc_v; p.bc_psi = c.bc_psi;
     p.bc_rho = c.rhow + (c.rhos - c.rhow) * c.bc_psi;   // Density (src/Closures.f90)
     p.oned = c.ny_tiles * c.ny_per_tile == 1;
+    wide_shape(p);
 }
 
 int read_ctrl(kst_handle* h, Ctrl* c) {
@@ -2812,7 +2875,8 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
     const int spt_s = ((p.nx + B - 1) / B) * ((p.ny + BY_SMALL - 1) / BY_SMALL);
     // a grid limit (a multiple of 8) keeps that many blocks, each taking
     // further items in turn
-    const int nblk_stage = sm ? 8 * ((cap * spt_s + 7) / 8) : (grid_limit > 0 ? std::min(nblk, grid_limit) : nblk);
+    const int nblk_w = 8 * ((cap * p.spt + 7) / 8);
+    const int nblk_stage = sm ? 8 * ((cap * spt_s + 7) / 8) : (grid_limit > 0 ? std::min(nblk_w, grid_limit) : nblk_w);
     const Dev* const A = h->d_args;
     const Params* const P = h->d_par;
     LAUNCH(KW_ACTIVATE, activate_kernel, dim3(1), dim3(ACT_NT), A, P);
@@ -2933,8 +2997,7 @@ int autotune_bucket(kst_handle* h, const Ctrl& c0, int cap, kst_handle::Tune* ou
     if (rc) return rc;
     const Params& p = h->p;
     const bool visc = p.nu != 0.0, mixed = h->d.mixed != 0;
-    const int spt = ((p.nx + B - 1) / B) * ((p.ny + B - 1) / B);
-    const int nblk = 8 * ((cap * spt + 7) / 8);
+    const int nblk = 8 * ((cap * p.spt + 7) / 8);
     struct Cand { int small, grid; } cand[4] = {{0, 0}, {0, h->resident}, {0, 2 * h->resident}, {1, 0}};
     const int ncand = mixed ? 3 : 4;
     kst_handle::Tune t{};
@@ -3907,7 +3970,7 @@ static int batch_launch_iteration(kst_batch* b) {
     const BatchSet& k = batch_set(b->visc == 1, b->mixed == 1, b->anylim == 1);
     const bool mo = b->morpho != 0;
     hipLaunchKernelGGL(batch_activate_kernel, dim3(b->nslot), dim3(ACT_NT), 0, b->stream, bt);
-    hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(BATCH_PLAN_THREADS), 0, b->stream, bt, mo ? 3 : 1);
+    hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(BATCH_PLAN_THREADS), 0, b->stream, bt, mo ? 4 : 1);
     for (int q = 0; q < 4; ++q)
         hipLaunchKernelGGL(k.fn[q], dim3(b->grid), dim3(STAGE_NT), 0, b->stream, bt, 0);
     if (mo) {
@@ -3970,16 +4033,18 @@ int kst_batch_create(int max_slots, kst_batch** out) {
         hipMalloc(&b->d_off, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMalloc(&b->d_off2, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMalloc(&b->d_off3, sizeof(int) * (max_slots + 1)) != hipSuccess ||
+        hipMalloc(&b->d_off4, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMalloc(&b->d_status, sizeof(int) * max_slots) != hipSuccess)
         return fail(KST_ERR_HIP);
     if (hipMemset(b->d_on, 0, sizeof(int) * max_slots) != hipSuccess ||
         hipMemset(b->d_off, 0, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMemset(b->d_off2, 0, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMemset(b->d_off3, 0, sizeof(int) * (max_slots + 1)) != hipSuccess ||
+        hipMemset(b->d_off4, 0, sizeof(int) * (max_slots + 1)) != hipSuccess ||
         hipMemset(b->d_status, 0, sizeof(int) * max_slots) != hipSuccess)
         return fail(KST_ERR_HIP);
     b->bt = Batch{b->d_dev, b->d_par, b->d_on, b->d_off, b->d_status, max_slots,
-                  b->d_dev2, b->d_off2, b->d_off3};
+                  b->d_dev2, b->d_off2, b->d_off3, b->d_off4};
     // resident grids: each kernel's occupancy on every CU, a multiple of 8
     int cus = 0, per_cu = 0, per_cu_m = 0, per_cu_t = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess ||
@@ -4125,7 +4190,8 @@ void kst_batch_destroy(kst_batch* b) {
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     if (b->gexec) (void)hipGraphExecDestroy(b->gexec);
     (void)hipFree(b->d_dev); (void)hipFree(b->d_dev2); (void)hipFree(b->d_par); (void)hipFree(b->d_on);
-    (void)hipFree(b->d_off); (void)hipFree(b->d_off2); (void)hipFree(b->d_off3); (void)hipFree(b->d_status);
+    (void)hipFree(b->d_off); (void)hipFree(b->d_off2); (void)hipFree(b->d_off3); (void)hipFree(b->d_off4);
+    (void)hipFree(b->d_status);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     delete b;
 }
