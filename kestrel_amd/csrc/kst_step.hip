@@ -2571,6 +2571,7 @@ __global__ __launch_bounds__(256) void cell_gamma_kernel(Dev d, Params p, Topo T
 
 #include "kst_morpho.hpp"
 #include "kst_output.hpp"
+#include "kst_io.hpp"
 
 // ===========================================================================
 // host side: the C-ABI (include/kestrel_step.h)
@@ -2591,6 +2592,7 @@ struct kst_handle {
     int nx, ny, ntx, nty, ntiles, NX, NY, NC;
     bool have_topo = false, have_state = false;
     std::vector<std::vector<double>> src_times;   // flux-source knot times (host copy)
+    std::vector<double> src_xyr;                  // flux sources' x, y, radius (host copy)
     double t = 0.0;
     // profiling: per-iteration event pairs around the four stage kernels
     bool profiling = false;
@@ -2606,6 +2608,7 @@ struct kst_handle {
     };
     std::map<int, Tune> tuned;           // bucket (active tiles, rounded up to a power of two)
     double* vol_part = nullptr;          // volume partials (VOL_BLOCKS_MAX + 1 groups)
+    double* io = nullptr;                // staging of the boundary's arrays (stage_buffer)
     double* out_buf = nullptr;           // kst_get_output staging, out_cap doubles
     size_t out_cap = 0;
     std::vector<hipEvent_t> ev;          // 8 per iteration of the current batch
@@ -2798,20 +2801,37 @@ int write_ctrl(kst_handle* h, const Ctrl* c) {
     return 0;
 }
 
-// Global row-major (NY, NX) <-> tile-major [tile][ny][nx].
-void to_tiles(const kst_handle* h, const double* g, double* t) {
-    for (int J = 0; J < h->NY; ++J)
-        for (int I = 0; I < h->NX; ++I) {
-            const int ti = I / h->nx, tj = J / h->ny, i = I % h->nx, j = J % h->ny;
-            t[(size_t)(ti + tj * h->ntx) * h->NC + j * h->nx + i] = g[(size_t)J * h->NX + I];
-        }
+// The handle's staging buffer for the boundary's arrays (kst_io.hpp): five
+// cell arrays, one vertex array and the time, allocated at the first call that
+// needs it.
+int stage_buffer(kst_handle* h) {
+    if (h->io) return 0;
+    const size_t cells = (size_t)h->NX * h->NY, verts = (size_t)(h->NX + 1) * (h->NY + 1);
+    void* p = nullptr;
+    HIPCHK(h, hipMalloc(&p, (5 * cells + verts + 1) * sizeof(double)));
+    h->allocs.push_back(p);
+    h->io = static_cast<double*>(p);
+    return 0;
 }
-void from_tiles(const kst_handle* h, const double* t, double* g) {
-    for (int J = 0; J < h->NY; ++J)
-        for (int I = 0; I < h->NX; ++I) {
-            const int ti = I / h->nx, tj = J / h->ny, i = I % h->nx, j = J % h->ny;
-            g[(size_t)J * h->NX + I] = t[(size_t)(ti + tj * h->ntx) * h->NC + j * h->nx + i];
-        }
+
+// Blocks of a kernel that walks n elements (grid-stride).
+int io_blocks(size_t n) { return (int)std::min<size_t>((n + IO_NT - 1) / IO_NT, 65536); }
+
+// One cell array to the device and into tile order, or back (ts: 0 outside
+// allocated tiles); on the handle's stream.
+int put_cells(kst_handle* h, const double* host, double* dev) {
+    const size_t n = (size_t)h->NX * h->NY;
+    HIPCHK(h, hipMemcpyAsync(h->io, host, n * 8, hipMemcpyHostToDevice, h->stream));
+    hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, h->io,
+                       (const uint8_t*)nullptr, dev);
+    return 0;
+}
+int get_cells(kst_handle* h, const double* dev, const uint8_t* ts, double* host) {
+    const size_t n = (size_t)h->NX * h->NY;
+    hipLaunchKernelGGL(gather_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, dev, ts, h->io);
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipMemcpyAsync(host, h->io, n * 8, hipMemcpyDeviceToHost, h->stream));
+    return 0;
 }
 
 typedef void (*StageFn)(const Dev*, const Params*);
@@ -3285,6 +3305,7 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
             off[i] = (int)tt.size();
             for (int k = 0; k < s.n_series; ++k) { tt.push_back(s.time[k]); q.push_back(s.flux[k]); ps.push_back(s.psi[k]); }
             h->src_times.emplace_back(s.time, s.time + s.n_series);
+            h->src_xyr.insert(h->src_xyr.end(), {s.x, s.y, s.radius});
         }
         (void)hipMemcpy(d.src_x, x.data(), 8 * ns, hipMemcpyHostToDevice);
         (void)hipMemcpy(d.src_y, y.data(), 8 * ns, hipMemcpyHostToDevice);
@@ -3321,18 +3342,13 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
 
 int kst_set_topography(kst_handle* h, const double* b0v) {
     if (!h || !b0v) return KST_ERR_CONFIG;
-    const int nx = h->nx, ny = h->ny, NV1 = nx + 1;
-    const size_t NV = (size_t)(nx + 1) * (ny + 1);
-    std::vector<double> tv((size_t)h->ntiles * NV);
-    for (int tj = 0; tj < h->nty; ++tj)
-        for (int ti = 0; ti < h->ntx; ++ti) {
-            double* dst = &tv[(size_t)(ti + tj * h->ntx) * NV];
-            for (int j = 0; j <= ny; ++j)
-                for (int i = 0; i <= nx; ++i)
-                    dst[j * NV1 + i] = b0v[(size_t)(tj * ny + j) * (h->NX + 1) + ti * nx + i];
-        }
-    HIPCHK(h, hipMemcpy(h->d.vb0, tv.data(), tv.size() * 8, hipMemcpyHostToDevice));
-    int rc = refresh_topography(h);
+    int rc = stage_buffer(h);
+    if (rc) return rc;
+    const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
+    HIPCHK(h, hipMemcpyAsync(h->io, b0v, verts * 8, hipMemcpyHostToDevice, h->stream));
+    hipLaunchKernelGGL(scatter_vertices_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->p, h->io,
+                       (const uint8_t*)nullptr, VertexSets{{h->d.vb0}, 1});
+    rc = refresh_topography(h);
     if (rc) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     h->have_topo = true;
@@ -3355,6 +3371,8 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                   const double* hnmax0) {
     if (!h || !w || !rhu || !rhv || !hnpsi || !ts) return KST_ERR_CONFIG;
     if (!h->have_topo) return set_err(h, KST_ERR_STATE, "kst_set_topography must come first");
+    int rc = stage_buffer(h);
+    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
     // tile lists: active sorted by id; ghosts = the non-active neighbours of
     // active tiles that AddGhostTiles takes (src/UpdateTiles.f90:389-481):
@@ -3395,115 +3413,51 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                 if (st[n] == KST_TILE_OFF) { st[n] = KST_TILE_GHOST; gh.push_back(n); }
             }
     }
-    bool flat = true;
+    HIPCHK(h, hipMemcpyAsync(h->d.tstate, st.data(), st.size(), hipMemcpyHostToDevice, h->stream));
     // vertex bt: each active tile takes its own copy of the global values
     // (ghost tiles keep bt = 0, as AllocateTopographicData leaves them),
     // then the topography of every set follows
+    bool flat = true;
     {
-        const int nx = h->nx, ny = h->ny, NV1 = nx + 1;
-        const size_t NV = (size_t)(nx + 1) * (ny + 1);
-        std::vector<double> tv((size_t)h->ntiles * NV, 0.0);
-        if (btv)
-            for (int k : act) {
-                const int ti = k % h->ntx, tj = k / h->ntx;
-                double* dst = &tv[(size_t)k * NV];
-                for (int j = 0; j <= ny; ++j)
-                    for (int i = 0; i <= nx; ++i)
-                        dst[j * NV1 + i] = btv[(size_t)(tj * ny + j) * (h->NX + 1) + ti * nx + i];
-            }
+        const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
         // all +0 to the last bit
-        for (size_t q = 0; btv && flat && q < tv.size(); ++q) flat = tv[q] == 0.0 && !std::signbit(tv[q]);
-        Topo* sets[4] = {&h->d.TA, &h->d.TB, &h->d.TM[0], &h->d.TM[1]};
-        for (int q = 0; q < (h->d.morpho ? 4 : 1); ++q)
-            HIPCHK(h, hipMemcpy(sets[q]->vbt, tv.data(), tv.size() * 8, hipMemcpyHostToDevice));
-        int rc = refresh_topography(h);
+        for (size_t q = 0; btv && flat && q < verts; ++q) flat = btv[q] == 0.0 && !std::signbit(btv[q]);
+        if (btv) HIPCHK(h, hipMemcpyAsync(h->io, btv, verts * 8, hipMemcpyHostToDevice, h->stream));
+        VertexSets sets{{h->d.TA.vbt, h->d.TB.vbt, h->d.TM[0].vbt, h->d.TM[1].vbt}, h->d.morpho ? 4 : 1};
+        hipLaunchKernelGGL(scatter_vertices_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->p,
+                           btv ? h->io : (double*)nullptr, h->d.tstate, sets);
+        rc = refresh_topography(h);
         if (rc) return rc;
-        HIPCHK(h, hipStreamSynchronize(h->stream));
     }
-    // fields: active tiles take the given state, ghosts the data of
-    // UpdateGhostTileBCs (src/UpdateTiles.f90:571-585): on the domain edge
-    // the Dirichlet boundary data, or none with periodic boundaries
-    // (AllocateU's zeros), else SetDefaultTileData's dry data
-    std::vector<double> b0c(FS), btc, cgam;
-    HIPCHK(h, hipMemcpy(b0c.data(), h->d.b0c, FS * 8, hipMemcpyDeviceToHost));
-    if (h->cfg.bc == KST_BC_DIRICHLET) {
-        btc.resize(FS);
-        cgam.resize(FS);
-        HIPCHK(h, hipMemcpy(btc.data(), h->d.T.btc, FS * 8, hipMemcpyDeviceToHost));
-        HIPCHK(h, hipMemcpy(cgam.data(), h->d.T.cgam, FS * 8, hipMemcpyDeviceToHost));
+    // the fields, and all that starts from them
+    {
+        const double* in[5] = {w, rhu, rhv, hnpsi, hnmax0};
+        for (int q = 0; q < 5; ++q)
+            if (in[q]) HIPCHK(h, hipMemcpyAsync(h->io + q * FS, in[q], FS * 8, hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(scatter_state_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->d, h->p, h->io,
+                           hnmax0 ? 1 : 0);
+        HIPCHK(h, hipGetLastError());
     }
-    std::vector<double> S(4 * FS, 0.0);
-    to_tiles(h, w, S.data());
-    to_tiles(h, rhu, S.data() + FS);
-    to_tiles(h, rhv, S.data() + 2 * FS);
-    to_tiles(h, hnpsi, S.data() + 3 * FS);
-    const kst_config& cf = h->cfg;
-    const double bc_rho = cf.rhow + (cf.rhos - cf.rhow) * cf.bc_psi;
-    for (int k = 0; k < h->ntiles; ++k) {
-        if (st[k] == KST_TILE_ACTIVE) continue;
-        const bool on_edge = st[k] == KST_TILE_GHOST && edge(k);
-        for (int c = 0; c < h->NC; ++c) {
-            const size_t gi = (size_t)k * h->NC + c;
-            if (on_edge && cf.bc == KST_BC_PERIODIC) {
-                S[gi] = 0.0;
-                S[FS + gi] = 0.0; S[2 * FS + gi] = 0.0; S[3 * FS + gi] = 0.0;
-            } else if (on_edge && cf.bc == KST_BC_DIRICHLET) {
-                const double hn = cf.bc_hn;
-                double wv = btc[gi] + hn / cgam[gi];
-                wv = wv + b0c[gi];
-                S[gi] = wv;
-                S[FS + gi] = bc_rho * hn * cf.bc_u;
-                S[2 * FS + gi] = bc_rho * hn * cf.bc_v;
-                S[3 * FS + gi] = hn * cf.bc_psi;
-            } else {
-                S[gi] = b0c[gi];
-                S[FS + gi] = 0.0; S[2 * FS + gi] = 0.0; S[3 * FS + gi] = 0.0;
-            }
-        }
-    }
-    HIPCHK(h, hipMemcpy(h->d.S0, S.data(), S.size() * 8, hipMemcpyHostToDevice));
-    if (h->d.mixed) {
-        HIPCHK(h, hipMemcpy(h->d.S0b, S.data(), S.size() * 8, hipMemcpyHostToDevice));
-        HIPCHK(h, hipMemset(h->d.S2, 0, 4 * FS * 4));
-        HIPCHK(h, hipMemset(h->d.S3, 0, 4 * FS * 4));
-        HIPCHK(h, hipMemset(h->d.R, 0, 5 * FS * 4));
-    } else {
-        HIPCHK(h, hipMemcpy(h->d.S2, S.data(), S.size() * 8, hipMemcpyHostToDevice));
-        HIPCHK(h, hipMemcpy(h->d.S3, S.data(), S.size() * 8, hipMemcpyHostToDevice));
-        HIPCHK(h, hipMemset(h->d.R, 0, 5 * FS * 8));
-    }
-    if (h->d.morpho) {
-        HIPCHK(h, hipMemcpy(h->d.SH, S.data(), S.size() * 8, hipMemcpyHostToDevice));
-        for (int q = 0; q < 3; ++q) {
-            HIPCHK(h, hipMemcpy(h->d.SM[q], S.data(), FS * 8, hipMemcpyHostToDevice));
-            HIPCHK(h, hipMemcpy(h->d.SM[q] + FS, S.data() + 3 * FS, FS * 8, hipMemcpyHostToDevice));
-        }
-        HIPCHK(h, hipMemset(h->d.UV, 0, 2 * FS * 8));
-        HIPCHK(h, hipMemset(h->d.R2, 0, 5 * FS * 8));
-    }
-    HIPCHK(h, hipMemset(h->d.gsx, 0, FS * 8));
-    HIPCHK(h, hipMemset(h->d.gsy, 0, FS * 8));
-    // maxima
-    std::vector<double> M(11 * FS, 0.0);
-    for (size_t i = 0; i < FS; ++i) M[10 * FS + i] = -1.0;
-    if (hnmax0) to_tiles(h, hnmax0, M.data());
-    HIPCHK(h, hipMemcpy(h->d.maxima, M.data(), M.size() * 8, hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->d.tstate, st.data(), st.size(), hipMemcpyHostToDevice));
     std::vector<int> actp(act), ghp(gh);
     actp.resize(h->ntiles + 1); ghp.resize(h->ntiles + 1);
-    HIPCHK(h, hipMemcpy(h->d.active, actp.data(), actp.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemcpy(h->d.ghosts, ghp.data(), ghp.size() * 4, hipMemcpyHostToDevice));
-    HIPCHK(h, hipMemset(h->d.eflags, 0, (size_t)h->ntiles * 4));
+    HIPCHK(h, hipMemcpyAsync(h->d.active, actp.data(), actp.size() * 4, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipMemcpyAsync(h->d.ghosts, ghp.data(), ghp.size() * 4, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, hipMemsetAsync(h->d.eflags, 0, (size_t)h->ntiles * 4, h->stream));
     std::vector<uint8_t> hs(h->ntiles, 0);
     // containsSource: tiles holding a cell within a flux source's radius
     // (src/SetSources.f90:357-375)
     for (int q = 0; q < h->cfg.n_sources; ++q) {
-        double sx, sy, sr;
-        (void)hipMemcpy(&sx, h->d.src_x + q, 8, hipMemcpyDeviceToHost);
-        (void)hipMemcpy(&sy, h->d.src_y + q, 8, hipMemcpyDeviceToHost);
-        (void)hipMemcpy(&sr, h->d.src_r + q, 8, hipMemcpyDeviceToHost);
-        for (int J = 0; J < h->NY; ++J)
-            for (int I = 0; I < h->NX; ++I) {
+        const double sx = h->src_xyr[3 * q], sy = h->src_xyr[3 * q + 1], sr = h->src_xyr[3 * q + 2];
+        // the rows and columns that the circle can touch, and one more
+        auto range = [&](double at, double size, double d, int n, int& lo, int& hi) {
+            lo = (int)std::max(0.0, std::min((double)n, std::floor((at - sr + 0.5 * size) / d) - 1.0));
+            hi = (int)std::min((double)n, std::max(0.0, std::ceil((at + sr + 0.5 * size) / d) + 1.0));
+        };
+        int I0, I1, J0 = 0, J1 = h->NY;
+        range(sx, h->cfg.x_size, h->cfg.dx, h->NX, I0, I1);
+        if (!h->p.oned) range(sy, h->cfg.y_size, h->cfg.dy, h->NY, J0, J1);
+        for (int J = J0; J < J1; ++J)
+            for (int I = I0; I < I1; ++I) {
                 const int ti = I / h->nx, tj = J / h->ny, i = I % h->nx, j = J % h->ny;
                 const double x = -0.5 * h->cfg.x_size + h->cfg.dx * ((ti + 1 - 1.0) * h->nx + (i + 1 - 0.5));
                 const double y = -0.5 * h->cfg.y_size + h->cfg.dy * ((tj + 1 - 1.0) * h->ny + (j + 1 - 0.5));
@@ -3512,7 +3466,7 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                 if (r2 <= sr * sr) hs[ti + tj * h->ntx] = 1;
             }
     }
-    HIPCHK(h, hipMemcpy(h->d.has_src, hs.data(), hs.size(), hipMemcpyHostToDevice));
+    HIPCHK(h, hipMemcpyAsync(h->d.has_src, hs.data(), hs.size(), hipMemcpyHostToDevice, h->stream));
     Ctrl c;
     std::memset(&c, 0, sizeof c);
     c.t = t;
@@ -3524,14 +3478,13 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
     c.n_active = (int)act.size();
     c.n_ghost = (int)gh.size();
     c.flat = h->d.morpho ? 0 : (int)flat;
-    int rc = write_ctrl(h, &c);
+    rc = write_ctrl(h, &c);
     if (rc) return rc;
     if (!gh.empty())
         hipLaunchKernelGGL(init_ghosts_kernel, dim3(gh.size()), dim3(256), 0, h->stream, h->d, h->p);
     if (!act.empty())
         hipLaunchKernelGGL(init_flags_kernel, dim3(act.size()), dim3(256), 0, h->stream, h->d, h->p);
     // tileContainer's velocities after the state is set: desingularised from it
-    HIPCHK(h, hipMemsetAsync(h->d.UVo, 0, 2 * (size_t)h->ntiles * h->NC * sizeof(double), h->stream));
     if (!act.empty())
         hipLaunchKernelGGL(uv_init_kernel, dim3(std::min((int)act.size(), VOL_BLOCKS_MAX)), dim3(VOL_NT), 0,
                            h->stream, h->d_args, h->d_par);
@@ -3583,70 +3536,28 @@ int kst_step_n(kst_handle* h, int64_t n, kst_stats* st) {
 int kst_get_state(kst_handle* h, double* w, double* rhu, double* rhv, double* hnpsi, double* hn,
                   double* btv, uint8_t* ts, double* t) {
     if (!h) return KST_ERR_CONFIG;
-    const size_t FS = (size_t)h->ntiles * h->NC;
-    std::vector<double> S(4 * FS);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    const double* Sn = h->d.S0;
-    if (h->d.mixed) {
-        Ctrl c;
-        int rc = read_ctrl(h, &c);
-        if (rc) return rc;
-        if (c.cur) Sn = h->d.S0b;
-    }
-    HIPCHK(h, hipMemcpy(S.data(), Sn, S.size() * 8, hipMemcpyDeviceToHost));
-    std::vector<uint8_t> st(h->ntiles);
-    HIPCHK(h, hipMemcpy(st.data(), h->d.tstate, st.size(), hipMemcpyDeviceToHost));
-    // Fields outside allocated (active or ghost) tiles read as zero.
-    for (int k = 0; k < h->ntiles; ++k)
-        if (st[k] == KST_TILE_OFF)
-            for (int q = 0; q < 4; ++q) std::fill_n(&S[q * FS + (size_t)k * h->NC], h->NC, 0.0);
-    if (w) from_tiles(h, S.data(), w);
-    if (rhu) from_tiles(h, S.data() + FS, rhu);
-    if (rhv) from_tiles(h, S.data() + 2 * FS, rhv);
-    if (hnpsi) from_tiles(h, S.data() + 3 * FS, hnpsi);
-    if (hn) {
-        std::vector<double> b0c(FS), bt(FS), g(FS), H(FS, 0.0);
-        HIPCHK(h, hipMemcpy(b0c.data(), h->d.b0c, FS * 8, hipMemcpyDeviceToHost));
-        HIPCHK(h, hipMemcpy(bt.data(), h->d.TA.btc, FS * 8, hipMemcpyDeviceToHost));
-        HIPCHK(h, hipMemcpy(g.data(), h->d.TA.cgam, FS * 8, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < FS; ++i) {
-            const int k = (int)(i / h->NC);
-            if (st[k] == KST_TILE_OFF) continue;
-            if (st[k] == KST_TILE_GHOST) {
-                // a ghost's Hn is the one it was given: zero, or the
-                // Dirichlet boundary depth on the domain edge
-                const int gi = k % h->ntx, gj = k / h->ntx;
-                const bool edge = gi == 0 || gi == h->ntx - 1 || (h->nty > 1 && (gj == 0 || gj == h->nty - 1));
-                H[i] = (h->cfg.bc == KST_BC_DIRICHLET && edge) ? h->cfg.bc_hn : 0.0;
-                continue;
-            }
-            double x = -bt[i];
-            x = x + (S[i] - b0c[i]);
-            x = x * g[i];
-            H[i] = x < 0.0 ? 0.0 : x;
-        }
-        from_tiles(h, H.data(), hn);
-    }
-    if (btv) {
-        // vertex (I, J) from the copy of the tile holding cell (min(I, NX-1), min(J, NY-1))
-        const int nx = h->nx, ny = h->ny, NV1 = nx + 1;
-        const size_t NV = (size_t)(nx + 1) * (ny + 1);
-        std::vector<double> tv((size_t)h->ntiles * NV);
-        HIPCHK(h, hipMemcpy(tv.data(), h->d.TA.vbt, tv.size() * 8, hipMemcpyDeviceToHost));
-        for (int J = 0; J <= h->NY; ++J)
-            for (int I = 0; I <= h->NX; ++I) {
-                const int ci = std::min(I, h->NX - 1), cj = std::min(J, h->NY - 1);
-                const int k = (cj / ny) * h->ntx + ci / nx;
-                double v = 0.0;
-                if (st[k] != KST_TILE_OFF) v = tv[(size_t)k * NV + (J - (cj / ny) * ny) * NV1 + (I - (ci / nx) * nx)];
-                btv[(size_t)J * (h->NX + 1) + I] = v;
-            }
-    }
-    if (ts) std::memcpy(ts, st.data(), st.size());
-    Ctrl c;
-    int rc = read_ctrl(h, &c);
+    int rc = stage_buffer(h);
     if (rc) return rc;
-    if (t) *t = c.t;
+    const size_t FS = (size_t)h->ntiles * h->NC;
+    const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1), total = 5 * FS + verts + 1;
+    hipLaunchKernelGGL(gather_state_kernel, dim3(io_blocks(verts)), dim3(IO_NT), 0, h->stream, h->d, h->p, h->io);
+    HIPCHK(h, hipGetLastError());
+    double* out[7] = {w, rhu, rhv, hnpsi, hn, btv, t};
+    const size_t at[8] = {0, FS, 2 * FS, 3 * FS, 4 * FS, 5 * FS, 5 * FS + verts, total};
+    // a small state in one copy (each costs about 15 us), a large one array by array
+    std::vector<double> all;
+    if (total * 8 <= (1u << 20)) {
+        all.resize(total);
+        HIPCHK(h, hipMemcpyAsync(all.data(), h->io, total * 8, hipMemcpyDeviceToHost, h->stream));
+    } else {
+        for (int q = 0; q < 7; ++q)
+            if (out[q])
+                HIPCHK(h, hipMemcpyAsync(out[q], h->io + at[q], (at[q + 1] - at[q]) * 8, hipMemcpyDeviceToHost, h->stream));
+    }
+    if (ts) HIPCHK(h, hipMemcpyAsync(ts, h->d.tstate, (size_t)h->ntiles, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipStreamSynchronize(h->stream));
+    for (int q = 0; q < 7 && !all.empty(); ++q)
+        if (out[q]) std::memcpy(out[q], all.data() + at[q], (at[q + 1] - at[q]) * 8);
     return KST_OK;
 }
 
@@ -3745,24 +3656,30 @@ int kst_get_output(kst_handle* h, int32_t max_tiles, double* fields, int32_t* ti
 
 int kst_get_maxima(kst_handle* h, double* const mx[11]) {
     if (!h || !mx) return KST_ERR_CONFIG;
+    int rc = stage_buffer(h);
+    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
-    std::vector<double> M(11 * FS);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(M.data(), h->d.maxima, M.size() * 8, hipMemcpyDeviceToHost));
     for (int q = 0; q < 11; ++q)
-        if (mx[q]) from_tiles(h, M.data() + q * FS, mx[q]);
+        if (mx[q]) {
+            rc = get_cells(h, h->d.maxima + q * FS, nullptr, mx[q]);
+            if (rc) return rc;
+        }
+    HIPCHK(h, hipStreamSynchronize(h->stream));
     return KST_OK;
 }
 
 int kst_set_maxima(kst_handle* h, const double* const mx[11]) {
     if (!h || !mx) return KST_ERR_CONFIG;
+    int rc = stage_buffer(h);
+    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
-    std::vector<double> M(11 * FS);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
-    HIPCHK(h, hipMemcpy(M.data(), h->d.maxima, M.size() * 8, hipMemcpyDeviceToHost));
     for (int q = 0; q < 11; ++q)
-        if (mx[q]) to_tiles(h, mx[q], M.data() + q * FS);
-    HIPCHK(h, hipMemcpy(h->d.maxima, M.data(), M.size() * 8, hipMemcpyHostToDevice));
+        if (mx[q]) {
+            rc = put_cells(h, mx[q], h->d.maxima + q * FS);
+            if (rc) return rc;
+        }
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, hipStreamSynchronize(h->stream));
     return KST_OK;
 }
 
@@ -3778,24 +3695,23 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
                             const uint8_t* cells) {
     if (!h || !btc || !dbdx || !dbdy || !cells) return KST_ERR_CONFIG;
     if (!h->have_state) return set_err(h, KST_ERR_STATE, "kst_set_state must come first");
-    const size_t FS = (size_t)h->ntiles * h->NC, NC = (size_t)h->NX * h->NY;
-    std::vector<double> g(NC), in(FS), cur(FS);
-    std::vector<double> mk(NC), mt(FS);
-    for (size_t q = 0; q < NC; ++q) mk[q] = cells[q] ? 1.0 : 0.0;
-    to_tiles(h, mk.data(), mt.data());
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    int rc = stage_buffer(h);
+    if (rc) return rc;
+    const size_t FS = (size_t)h->ntiles * h->NC;
+    // every set takes the given cells of each field (all hold the same cell
+    // topography after kst_set_state); the mask after the field in the stage
     Topo* sets[4] = {&h->d.TA, &h->d.TB, &h->d.TM[0], &h->d.TM[1]};
     const int nsets = h->d.morpho ? 4 : 1;
     const double* src[3] = {btc, dbdx, dbdy};
+    uint8_t* mask = reinterpret_cast<uint8_t*>(h->io + FS);
+    HIPCHK(h, hipMemcpyAsync(mask, cells, FS, hipMemcpyHostToDevice, h->stream));
     for (int f = 0; f < 3; ++f) {
-        double* dst = f == 0 ? h->d.TA.btc : (f == 1 ? h->d.TA.cbx : h->d.TA.cby);
-        HIPCHK(h, hipMemcpy(cur.data(), dst, FS * 8, hipMemcpyDeviceToHost));
-        to_tiles(h, src[f], in.data());
-        for (size_t q = 0; q < FS; ++q)
-            if (mt[q] != 0.0) cur[q] = in[q];
-        for (int k = 0; k < nsets; ++k) {
+        double* from = f == 0 ? h->d.TA.btc : (f == 1 ? h->d.TA.cbx : h->d.TA.cby);
+        HIPCHK(h, hipMemcpyAsync(h->io, src[f], FS * 8, hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(FS)), dim3(IO_NT), 0, h->stream, h->p, h->io, mask, from);
+        for (int k = 1; k < nsets; ++k) {
             double* to = f == 0 ? sets[k]->btc : (f == 1 ? sets[k]->cbx : sets[k]->cby);
-            HIPCHK(h, hipMemcpy(to, cur.data(), FS * 8, hipMemcpyHostToDevice));
+            HIPCHK(h, hipMemcpyAsync(to, from, FS * 8, hipMemcpyDeviceToDevice, h->stream));
         }
     }
     for (int k = 0; k < nsets; ++k)
@@ -3805,14 +3721,14 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
     // what kst_set_state derived from the cell topography: the activation
     // flags of the active tiles and tileContainer's velocities
     Ctrl c;
-    int rc = read_ctrl(h, &c);
+    rc = read_ctrl(h, &c);
     if (rc) return rc;
     if (c.flat) {   // the cells' bt may now differ from the vertices'
         c.flat = 0;
         rc = write_ctrl(h, &c);
         if (rc) return rc;
     }
-    HIPCHK(h, hipMemset(h->d.eflags, 0, (size_t)h->ntiles * 4));
+    HIPCHK(h, hipMemsetAsync(h->d.eflags, 0, (size_t)h->ntiles * 4, h->stream));
     if (c.n_active > 0)
         hipLaunchKernelGGL(init_flags_kernel, dim3(c.n_active), dim3(256), 0, h->stream, h->d, h->p);
     HIPCHK(h, hipMemsetAsync(h->d.UVo, 0, 2 * FS * sizeof(double), h->stream));
@@ -3826,16 +3742,16 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
 
 int kst_get_cell_topography(kst_handle* h, double* b0c, double* btc, double* dbdx, double* dbdy) {
     if (!h) return KST_ERR_CONFIG;
-    const size_t FS = (size_t)h->ntiles * h->NC;
-    std::vector<double> v(FS);
-    HIPCHK(h, hipStreamSynchronize(h->stream));
+    int rc = stage_buffer(h);
+    if (rc) return rc;
     double* outs[4] = {b0c, btc, dbdx, dbdy};
     const double* srcs[4] = {h->d.b0c, h->d.TA.btc, h->d.TA.cbx, h->d.TA.cby};
-    for (int q = 0; q < 4; ++q) {
-        if (!outs[q]) continue;
-        HIPCHK(h, hipMemcpy(v.data(), srcs[q], FS * 8, hipMemcpyDeviceToHost));
-        from_tiles(h, v.data(), outs[q]);
-    }
+    for (int q = 0; q < 4; ++q)
+        if (outs[q]) {
+            rc = get_cells(h, srcs[q], nullptr, outs[q]);
+            if (rc) return rc;
+        }
+    HIPCHK(h, hipStreamSynchronize(h->stream));
     return KST_OK;
 }
 

@@ -188,8 +188,8 @@ class Stepper:
 
     def state(self) -> dict:
         c = self.cfg
-        out = {k: np.zeros((c.NY, c.NX)) for k in ("w", "rhoHnu", "rhoHnv", "Hnpsi", "Hn")}
-        out["btv"] = np.zeros((c.NY + 1, c.NX + 1))
+        out = {k: np.empty((c.NY, c.NX)) for k in ("w", "rhoHnu", "rhoHnv", "Hnpsi", "Hn")}
+        out["btv"] = np.empty((c.NY + 1, c.NX + 1))
         ts = np.zeros(c.ntiles, dtype=np.uint8)
         t = ctypes.c_double()
         self._check(self.L.kst_get_state(self.h, _ptr(out["w"]), _ptr(out["rhoHnu"]), _ptr(out["rhoHnv"]),
@@ -299,7 +299,7 @@ class Stepper:
 
     def maxima(self) -> list:
         c = self.cfg
-        arrs = [np.zeros((c.NY, c.NX)) for _ in range(11)]
+        arrs = [np.empty((c.NY, c.NX)) for _ in range(11)]
         ptrs = (_dp * 11)(*[_ptr(a) for a in arrs])
         self._check(self.L.kst_get_maxima(self.h, ptrs))
         return arrs

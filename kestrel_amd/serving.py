@@ -30,8 +30,9 @@ from .runtime import SLOT_DONE, SLOT_ERROR, SLOT_RUNNING, Batch, KestrelError, S
 
 # Device bytes per cell of a scenario (every tile of the grid), by precision:
 # the FP64 state, stages and RHS, the cell and face topography, ghost slopes,
-# maxima and tile lists (kst_create's allocations).
-BYTES_PER_CELL = {C.PREC_FP64: 8 * 48, C.PREC_MIXED: 8 * 45}
+# maxima and tile lists (kst_create's allocations), and the staging of the
+# boundary's arrays.
+BYTES_PER_CELL = {C.PREC_FP64: 8 * 54, C.PREC_MIXED: 8 * 51}
 
 
 def device_bytes(cfg) -> int:
