@@ -984,16 +984,23 @@ __device__ void commit_part(const DevT& d, const Params& p, int t, int part) {
     }
 }
 
+// Whether the attempt that ends is accepted, so that its bed becomes current.
+// Runs before the step control, which resets what this reads.
+template <class DevT>
+__device__ __forceinline__ bool commit_due(const DevT& d, const Params& p) {
+    const CtrlSnap cs = snap_ctrl(ctrl_view(d));
+    return d.morpho && (cs.status == ST_NEW || cs.status == ST_RETRY) && !verdict(d, p, &cs).reject;
+}
+
 // The accepted step's bed becomes the current one (CopySolutionData
 // intermed3 -> tileContainer, src/TimeStepper.f90:263), in (tile, part) items
 // over a grid sized for the active set the host last saw.
 __global__ __launch_bounds__(256) void commit_kernel(const Dev* __restrict__ dp, const Params* __restrict__ pp) {
     const auto& d = const_arg(dp);
     const Params& p = *pp;
-    const auto* c = ctrl_view(d);
-    if (!c->commit) return;
+    if (!commit_due(d, p)) return;
     if (threadIdx.x == 0) count_work(d.ctrl, KW_COMMIT);
-    const int n = c->n_active * TILE_PARTS;
+    const int n = ctrl_view(d)->n_active * TILE_PARTS;
     for (int it = blockIdx.x; it < n; it += gridDim.x)
         commit_part(d, p, d.active[it / TILE_PARTS], it % TILE_PARTS);
 }
@@ -1048,7 +1055,7 @@ __global__ __launch_bounds__(256) void batch_tile_part_kernel(Batch bt) {
             const auto& d = const_arg(bt.dev + sl);
             sh_slot = sl;
             sh_go = KIND == 0 ? (face_topo_due(d, generic(const_arg(bt.par + sl))) ? 1 : 0)
-                              : (ctrl_view(d)->commit ? 1 : 0);
+                              : (commit_due(d, generic(const_arg(bt.par + sl))) ? 1 : 0);
         }
         __syncthreads();
         const int sl = __builtin_amdgcn_readfirstlane(sh_slot);

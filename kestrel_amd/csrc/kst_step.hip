@@ -64,7 +64,7 @@ struct Ctrl {
     int status, err, n_active, n_ghost, mode;
     int mref;                  // morphodynamic step refused: 1 checks, 2 redistribution
     int ncand;                 // redistribution candidates of this attempt
-    int commit;                // the step was accepted: the new bed becomes current
+    int edge;                  // some tile has eflags set (stage 4): the activation has work
     long long work[16];        // launches that did work, per kernel (KW_*)
     int cur;                   // mixed precision: u^n is in S0 (0) or S0b (1)
     double next_t;             // NextFluxSeriesTime of t, kept with t
@@ -93,8 +93,8 @@ enum {
 
 // An atomic whose result is unused: the thread does not wait for it (a
 // read-modify-write would hold block 0 for a round trip before its barrier).
-__device__ __forceinline__ void count_work(const Ctrl* c, int id) {
-    if (blockIdx.x == 0) atomicAdd((unsigned long long*)&const_cast<Ctrl*>(c)->work[id], 1ULL);
+__device__ __forceinline__ void count_work(const Ctrl* c, int id, bool any = false) {
+    if (any || blockIdx.x == 0) atomicAdd((unsigned long long*)&const_cast<Ctrl*>(c)->work[id], 1ULL);
 }
 
 // Bed-dependent topography of one generation, per tile.  Each tile holds its
@@ -1524,6 +1524,8 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         if (d.last) { d.UVo[oidx] = ou; d.UVo[FS + oidx] = ov; }
         // activation flags from this state's Hn (CheckIfNearBoundaries,
         // src/TimeStepper.f90:946-1150): bit 0 N, 1 S, 2 E, 3 W
+        // toward active neighbours they would change nothing (tiles only become
+        // active): most steps set none, and their activation ends at once
         if (d.last && ohn > p.hthr) {
             const int i = blk.bx0 + tx, j = blk.by0 + ty, tb = p.tile_buffer;
             unsigned f = 0;
@@ -1531,7 +1533,12 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             if (j + 1 <= tb) f |= 2u;
             if (i + 1 > p.nx - tb) f |= 4u;
             if (i + 1 <= tb) f |= 8u;
-            if (f) atomicOr(&d.eflags[t], f);
+            const unsigned on = blk.nact;   // W, E, S, N
+            f &= ~(((on >> 3) & 1u) | ((on >> 1) & 2u) | ((on << 1) & 4u) | ((on << 3) & 8u));
+            if (f) {
+                atomicOr(&d.eflags[t], f);
+                d.ctrl->edge = 1;
+            }
         }
     }
     return more;
@@ -2096,6 +2103,7 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
     if (c->status != ST_NEW) return;
     if (threadIdx.x == 0) count_work(c, KW_ACTIVATE);
     if (d.morpho) refresh_ghost_overlay(d, p);
+    if (!c->edge) return;               // no flag is set
     const int n0 = c->n_active;
     const int s0 = p.oned ? 2 : 0;      // E and W only on a 1D grid
     // candidates in list order; each thread takes ACT_R consecutive entries
@@ -2149,6 +2157,7 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
             }
         }
     }
+    if (threadIdx.x == 0) c->edge = 0;   // (after the append's barriers: every thread has read it)
     if (ncand == 0) return;   // every flag cleared, nothing to add
     __syncthreads();
     if (ncand > d.act_cand) {
@@ -2308,11 +2317,6 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
     }
 }
 
-__global__ __launch_bounds__(ACT_NT) void activate_kernel(const Dev* __restrict__ d,
-                                                          const Params* __restrict__ p) {
-    activate_body(const_arg(d), *p);
-}
-
 // Rebuild every ghost's edge slopes (end of LoadSourceConditions,
 // src/SetSources.f90:388-392) and the activation flags of every active tile.
 __global__ __launch_bounds__(256) void init_ghosts_kernel(Dev d, Params p) {
@@ -2339,7 +2343,10 @@ __global__ __launch_bounds__(256) void init_flags_kernel(Dev d, Params p) {
             if (i + 1 <= tb) f |= 8u;
         }
     }
-    if (f) atomicOr(&d.eflags[t], f);
+    if (f) {
+        atomicOr(&d.eflags[t], f);
+        d.ctrl->edge = 1;
+    }
 }
 
 // Accept or roll back the step (src/TimeStepper.f90:173-275).  With
@@ -2348,68 +2355,63 @@ __global__ __launch_bounds__(256) void init_flags_kernel(Dev d, Params p) {
 // morphodynamic checks or redistribution (dt <- dt/2), the second
 // operator's substep-1 advice (dt <- 0.9 dt or the advice), or its CFL
 // re-checks (dt <- 0.9 dt_k).
+struct Verdict {
+    bool reject;
+    int evals;        // hydraulic RHS evaluations of the attempt
+    double dt, retry;
+};
 template <class DevT>
-__device__ void finalize_body(const DevT& d, const Params& p) {
-    Ctrl* c = d.ctrl;
-    c->commit = 0;
-    if (c->status == ST_DONE || c->status == ST_ERROR) return;
-    c->work[KW_FINALIZE] += 1;
-    const bool ran_p1 = (c->status == ST_NEW);
-    const double dt = step_dt(d, p, d.ctrl);
-    c->rhs_evals += (ran_p1 ? 1 : 0) + 1;
-    bool reject = false;
-    double retry = 0.0;
-    const double dt1 = advised_from_slot(p, c->slot[1].bits, c->n_active);
-    if (dt1 < dt) {
-        reject = true;
-        retry = 0.9 * dt1;
-    } else {
-        c->rhs_evals += 1;
-        const double dt2 = advised_from_slot(p, c->slot[2].bits, c->n_active);
-        if (dt2 < dt) {
-            reject = true;
-            retry = 0.9 * dt2;
+__device__ __forceinline__ Verdict verdict(const DevT& d, const Params& p, const CtrlSnap* c) {
+    Verdict v{false, (c->status == ST_NEW ? 1 : 0) + 1, step_dt(d, p, c), 0.0};
+    const double dt = v.dt;
+    auto check = [&](unsigned long long bits) {      // a CFL re-check
+        const double adv = advised_from_slot(p, bits, c->n_active);
+        if (adv < dt) {
+            v.reject = true;
+            v.retry = 0.9 * adv;
         } else {
-            c->rhs_evals += 1;
+            v.evals += 1;
         }
-    }
-    if (d.morpho && !reject) {
+    };
+    check(c->slot[1].bits);
+    if (!v.reject) check(c->slot[2].bits);
+    if (d.morpho && !v.reject) {
         if (c->mref) {
-            reject = true;
-            retry = 0.5 * dt;
+            v.reject = true;
+            v.retry = 0.5 * dt;
         } else {
-            c->rhs_evals += 1;
+            v.evals += 1;
             const double adv = 0.9 * advised_from_slot(p, c->slot[3].bits, c->n_active);
             if (adv < dt) {
-                reject = true;
-                retry = ((dt - adv) / dt < 0.1) ? 0.9 * dt : adv;
+                v.reject = true;
+                v.retry = ((dt - adv) / dt < 0.1) ? 0.9 * dt : adv;
             } else {
-                c->rhs_evals += 1;
-                const double e1 = advised_from_slot(p, c->slot[4].bits, c->n_active);
-                if (e1 < dt) {
-                    reject = true;
-                    retry = 0.9 * e1;
-                } else {
-                    c->rhs_evals += 1;
-                    const double e2 = advised_from_slot(p, c->slot[5].bits, c->n_active);
-                    if (e2 < dt) {
-                        reject = true;
-                        retry = 0.9 * e2;
-                    } else {
-                        c->rhs_evals += 1;
-                    }
-                }
+                v.evals += 1;
+                check(c->slot[4].bits);
+                if (!v.reject) check(c->slot[5].bits);
             }
         }
     }
+    return v;
+}
+
+template <class DevT>
+__device__ void finalize_body(const DevT& d, const Params& p) {
+    Ctrl* c = d.ctrl;
+    const CtrlSnap cs = snap_ctrl(ctrl_view(d));
+    if (cs.status == ST_DONE || cs.status == ST_ERROR) return;
+    count_work(c, KW_FINALIZE, true);
+    const Verdict v = verdict(d, p, &cs);
+    const double dt = v.dt;
+    c->rhs_evals += v.evals;
     const unsigned long long huge = dbits(kHuge);
     c->mref = 0;
     c->ncand = 0;
     for (int k = 1; k < 6; ++k) c->slot[k].bits = huge;
-    if (reject) {
+    if (v.reject) {
         c->rejected++;
         c->status = ST_RETRY;
-        c->dt_retry = retry;
+        c->dt_retry = v.retry;
         return;
     }
     c->t = d.morpho ? c->t + 2.0 * dt : c->t + dt;
@@ -2421,7 +2423,6 @@ __device__ void finalize_body(const DevT& d, const Params& p) {
     if (dt > c->max_dt) c->max_dt = dt;
     c->slot[0].bits = huge;
     c->status = ST_NEW;
-    c->commit = d.morpho ? 1 : 0;
     if (d.mixed) c->cur ^= 1;
     if (c->mode == 0) {
         if (c->t >= c->tend) c->status = ST_DONE;
@@ -2430,8 +2431,18 @@ __device__ void finalize_body(const DevT& d, const Params& p) {
     }
 }
 
-__global__ void finalize_kernel(const Dev* __restrict__ d, const Params* __restrict__ p) {
-    finalize_body(const_arg(d), *p);
+// Between the last stage of one attempt and the first of the next: step
+// control (FIN), then the activation (ACT), which an accepted step calls for.
+// One launch does both where an iteration follows another -- each is a few
+// dependent reads of the control block, about 5 us with a launch of its own;
+// together, with nothing flagged, 4 us.
+template <bool FIN, bool ACT>
+__global__ __launch_bounds__(ACT_NT) void control_kernel(const Dev* __restrict__ d, const Params* __restrict__ p) {
+    if (FIN) {
+        if (threadIdx.x == 0) finalize_body(const_arg(d), *p);
+        if (ACT) __syncthreads();
+    }
+    if (ACT) activate_body(const_arg(d), *p);
 }
 
 // ---------------------------------------------------------------------------
@@ -2460,11 +2471,23 @@ struct Batch {
 
 constexpr int BATCH_PLAN_THREADS = 1024;
 
-// Activation of every slot (one block per slot).
-__global__ __launch_bounds__(ACT_NT) void batch_activate_kernel(Batch bt) {
+// Step control and activation of every slot (one block per slot, as
+// control_kernel), and the status table the host polls.
+template <bool FIN, bool ACT>
+__global__ __launch_bounds__(ACT_NT) void batch_control_kernel(Batch bt) {
     const int s = blockIdx.x;
     if (!bt.on[s]) return;
-    activate_body(const_arg(bt.dev + s), generic(const_arg(bt.par + s)));
+    const auto& d = const_arg(bt.dev + s);
+    const Params& p = generic(const_arg(bt.par + s));
+    if (FIN) {
+        if (threadIdx.x == 0) finalize_body(d, p);
+        __syncthreads();
+    }
+    if (ACT) {
+        activate_body(d, p);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) bt.status[s] = d.ctrl->status;
 }
 
 // Work list of the iteration: the running slots' active sub-blocks.
@@ -2537,14 +2560,6 @@ __global__ __launch_bounds__(STAGE_NT, 4) void batch_stage_kernel(Batch bt, int 
                                           w - off[sl]);
         __syncthreads();
     }
-}
-
-// Step control of every slot, and the status table the host polls.
-__global__ void batch_finalize_kernel(Batch bt) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= bt.nslot || !bt.on[s]) return;
-    finalize_body(bt.dev[s], bt.par[s]);
-    bt.status[s] = bt.dev[s].ctrl->status;
 }
 
 // Topography of every tile of a set (after kst_set_topography / kst_set_state).
@@ -2873,7 +2888,10 @@ const StageSet& stage_set(bool visc, int limiter, bool mixed, bool small, bool o
 
 // Launch grids cover `cap` active tiles (the kernels take further items in
 // turn when the active set has outgrown it).
-int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid_limit = 0) {
+// begins / ends: the iteration is the first / last of its sequence; between
+// two, one launch does the step control of the one and the activation of the
+// other.
+int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid_limit, bool begins, bool ends) {
     const Params& p = h->p;
     const Dev& d = h->d;
     // while profiling, the dispatch of each launch carries the event pair of
@@ -2899,7 +2917,7 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
     const int nblk_stage = sm ? 8 * ((cap * spt_s + 7) / 8) : (grid_limit > 0 ? std::min(nblk_w, grid_limit) : nblk_w);
     const Dev* const A = h->d_args;
     const Params* const P = h->d_par;
-    LAUNCH(KW_ACTIVATE, activate_kernel, dim3(1), dim3(ACT_NT), A, P);
+    if (begins) LAUNCH(KW_ACTIVATE, (control_kernel<false, true>), dim3(1), dim3(ACT_NT), A, P);
     const StageSet& k = stage_set(visc, p.limiter, d.mixed != 0, sm, p.oned != 0);
     for (int q = 0; q < 4; ++q)
         LAUNCH(KW_STAGE + q, k.fn[q], dim3(nblk_stage), dim3(STAGE_NT), A, P);
@@ -2927,8 +2945,9 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
         for (int q = 0; q < 4; ++q)
             LAUNCH(KW_STAGE + 4 + q, k.fn[q], dim3(nblk_stage), dim3(STAGE_NT), A + 1, P);
     }
-    LAUNCH(KW_FINALIZE, finalize_kernel, dim3(1), dim3(1), A, P);
     if (d.morpho) LAUNCH(KW_COMMIT, commit_kernel, dim3(cap * TILE_PARTS), dim3(256), A, P);
+    if (ends) LAUNCH(KW_FINALIZE, (control_kernel<true, false>), dim3(1), dim3(64), A, P);
+    else LAUNCH(KW_FINALIZE, (control_kernel<true, true>), dim3(1), dim3(ACT_NT), A, P);
 #undef LAUNCH
     HIPCHK(h, hipGetLastError());
     return 0;
@@ -2962,7 +2981,7 @@ int ensure_graph(kst_handle* h, bool small, int cap, int grid_limit, hipGraphExe
     hipGraph_t g = nullptr;
     HIPCHK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
     for (int q = 0; q < kGraphIters; ++q) {
-        int rc = launch_iteration(h, false, small, cap, grid_limit);
+        int rc = launch_iteration(h, false, small, cap, grid_limit, q == 0, q == kGraphIters - 1);
         if (rc) {
             hipGraph_t dummy = nullptr;
             (void)hipStreamEndCapture(h->stream, &dummy);
@@ -3102,7 +3121,7 @@ int run_until_done(kst_handle* h, kst_stats* st, long long max_iters) {
             grid_limit = it->second.grid;
         }
         if (h->profiling) {
-            rc = launch_iteration(h, true, small, cap, grid_limit);
+            rc = launch_iteration(h, true, small, cap, grid_limit, true, true);
             if (rc) return rc;
         } else {
             hipGraphExec_t gx = nullptr;
@@ -3508,7 +3527,7 @@ static int start_run(kst_handle* h, int mode, double tend, long long nsteps, kst
     c.steps_left = nsteps;
     c.steps = c.rejected = c.rhs_evals = c.cell_updates = 0;
     c.redist_cells = c.redist_ghost = 0;
-    c.mref = 0; c.ncand = 0; c.commit = 0;
+    c.mref = 0; c.ncand = 0;
     c.min_dt = 0.0; c.max_dt = 0.0;
     rc = write_ctrl(h, &c);
     if (rc) return rc;
@@ -3881,11 +3900,11 @@ static const BatchSet& batch_set(bool visc, bool mixed, bool anylim) {
 // with morphodynamic slots their M(2dt) (three stages, redistribution, face
 // topography of the new bed) and second hydraulic operator; step control;
 // the accepted beds' commit (the launch sequence of one scenario).
-static int batch_launch_iteration(kst_batch* b) {
+static int batch_launch_iteration(kst_batch* b, bool begins, bool ends) {
     const Batch& bt = b->bt;
     const BatchSet& k = batch_set(b->visc == 1, b->mixed == 1, b->anylim == 1);
     const bool mo = b->morpho != 0;
-    hipLaunchKernelGGL(batch_activate_kernel, dim3(b->nslot), dim3(ACT_NT), 0, b->stream, bt);
+    if (begins) hipLaunchKernelGGL((batch_control_kernel<false, true>), dim3(b->nslot), dim3(ACT_NT), 0, b->stream, bt);
     hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(BATCH_PLAN_THREADS), 0, b->stream, bt, mo ? 4 : 1);
     for (int q = 0; q < 4; ++q)
         hipLaunchKernelGGL(k.fn[q], dim3(b->grid), dim3(STAGE_NT), 0, b->stream, bt, 0);
@@ -3899,8 +3918,9 @@ static int batch_launch_iteration(kst_batch* b) {
         for (int q = 0; q < 4; ++q)
             hipLaunchKernelGGL(k.fn[q], dim3(b->grid), dim3(STAGE_NT), 0, b->stream, bt, 1);
     }
-    hipLaunchKernelGGL(batch_finalize_kernel, dim3((b->nslot + 63) / 64), dim3(64), 0, b->stream, bt);
     if (mo) hipLaunchKernelGGL((batch_tile_part_kernel<1>), dim3(b->tgrid), dim3(256), 0, b->stream, bt);
+    if (ends) hipLaunchKernelGGL((batch_control_kernel<true, false>), dim3(b->nslot), dim3(64), 0, b->stream, bt);
+    else hipLaunchKernelGGL((batch_control_kernel<true, true>), dim3(b->nslot), dim3(ACT_NT), 0, b->stream, bt);
     BCHK(b, hipGetLastError());
     return 0;
 }
@@ -3910,7 +3930,7 @@ static int batch_ensure_graph(kst_batch* b) {
     hipGraph_t g = nullptr;
     BCHK(b, hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     for (int q = 0; q < kBatchIters; ++q) {
-        int rc = batch_launch_iteration(b);
+        int rc = batch_launch_iteration(b, q == 0, q == kBatchIters - 1);
         if (rc) {
             hipGraph_t dummy = nullptr;
             (void)hipStreamEndCapture(b->stream, &dummy);
@@ -4039,7 +4059,7 @@ int kst_batch_start(kst_batch* b, int slot, double tend, int64_t nsteps) {
     c.steps_left = by_steps ? nsteps : 0;
     c.steps = c.rejected = c.rhs_evals = c.cell_updates = 0;
     c.redist_cells = c.redist_ghost = 0;
-    c.mref = 0; c.ncand = 0; c.commit = 0;
+    c.mref = 0; c.ncand = 0;
     c.min_dt = 0.0; c.max_dt = 0.0;
     if (write_ctrl(h, &c)) return batch_err(b, KST_ERR_HIP, h->err);
     const int st = ST_NEW;
