@@ -126,6 +126,7 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int 
     asm("" : "+v"(tidu) : "s"(pass));
     const int tid = (int)(tidu & (NT - 1));
     if (tid == 0) morpho_work<BY>(d, p, m, false, KW_MORPHO + S - 1, pass, witem);
+    if (BY < B && tid >= 64 && tid < 128) { touch(*(ConstArg<Dev>*)&d); touch(*(ConstArg<Params>*)&p); }
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(m.skip)) return false;   // wave-uniform (a uniform loop)
     const bool more = __builtin_amdgcn_readfirstlane(m.more) != 0;

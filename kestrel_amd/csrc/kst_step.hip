@@ -187,6 +187,26 @@ __device__ __forceinline__ ConstArg<T>& const_arg(const T* p) {
     return *(ConstArg<T>*)p;
 }
 
+// A double that every lane of the wave holds, in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)b);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Reads one word of every cache line of a kernel argument object, so that the
+// scalar cache holds it when its fields are used: a wave that would wait at a
+// barrier does this while another finds the workgroup's item.
+template <class T>
+__device__ __forceinline__ void touch(ConstArg<T>& r) {
+    ConstArg<int>* q = (ConstArg<int>*)&r;
+    int x = 0;
+#pragma unroll
+    for (unsigned k = 0; k < sizeof(T) / 4; k += 16) x |= q[k];
+    asm volatile("" ::"s"(x));
+}
+
 // The same object as an ordinary reference (reads through it still become
 // scalar loads once the compiler sees where it came from).
 template <class T>
@@ -414,7 +434,7 @@ struct SmemT : PairT<RegionT<NQ_, MIX, BY, ONED>, FluxT<NQ_, MIX, BY>, BY == B> 
     static constexpr bool oned = ONED;
     static constexpr int NQ = NQ_;
     static constexpr int NFX = FluxT<NQ_, MIX, BY>::NFX, NFY = FluxT<NQ_, MIX, BY>::NFY;
-    // stage 2: the owned cells' u1 momenta, over the face pass
+    // wide: the owned cells' stage momenta, over the face pass
     double mom[2][alias && !MIX ? B * BY : 1];
     double red[STAGE_NT / 64];
     int tile, bx0, by0, bxa, bya, skip, cur, more, flat;
@@ -1025,13 +1045,14 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         s.more = more;
         s.solids = 0;
     }
+    if (!Smem::alias && tid >= 64 && tid < 128) { touch(*(ConstArg<Dev>*)&d); touch(*(ConstArg<Params>*)&p); }
     __syncthreads();
     // read as wave-uniform values, so that the block's loop over items is a
     // uniform loop (a loop the compiler must treat as divergent costs far more)
     if (__builtin_amdgcn_readfirstlane(s.skip)) return false;
     const bool more = __builtin_amdgcn_readfirstlane(s.more) != 0;
     const int t = __builtin_amdgcn_readfirstlane(s.tile);
-    const double dt = s.dt;
+    const double dt = uniform(s.dt);   // in scalar registers
     const int FS = (int)d.FS;
     const int bxa = __builtin_amdgcn_readfirstlane(s.bxa), bya = __builtin_amdgcn_readfirstlane(s.bya);
     const double* Un = (MIX && s.cur) ? d.S0b : d.S0;   // u^n of the step
@@ -1184,7 +1205,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         }
     }
     if (__ballot(solids) != 0 && (tid & 63) == 0) s.solids = 1;
-    constexpr bool STASH = Smem::alias && !MIX && STAGE == 2;
+    constexpr bool STASH = Smem::alias && !MIX && STAGE >= 2;
     if (STASH && own) { s.mom[0][tid] = oru; s.mom[1][tid] = orv; }
     // DragClosure + ImplicitSourceTerms (src/Equations.f90:627-658) of the
     // owned cell.  Here and not with the rest of its right-hand side: the
@@ -1221,6 +1242,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     double mxv[6] = {0, 0, 0, 0, 0, 0}, mun[4] = {0, 0, 0, 0};
     auto load_cell = [&]() {
         if (!own) return;
+        if (Smem::alias && !MIX) {
+            ob0 = ld(d.b0c, oidx); obt = blk.flat ? 0.0 : ld(d.T.btc, oidx); og = ld(d.T.cgam, oidx);
+            if (STAGE == 2) { pw = ld(d.Uw, oidx); pru = ld(d.Uu, oidx); prv = ld(d.Uv, oidx); ph = ld(d.Uh, oidx); }
+        }
         if (STAGE == 3 && !MIX) { pw0 = ld(d.Uw, oidx); pu0 = ld(d.Uu, oidx); pv0 = ld(d.Uv, oidx); ph0 = ld(d.Uh, oidx); }
         pbx = ld(d.T.cbx, oidx); pby = ld(d.T.cby, oidx);
         pgxu = ld(d.T.pxu, oidx); pgxv = ld(d.T.pxv, oidx); pgyv = ld(d.T.pyv, oidx);
@@ -1315,10 +1340,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             // rather than registers held over the face pass
             const int r = rgi(tx, ty, rw);
             ow = s.r.w[r]; oh = s.r.h[r]; ou = s.r.u[r]; ov = s.r.v[r]; orho = s.r.rho[r];
-            ob0 = ld(d.b0c, oidx); obt = blk.flat ? 0.0 : ld(d.T.btc, oidx); og = ld(d.T.cgam, oidx);
             if (STASH) { oru = s.mom[0][tid]; orv = s.mom[1][tid]; }
-            if (STAGE == 2) { pw = ld(d.Uw, oidx); pru = ld(d.Uu, oidx); prv = ld(d.Uv, oidx); ph = ld(d.Uh, oidx); }
-            else if (STAGE >= 3) { const double* S = (STAGE == 3) ? d.S2 : d.S3; oru = ld(S + FS, oidx); orv = ld(S + 2 * (size_t)FS, oidx); }
         }
         load_cell();
         if (CFL) wave_min(s, cflm);
