@@ -26,6 +26,7 @@ constexpr int MV = B + 1;    // vertices along a sub-block edge
 template <int BY>
 constexpr int morpho_nt() { return BY == B ? 512 : 256; }
 static_assert(morpho_nt<B>() >= NREG && morpho_nt<B>() >= MR1 * MR1, "one round per phase");
+static_assert(morpho_nt<B / 4>() == STAGE_NT, "stage_side");
 static_assert(morpho_nt<B / 4>() >= RW * (B / 4 + 4), "one round per phase");
 
 // Thread 0: whether the morphodynamic operator runs in this attempt (the
@@ -39,14 +40,14 @@ struct MWork {
 // witem >= 0: that item of the scenario's list (a batch's work list), else
 // the block's pass-th item of a one-scenario launch.
 template <int BY, class DevT>
-__device__ void morpho_work(const DevT& d, const Params& p, MWork& m, bool need_no_refine, int kw,
+__device__ void morpho_work(const DevT& d, const Params& p, MWork& m, const Launch& l, bool need_no_refine, int kw,
                             int pass, int witem = -1) {
     const int sbx = (p.nx + B - 1) / B, sby = (p.ny + BY - 1) / BY, spt = sbx * sby;
     // the small shape's item and tile ahead of the control block (cap_item)
     constexpr bool SPEC = BY < B;
     int wspec = 0, tspec = 0;
     if (SPEC && witem < 0) {
-        wspec = cap_item();
+        wspec = cap_item(l);
         tspec = d.active[min(wspec / spt, p.ntiles)];   // the list holds ntiles + 1 entries
     }
     const CtrlSnap cs = snap_ctrl(ctrl_view(d));
@@ -58,11 +59,11 @@ __device__ void morpho_work(const DevT& d, const Params& p, MWork& m, bool need_
         if (!first_operator_ok(c, p, dt)) skip = 1;
         if (need_no_refine && c->mref) skip = 1;
     }
-    if (!skip) count_work(d.ctrl, kw);
+    if (!skip) count_work(d.ctrl, kw, l.b);
     const int nwork = c->n_active * spt;
-    const bool spec = SPEC && witem < 0 && nwork <= (int)gridDim.x;
+    const bool spec = SPEC && witem < 0 && nwork <= l.G;
     bool more = false;
-    const int w = witem >= 0 ? witem : (spec ? (pass == 0 ? wspec : nwork) : xcd_item(nwork, pass, &more));
+    const int w = witem >= 0 ? witem : (spec ? (pass == 0 ? wspec : nwork) : xcd_item(l, nwork, pass, &more));
     if (w >= nwork) skip = 1;
     m.more = more;
     if (!skip) {
@@ -112,7 +113,8 @@ __device__ __forceinline__ double excess_deposition(const DevT& d, const Params&
 // ONED: a 1D grid (one row of cells; its vertex rates and cell topography
 // take the reference's 1D forms, its upper vertex row keeps a zero rate).
 template <int S, int BY, bool ONED, class DevT>
-__device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int pass, int witem = -1) {
+__device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, const Launch& l, int pass,
+                                            int witem = -1) {
     constexpr int NT = morpho_nt<BY>();
     constexpr int NH = RW * (BY + 4), NE = MR1 * (BY + 2), NVB = MV * (BY + 1);
     __shared__ double hn[NH];              // Hn of intermed_{S-1}, 2-cell halo
@@ -125,7 +127,7 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int 
     unsigned tidu = threadIdx.x;
     asm("" : "+v"(tidu) : "s"(pass));
     const int tid = (int)(tidu & (NT - 1));
-    if (tid == 0) morpho_work<BY>(d, p, m, false, KW_MORPHO + S - 1, pass, witem);
+    if (tid == 0) morpho_work<BY>(d, p, m, l, false, KW_MORPHO + S - 1, pass, witem);
     if (BY < B && tid >= 64 && tid < 128) { touch(*(ConstArg<Dev>*)&d); touch(*(ConstArg<Params>*)&p); }
     __syncthreads();
     if (__builtin_amdgcn_readfirstlane(m.skip)) return false;   // wave-uniform (a uniform loop)
@@ -133,8 +135,12 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int 
     const long long FS = d.FS;
     const int t = m.tile, bx0 = m.bx0, by0 = m.by0, bxa = m.bxa, bya = m.bya;
     const double dtm = 2.0 * m.dt;
-    const double* Win = (S == 1) ? d.SH : d.SM[S - 2];
-    const double* Hin = (S == 1) ? d.SH + 3 * FS : d.SM[S - 2] + FS;
+    // intermed0's w and Hnpsi: stage 3's of the first operator, which its last
+    // stage copies to SH -- maybe beside this stage, so the first one reads
+    // stage 3's own
+    const double* W0 = (S == 1) ? d.S3 : d.SH;
+    const double* Win = (S == 1) ? W0 : d.SM[S - 2];
+    const double* Hin = (S == 1) ? W0 + 3 * FS : d.SM[S - 2] + FS;
     const auto& Tin = (S == 1) ? d.TA : d.TM[S - 2];
     const auto& Tout = (S == 3) ? d.TB : d.TM[S - 1];
     double* Wout = d.SM[S - 1];
@@ -303,7 +309,7 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int 
     const double gn = gamma_of(p.geometric, dbdx, dbdy);
     const size_t gi = (size_t)t * p.NC + j * p.nx + i;
     const double b0c = d.b0c[gi];
-    const double w0 = d.SH[gi], h0 = d.SH[3 * FS + gi];
+    const double w0 = W0[gi], h0 = W0[3 * FS + gi];
     const double btc0 = d.TA.btc[gi], go = d.TA.cgam[gi];
     const double ho = compute_hn(w0, b0c, btc0, go);
     const double db = btc - btc0;
@@ -348,11 +354,8 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, int 
 
 // The grid is sized for the active set the host last saw; a block whose
 // share of the list holds more items takes them in turn.
-template <int S, int BY = B, bool ONED = false>
-// (the 16 x 16 shape keeps 4 waves per SIMD, two of its 512-thread blocks
-// per CU: at most 128 VGPRs)
-__global__ __launch_bounds__(morpho_nt<BY>(), BY == B ? 4 : 1) void morpho_kernel(const Dev* __restrict__ dp,
-                                                               const Params* __restrict__ pp) {
+template <int S, int BY, bool ONED>
+__device__ __forceinline__ void morpho_loop(const Dev* dp, const Params* pp, const Launch& l) {
     for (int pass = 0;; ++pass) {
         // fresh argument pointers per pass: loads through them are not
         // hoisted out of the loop and held in registers across passes
@@ -361,9 +364,17 @@ __global__ __launch_bounds__(morpho_nt<BY>(), BY == B ? 4 : 1) void morpho_kerne
         const Dev* d = dp;
         ConstArg<Params>* p = (ConstArg<Params>*)pp;
         asm("" : "+s"(d), "+s"(p) : "s"(pass));
-        if (!morpho_pass<S, BY, ONED>(const_arg(d), generic(*p), pass)) break;
+        if (!morpho_pass<S, BY, ONED>(const_arg(d), generic(*p), l, pass)) break;
         __syncthreads();
     }
+}
+
+template <int S, int BY = B, bool ONED = false>
+// (the 16 x 16 shape keeps 4 waves per SIMD, two of its 512-thread blocks
+// per CU: at most 128 VGPRs)
+__global__ __launch_bounds__(morpho_nt<BY>(), BY == B ? 4 : 1) void morpho_kernel(const Dev* __restrict__ dp,
+                                                               const Params* __restrict__ pp) {
+    morpho_loop<S, BY, ONED>(dp, pp, Launch{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // A write into a ghost tile's part of intermed3, listed for the next step's
@@ -831,7 +842,7 @@ __device__ __forceinline__ void redistribute_body(const DevT& d, const Params& p
             if (!first_operator_ok(&cs, p, dt) || cs.mref) skip = 1;
         }
         if (!skip && cs.ncand <= 0) skip = 1;
-        if (!skip) count_work(c, KW_REDIST);
+        if (!skip) count_work(c, KW_REDIST, 0);
         sh_skip = skip;
         sh_n = cs.ncand;
         sh_ndirty = ndirty;
@@ -932,7 +943,7 @@ __global__ __launch_bounds__(256) void face_topo_kernel(const Dev* __restrict__ 
     const auto* c = ctrl_view(d);
     if (threadIdx.x == 0) {
         const int skip = face_topo_due(d, p) ? 0 : 1;
-        if (!skip) count_work(d.ctrl, KW_FACETOPO);
+        if (!skip) count_work(d.ctrl, KW_FACETOPO, blockIdx.x);
         sh_skip = skip;
         sh_n = c->n_active * TILE_PARTS;
     }
@@ -996,14 +1007,23 @@ __device__ __forceinline__ bool commit_due(const DevT& d, const Params& p) {
 // The accepted step's bed becomes the current one (CopySolutionData
 // intermed3 -> tileContainer, src/TimeStepper.f90:263), in (tile, part) items
 // over a grid sized for the active set the host last saw.
-__global__ __launch_bounds__(256) void commit_kernel(const Dev* __restrict__ dp, const Params* __restrict__ pp) {
+__device__ __forceinline__ void commit_loop(const Dev* dp, const Params* pp, const Launch& l) {
     const auto& d = const_arg(dp);
     const Params& p = *pp;
     if (!commit_due(d, p)) return;
-    if (threadIdx.x == 0) count_work(d.ctrl, KW_COMMIT);
+    if (threadIdx.x == 0) count_work(d.ctrl, KW_COMMIT, l.b);
     const int n = ctrl_view(d)->n_active * TILE_PARTS;
-    for (int it = blockIdx.x; it < n; it += gridDim.x)
-        commit_part(d, p, d.active[it / TILE_PARTS], it % TILE_PARTS);
+    for (int it = l.b; it < n; it += l.G) commit_part(d, p, d.active[it / TILE_PARTS], it % TILE_PARTS);
+}
+__global__ __launch_bounds__(256) void commit_kernel(const Dev* __restrict__ dp, const Params* __restrict__ pp) {
+    commit_loop(dp, pp, Launch{(int)blockIdx.x, (int)gridDim.x});
+}
+
+// What the last hydraulic stage's launch takes beside it (stage_kernel).
+template <bool ONED>
+__device__ __forceinline__ void stage_side(const Dev* dp, const Params* pp, const Launch& l) {
+    if (const_arg(dp).second) commit_loop(dp, pp, l);
+    else morpho_loop<1, B / 4, ONED>(dp, pp, l);
 }
 
 // ---------------------------------------------------------------------------
@@ -1034,7 +1054,8 @@ __global__ __launch_bounds__(morpho_nt<B>()) void batch_morpho_kernel(Batch bt) 
         if (threadIdx.x == 0) sh_slot = batch_slot(bt.off2, bt.nslot, w);
         __syncthreads();
         const int sl = __builtin_amdgcn_readfirstlane(sh_slot);
-        morpho_pass<S, B, false>(const_arg(bt.dev + sl), generic(const_arg(bt.par + sl)), 0, w - bt.off2[sl]);
+        morpho_pass<S, B, false>(const_arg(bt.dev + sl), generic(const_arg(bt.par + sl)),
+                                 Launch{(int)blockIdx.x, (int)gridDim.x}, 0, w - bt.off2[sl]);
         __syncthreads();
     }
 }

@@ -93,8 +93,8 @@ enum {
 
 // An atomic whose result is unused: the thread does not wait for it (a
 // read-modify-write would hold block 0 for a round trip before its barrier).
-__device__ __forceinline__ void count_work(const Ctrl* c, int id, bool any = false) {
-    if (any || blockIdx.x == 0) atomicAdd((unsigned long long*)&const_cast<Ctrl*>(c)->work[id], 1ULL);
+__device__ __forceinline__ void count_work(const Ctrl* c, int id, int block) {
+    if (block == 0) atomicAdd((unsigned long long*)&const_cast<Ctrl*>(c)->work[id], 1ULL);
 }
 
 // Bed-dependent topography of one generation, per tile.  Each tile holds its
@@ -941,8 +941,12 @@ __device__ __forceinline__ double fluxv(const Smem& s, int q, int i) {
 // eighth of the list and neighbouring sub-blocks share an L2; within it block
 // b takes items b/8, b/8 + G/8, ...  Returns nwork when there is none; *more
 // tells whether the block has a further item.
-__device__ __forceinline__ int xcd_item(int nwork, int pass, bool* more) {
-    const int G = gridDim.x, b = blockIdx.x, x = b % 8, m = G / 8;
+struct Launch {
+    int b, G;      // this workgroup and how many share the items (a launch may hold two kinds of work)
+};
+
+__device__ __forceinline__ int xcd_item(const Launch& l, int nwork, int pass, bool* more) {
+    const int G = l.G, b = l.b, x = b % 8, m = G / 8;
     const int per = (nwork + 7) / 8;
     const int end = min((x + 1) * per, nwork);
     const int w = x * per + b / 8 + pass * m;
@@ -956,10 +960,7 @@ __device__ __forceinline__ int xcd_item(int nwork, int pass, bool* more) {
 // the active set to double), and a block uses it only then, so that the load
 // of its item's tile can be issued alongside the control-block reads.  (Large
 // sets keep xcd_item: this map would leave XCDs idle when nwork < G.)
-__device__ __forceinline__ int cap_item() {
-    const int G = gridDim.x;
-    return (blockIdx.x % 8) * (G / 8) + blockIdx.x / 8;
-}
+__device__ __forceinline__ int cap_item(const Launch& l) { return (l.b % 8) * (l.G / 8) + l.b / 8; }
 
 // Item of thread tid when na items of one kind and nb of another (each at
 // most 128) share a workgroup of four waves: the first kind on wave 0 and,
@@ -980,8 +981,8 @@ __device__ __forceinline__ int split_item(int tid, int na, int nb, bool* second)
 // item of the block in a one-scenario launch.  Returns whether the block has
 // a further item (false when it had none).
 template <int STAGE, bool VISC, int LIM, bool MIX, typename Smem, class DevT>
-__device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem& s, int witem,
-                                           int pass = 0) {
+__device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem& s, int witem, int pass = 0,
+                                           const Launch& l = {0, 8}) {
     constexpr int BY = Smem::by;       // sub-block height
     // the thread index as a fresh value per pass: in a block's loop over
     // items nothing derived from it is hoisted and held across items (which
@@ -997,7 +998,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         constexpr bool SPEC = BY < B;
         int wspec = 0, tspec = 0;
         if (SPEC && witem < 0) {
-            wspec = cap_item();
+            wspec = cap_item(l);
             tspec = d.active[min(wspec / spt, p.ntiles)];   // the list holds ntiles + 1 entries
         }
         const CtrlSnap cs = snap_ctrl(ctrl_view(d));
@@ -1025,11 +1026,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         // work item -> (tile, sub-block); contiguous chunks of the active
         // list go to the same XCD (blocks are dealt round-robin to 8 XCDs)
         const int nwork = c->n_active * spt;
-        const bool spec = SPEC && witem < 0 && nwork <= (int)gridDim.x;
+        const bool spec = SPEC && witem < 0 && nwork <= l.G;
         int w = witem;
         bool more = false;
         if (spec) w = pass == 0 ? wspec : nwork;
-        else if (witem < 0) w = xcd_item(nwork, pass, &more);
+        else if (witem < 0) w = xcd_item(l, nwork, pass, &more);
         if (!skip && w == 0)
             atomicAdd((unsigned long long*)&d.ctrl->work[KW_STAGE + STAGE - 1 + (d.second ? 4 : 0)], 1ULL);
         if (w >= nwork) skip = 1;
@@ -1577,11 +1578,31 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 // now (stage 2 spills 15 registers; at 3 waves without the spills it takes
 // 160 us).  Not reading the face and cell bt of a flat bed (8 of 31 words a
 // cell) by itself changed nothing at 3 waves.
-template <int STAGE, bool VISC, int LIM, bool MIX = false, int BY = B, bool ONED = false>
+//
+// SIDE (16 x 4, STAGE 4): nstage workgroups do the stage.  The last stage of a
+// Strang step's operators does not fill the chip then and nothing waits for it
+// but the step's end, so further workgroups of the same launch take what
+// would follow it (stage_side): after the first operator the first
+// morphodynamic stage, which reads w and Hnpsi as stage 3 left them (the last
+// stage does not change them); after the second the commit of the bed, which
+// is decided by the CFL re-check of stage 3.  A launch less for each (10 and
+// 7 us of an accepted attempt's 166 us on the 1024^2 hills).
+template <bool ONED>
+__device__ __forceinline__ void stage_side(const Dev* d, const Params* p, const Launch& l);
+
+// (A kernel of its own: the side work's registers cost the other launches 2%.)
+template <int STAGE, bool VISC, int LIM, bool MIX = false, int BY = B, bool ONED = false, bool SIDE = false>
 __global__ __launch_bounds__(STAGE_NT, BY == B ? 4 : 1) void stage_kernel(const Dev* __restrict__ d,
-                                                         const Params* __restrict__ p) {
+                                                                          const Params* __restrict__ p, int nstage) {
+    if constexpr (SIDE) {
+        if ((int)blockIdx.x >= nstage) {
+            stage_side<ONED>(d, p, Launch{(int)blockIdx.x - nstage, (int)gridDim.x - nstage});
+            return;
+        }
+    }
     __shared__ SmemT<VISC ? 7 : 5, MIX, BY, ONED> s;
-    for (int pass = 0; stage_body<STAGE, VISC, LIM, MIX>(const_arg(d), *p, s, -1, pass); ++pass)
+    const Launch l{(int)blockIdx.x, SIDE ? nstage : (int)gridDim.x};
+    for (int pass = 0; stage_body<STAGE, VISC, LIM, MIX>(const_arg(d), *p, s, -1, pass, l); ++pass)
         __syncthreads();
 }
 
@@ -2123,7 +2144,7 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
     __shared__ int nnew, bad, first_move, ng_start;
     Ctrl* c = d.ctrl;
     if (c->status != ST_NEW) return;
-    if (threadIdx.x == 0) count_work(c, KW_ACTIVATE);
+    if (threadIdx.x == 0) count_work(c, KW_ACTIVATE, 0);
     if (d.morpho) refresh_ghost_overlay(d, p);
     if (!c->edge) return;               // no flag is set
     const int n0 = c->n_active;
@@ -2422,7 +2443,7 @@ __device__ void finalize_body(const DevT& d, const Params& p) {
     Ctrl* c = d.ctrl;
     const CtrlSnap cs = snap_ctrl(ctrl_view(d));
     if (cs.status == ST_DONE || cs.status == ST_ERROR) return;
-    count_work(c, KW_FINALIZE, true);
+    count_work(c, KW_FINALIZE, 0);
     const Verdict v = verdict(d, p, &cs);
     const double dt = v.dt;
     c->rhs_evals += v.evals;
@@ -2871,13 +2892,15 @@ int get_cells(kst_handle* h, const double* dev, const uint8_t* ts, double* host)
     return 0;
 }
 
-typedef void (*StageFn)(const Dev*, const Params*);
-struct StageSet { StageFn fn[4]; };
+typedef void (*StageFn)(const Dev*, const Params*, int);
+struct StageSet { StageFn fn[4], side; };   // side: the last stage with its side work (16 x 4)
 
 template <bool VISC, int LIM, bool MIX, int BY, bool ONED>
 StageSet make_set() {
+    StageFn side = nullptr;
+    if constexpr (BY < B && !MIX) side = stage_kernel<4, VISC, LIM, MIX, BY, ONED, true>;
     return StageSet{{stage_kernel<1, VISC, LIM, MIX, BY, ONED>, stage_kernel<2, VISC, LIM, MIX, BY, ONED>,
-                     stage_kernel<3, VISC, LIM, MIX, BY, ONED>, stage_kernel<4, VISC, LIM, MIX, BY, ONED>}};
+                     stage_kernel<3, VISC, LIM, MIX, BY, ONED>, stage_kernel<4, VISC, LIM, MIX, BY, ONED>}, side};
 }
 
 template <bool MIX, int BY, bool ONED = false>
@@ -2941,18 +2964,22 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
     const Params* const P = h->d_par;
     if (begins) LAUNCH(KW_ACTIVATE, (control_kernel<false, true>), dim3(1), dim3(ACT_NT), A, P);
     const StageSet& k = stage_set(visc, p.limiter, d.mixed != 0, sm, p.oned != 0);
+    // the last stage's launch also takes the work that follows it (stage_side);
+    // with its own launch while profiling, which times each kernel
+    const bool side = d.morpho && sm && !E;
+    const int ncommit = cap * TILE_PARTS;
     for (int q = 0; q < 4; ++q)
-        LAUNCH(KW_STAGE + q, k.fn[q], dim3(nblk_stage), dim3(STAGE_NT), A, P);
+        LAUNCH(KW_STAGE + q, (side && q == 3 ? k.side : k.fn[q]), dim3(nblk_stage * (side && q == 3 ? 2 : 1)), dim3(STAGE_NT), A, P, nblk_stage);
     if (d.morpho) {
         // M(2dt): three SSP stages, redistribution, face topography of the new bed
         if (p.oned) {
             constexpr int NT = morpho_nt<BY_SMALL>();
-            LAUNCH(KW_MORPHO + 0, (morpho_kernel<1, BY_SMALL, true>), dim3(nblk_stage), dim3(NT), A, P);
+            if (!side) LAUNCH(KW_MORPHO + 0, (morpho_kernel<1, BY_SMALL, true>), dim3(nblk_stage), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 1, (morpho_kernel<2, BY_SMALL, true>), dim3(nblk_stage), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 2, (morpho_kernel<3, BY_SMALL, true>), dim3(nblk_stage), dim3(NT), A, P);
         } else if (sm) {
             constexpr int NT = morpho_nt<BY_SMALL>();
-            LAUNCH(KW_MORPHO + 0, (morpho_kernel<1, BY_SMALL>), dim3(nblk_stage), dim3(NT), A, P);
+            if (!side) LAUNCH(KW_MORPHO + 0, (morpho_kernel<1, BY_SMALL>), dim3(nblk_stage), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 1, (morpho_kernel<2, BY_SMALL>), dim3(nblk_stage), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 2, (morpho_kernel<3, BY_SMALL>), dim3(nblk_stage), dim3(NT), A, P);
         } else {
@@ -2965,9 +2992,10 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
         LAUNCH(KW_FACETOPO, face_topo_kernel, dim3(cap * TILE_PARTS), dim3(256), A, P);
         // second hydraulic operator
         for (int q = 0; q < 4; ++q)
-            LAUNCH(KW_STAGE + 4 + q, k.fn[q], dim3(nblk_stage), dim3(STAGE_NT), A + 1, P);
+            LAUNCH(KW_STAGE + 4 + q, (side && q == 3 ? k.side : k.fn[q]), dim3(nblk_stage + (side && q == 3 ? ncommit : 0)), dim3(STAGE_NT), A + 1, P,
+                   nblk_stage);
     }
-    if (d.morpho) LAUNCH(KW_COMMIT, commit_kernel, dim3(cap * TILE_PARTS), dim3(256), A, P);
+    if (d.morpho && !side) LAUNCH(KW_COMMIT, commit_kernel, dim3(ncommit), dim3(256), A, P);
     if (ends) LAUNCH(KW_FINALIZE, (control_kernel<true, false>), dim3(1), dim3(64), A, P);
     else LAUNCH(KW_FINALIZE, (control_kernel<true, true>), dim3(1), dim3(ACT_NT), A, P);
 #undef LAUNCH
@@ -3073,10 +3101,12 @@ int autotune_bucket(kst_handle* h, const Ctrl& c0, int cap, kst_handle::Tune* ou
         const StageSet& set = stage_set(visc, p.limiter, mixed, k.small != 0, false);
         const int spt_s = ((p.nx + B - 1) / B) * ((p.ny + BY_SMALL - 1) / BY_SMALL);
         const int grid = k.small ? 8 * ((cap * spt_s + 7) / 8) : (k.grid > 0 ? std::min(nblk, k.grid) : nblk);
-        hipLaunchKernelGGL(set.fn[0], dim3(grid), dim3(STAGE_NT), 0, h->stream, h->d_args, h->d_par);
+        hipLaunchKernelGGL(set.fn[0], dim3(grid), dim3(STAGE_NT), 0, h->stream, h->d_args, h->d_par,
+                           grid);
         HIPCHK(h, hipEventRecord(e0, h->stream));
         for (int r = 0; r < kTrials; ++r)
-            hipLaunchKernelGGL(set.fn[0], dim3(grid), dim3(STAGE_NT), 0, h->stream, h->d_args, h->d_par);
+            hipLaunchKernelGGL(set.fn[0], dim3(grid), dim3(STAGE_NT), 0, h->stream, h->d_args, h->d_par,
+                           grid);
         HIPCHK(h, hipEventRecord(e1, h->stream));
         HIPCHK(h, hipEventSynchronize(e1));
         float ms = 0.f;
