@@ -3637,17 +3637,14 @@ namespace {
 // CalculateVolume with the partial sums in `part`, which holds `cap` doubles
 // (VOL_BLOCKS_MAX + 1 groups of VOL_Q pairs suffice for any active set).
 int volume_into(kst_handle* h, double* part, size_t cap, double out[6]) {
-    Ctrl c;
-    int rc = read_ctrl(h, &c);
-    if (rc) return rc;
-    const int nb = std::max(1, std::min(c.n_active, VOL_BLOCKS_MAX));
+    const int nb = volume_partials(h->ntiles);
     if ((size_t)(VOL_BLOCKS_MAX + 1) * VOL_Q * 2 > cap)
         return set_err(h, KST_ERR_CONFIG, "volume: the partial-sum buffer holds " + std::to_string(cap) +
                                               " doubles; " + std::to_string((VOL_BLOCKS_MAX + 1) * VOL_Q * 2) +
                                               " are needed");
     double* fin = part + (size_t)VOL_BLOCKS_MAX * VOL_Q * 2;
     hipLaunchKernelGGL(volume_kernel, dim3(nb), dim3(VOL_NT), 0, h->stream, h->d_args, h->d_par, part);
-    hipLaunchKernelGGL(volume_final_kernel, dim3(1), dim3(VOL_NT), 0, h->stream, part, nb, fin);
+    hipLaunchKernelGGL(volume_final_kernel, dim3(1), dim3(VOL_NT), 0, h->stream, h->d_args, part, fin);
     HIPCHK(h, hipGetLastError());
     double r[VOL_Q * 2];
     HIPCHK(h, hipMemcpyAsync(r, fin, sizeof r, hipMemcpyDeviceToHost, h->stream));
