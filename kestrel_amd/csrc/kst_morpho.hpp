@@ -1033,16 +1033,6 @@ __device__ __forceinline__ void stage_side(const Dev* dp, const Params* pp, cons
 // items), the redistribution takes one workgroup per slot
 // ---------------------------------------------------------------------------
 
-// The slot of work item w of a list whose slot s starts at off[s].
-__device__ __forceinline__ int batch_slot(const int* off, int nslot, int w) {
-    int lo = 0, hi = nslot - 1;   // last slot with off <= w
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) / 2;
-        if (off[mid] <= w) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
 template <int S>
 __global__ __launch_bounds__(morpho_nt<B>()) void batch_morpho_kernel(Batch bt) {
     __shared__ int sh_slot;
@@ -1051,7 +1041,10 @@ __global__ __launch_bounds__(morpho_nt<B>()) void batch_morpho_kernel(Batch bt) 
     const int per = (total + 7) / 8;
     const int end = min((x + 1) * per, total);
     for (int w = x * per + (int)(blockIdx.x / 8); w < end; w += m) {
-        if (threadIdx.x == 0) sh_slot = batch_slot(bt.off2, bt.nslot, w);
+        if (threadIdx.x < 64) {
+            const int sl = batch_slot(bt.off2, bt.nslot, w);
+            if (threadIdx.x == 0) sh_slot = sl;
+        }
         __syncthreads();
         const int sl = __builtin_amdgcn_readfirstlane(sh_slot);
         morpho_pass<S, B, false>(const_arg(bt.dev + sl), generic(const_arg(bt.par + sl)),
@@ -1072,8 +1065,9 @@ __global__ __launch_bounds__(256) void batch_tile_part_kernel(Batch bt) {
     __shared__ int sh_slot, sh_go;
     const int total = bt.off3[bt.nslot];
     for (int w = blockIdx.x; w < total; w += gridDim.x) {
+        const int found = threadIdx.x < 64 ? batch_slot(bt.off3, bt.nslot, w) : 0;
         if (threadIdx.x == 0) {
-            const int sl = batch_slot(bt.off3, bt.nslot, w);
+            const int sl = __builtin_amdgcn_readfirstlane(found);
             const auto& d = const_arg(bt.dev + sl);
             sh_slot = sl;
             sh_go = KIND == 0 ? (face_topo_due(d, generic(const_arg(bt.par + sl))) ? 1 : 0)

@@ -1862,42 +1862,31 @@ __device__ void tile_static_terms(const DevT& d, const Params& p, const TopoT& T
 // tile activation (src/TimeStepper.f90:924-1150, src/UpdateTiles.f90:56-481)
 // ---------------------------------------------------------------------------
 
-// Ghost w slopes at the edges of tile g that face active tiles
-// (ReconstructwAtEdges, src/UpdateTiles.f90:669-750).
+// Ghost w slopes at the edge of tile g on side r (0..3: W, E, S, N) where it
+// faces an active tile (ReconstructwAtEdges, src/UpdateTiles.f90:669-750).
+// One wave's work; the loads leave whatever the neighbour's state (clamped
+// into the grid), with it.
 template <class DevT>
-__device__ void ghost_slopes(const DevT& d, const Params& p, int g) {
+__device__ __forceinline__ void ghost_side_slopes(const DevT& d, const Params& p, int g, int r) {
     const int nx = p.nx, ny = p.ny, NC = p.NC;
     const double* w = (d.mixed && d.ctrl->cur) ? d.S0b : d.S0;
-    const size_t base = (size_t)g * NC;
-    auto on = [&](int k) { return k >= 0 && k < p.ntiles && d.tstate[k] == KST_TILE_ACTIVE; };
-    int nb = nb_tile(p, g, -1, 0);
-    if (on(nb))
-        for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-            const double c = w[base + j * nx], e = w[base + j * nx + 1];
-            const double wv = w[(size_t)nb * NC + j * nx + nx - 1];
-            d.gsx[base + j * nx] = p.dxr * limiter(p.limiter, e - c, c - wv);
-        }
-    nb = nb_tile(p, g, 1, 0);
-    if (on(nb))
-        for (int j = threadIdx.x; j < ny; j += blockDim.x) {
-            const double c = w[base + j * nx + nx - 1], we = w[base + j * nx + nx - 2];
-            const double ev = w[(size_t)nb * NC + j * nx];
-            d.gsx[base + j * nx + nx - 1] = p.dxr * limiter(p.limiter, ev - c, c - we);
-        }
-    nb = nb_tile(p, g, 0, -1);
-    if (on(nb))
-        for (int i = threadIdx.x; i < nx; i += blockDim.x) {
-            const double c = w[base + i], n = w[base + nx + i];
-            const double sv = w[(size_t)nb * NC + (ny - 1) * nx + i];
-            d.gsy[base + i] = p.dyr * limiter(p.limiter, n - c, c - sv);
-        }
-    nb = nb_tile(p, g, 0, 1);
-    if (on(nb))
-        for (int i = threadIdx.x; i < nx; i += blockDim.x) {
-            const double c = w[base + (ny - 1) * nx + i], sv = w[base + (ny - 2) * nx + i];
-            const double nv = w[(size_t)nb * NC + i];
-            d.gsy[base + (ny - 1) * nx + i] = p.dyr * limiter(p.limiter, nv - c, c - sv);
-        }
+    const int nb = nb_tile(p, g, r == 0 ? -1 : (r == 1 ? 1 : 0), r == 2 ? -1 : (r == 3 ? 1 : 0));
+    if (nb < 0 || nb >= p.ntiles) return;
+    const bool on = d.tstate[nb] == KST_TILE_ACTIVE;
+    const bool X = r < 2;
+    const int n = X ? ny : nx;
+    const size_t base = (size_t)g * NC, nbase = (size_t)nb * NC;
+    for (int k = threadIdx.x & 63; k < n; k += 64) {
+        // the edge cell, the one inside it and the neighbour tile's
+        const int own = X ? k * nx + (r == 0 ? 0 : nx - 1) : k + (r == 2 ? 0 : (ny - 1) * nx);
+        const int in = X ? own + (r == 0 ? 1 : -1) : own + (r == 2 ? nx : -nx);
+        const int ex = X ? k * nx + (r == 0 ? nx - 1 : 0) : k + (r == 2 ? (ny - 1) * nx : 0);
+        const double c = w[base + own], i = w[base + in], e = w[nbase + ex];
+        if (!on) continue;
+        const bool low = r == 0 || r == 2;
+        const double up = low ? i - c : e - c, down = low ? c - e : c - i;
+        (X ? d.gsx : d.gsy)[base + own] = (X ? p.dxr : p.dyr) * limiter(p.limiter, up, down);
+    }
 }
 
 // The state of a freshly activated tile (ActivateTile sets w = b0 over
@@ -2315,7 +2304,8 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
     __syncthreads();
     // ActivateTile (src/UpdateTiles.f90:342-384): cell bt = 0, face
     // topography from the tile's and its neighbours' current vertex bt
-    for (int q = 0; q < nnew; ++q) {
+    // (over a flat bed what kst_set_state derived for every tile is the same)
+    for (int q = 0; q < nnew && !c->flat; ++q) {
         tile_cell_topo(d, p, d.T, newt[q], true);
         __syncthreads();
         tile_face_topo(d, p, d.T, newt[q]);
@@ -2355,7 +2345,8 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
         const int slot = block_append(touched ? 1 : 0, cnt, wsum);
         if (touched) tl[slot] = g;
         __syncthreads();
-        for (int j = 0; j < cnt; ++j) ghost_slopes(d, p, tl[j]);
+        // each side of each by a wave of its own
+        for (int j = threadIdx.x >> 6; j < 4 * cnt; j += ACT_NT / 64) ghost_side_slopes(d, p, tl[j >> 2], j & 3);
         __syncthreads();
     }
 }
@@ -2365,7 +2356,7 @@ __device__ __forceinline__ void activate_body(const DevT& d, const Params& p) {
 __global__ __launch_bounds__(256) void init_ghosts_kernel(Dev d, Params p) {
     const int q = blockIdx.x;
     if (q >= d.ctrl->n_ghost) return;
-    ghost_slopes(d, p, d.ghosts[q]);
+    ghost_side_slopes(d, p, d.ghosts[q], threadIdx.x >> 6);   // four waves, four sides
 }
 
 __global__ __launch_bounds__(256) void init_flags_kernel(Dev d, Params p) {
@@ -2539,7 +2530,8 @@ __global__ __launch_bounds__(ACT_NT) void batch_control_kernel(Batch bt) {
 // theirs alone for the morphodynamic kernels (off2, 16 x 16) and the second
 // operator's stages (off4), and off3, their (tile, part) items.
 __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt, int lists) {
-    __shared__ int sc[BATCH_PLAN_THREADS];
+    __shared__ int sc[BATCH_PLAN_THREADS / 64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     for (int kind = 0; kind < lists; ++kind) {
         int* off = kind == 0 ? bt.off : (kind == 1 ? bt.off2 : (kind == 2 ? bt.off3 : bt.off4));
         int carry = 0;
@@ -2557,21 +2549,42 @@ __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt
                 if (kind == 1 && run && d.morpho) n = c->n_active * spt;
                 if (kind == 2 && d.morpho) n = c->n_active * TILE_PARTS;
             }
-            sc[threadIdx.x] = n;
-            __syncthreads();
-            for (int o = 1; o < BATCH_PLAN_THREADS; o <<= 1) {
-                const int v = threadIdx.x >= (unsigned)o ? sc[threadIdx.x - o] : 0;
-                __syncthreads();
-                sc[threadIdx.x] += v;
-                __syncthreads();
+            int x = n;                      // inclusive sum within the wave
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(x, o, 64);
+                if (lane >= o) x += y;
             }
-            if (s < bt.nslot) off[s] = carry + sc[threadIdx.x] - n;
-            carry += sc[BATCH_PLAN_THREADS - 1];
+            if (lane == 63) sc[wv] = x;
+            __syncthreads();
+            int below = 0, sum = 0;
+            for (int k = 0; k < BATCH_PLAN_THREADS / 64; ++k) {
+                if (k < wv) below += sc[k];
+                sum += sc[k];
+            }
+            if (s < bt.nslot) off[s] = carry + below + x - n;
+            carry += sum;
             __syncthreads();
         }
         if (threadIdx.x == 0) off[bt.nslot] = carry;
         __syncthreads();
     }
+}
+
+// The slot of work item w of a list whose slot s starts at off[s]: the last
+// with off[s] <= w (slots without items share their start with the next).
+// One whole wave's work: 64 entries are compared at once, so that up to 64
+// slots take one load instead of a binary search's six dependent ones.
+__device__ __forceinline__ int batch_slot(const int* off, int nslot, int w) {
+    const int lane = threadIdx.x & 63;
+    int lo = 0;
+    for (int n = nslot; n > 1;) {
+        const int step = (n + 63) / 64, k = lane * step;
+        const int v = k < n ? off[lo + k] : INT_MAX;
+        const int hit = __popcll(__ballot(v <= w)) - 1;      // off[lo] <= w
+        lo += hit * step;
+        n = min(step, n - hit * step);
+    }
+    return lo;
 }
 
 // One RK stage over the work list.  The grid is a multiple of 8 blocks that
@@ -2589,13 +2602,9 @@ __global__ __launch_bounds__(STAGE_NT, 4) void batch_stage_kernel(Batch bt, int 
     const int per = (total + 7) / 8;
     const int end = min((x + 1) * per, total);
     for (int w = x * per + (int)(blockIdx.x / 8); w < end; w += m) {
-        if (threadIdx.x == 0) {
-            int lo = 0, hi = bt.nslot - 1;       // last slot with off <= w
-            while (lo < hi) {
-                const int mid = (lo + hi + 1) / 2;
-                if (off[mid] <= w) lo = mid; else hi = mid - 1;
-            }
-            sh_slot = lo;
+        if (threadIdx.x < 64) {
+            const int sl = batch_slot(off, bt.nslot, w);
+            if (threadIdx.x == 0) sh_slot = sl;
         }
         __syncthreads();
         const int sl = __builtin_amdgcn_readfirstlane(sh_slot);
