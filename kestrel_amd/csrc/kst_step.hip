@@ -434,8 +434,9 @@ struct SmemT : PairT<RegionT<NQ_, MIX, BY, ONED>, FluxT<NQ_, MIX, BY>, BY == B> 
     static constexpr bool oned = ONED;
     static constexpr int NQ = NQ_;
     static constexpr int NFX = FluxT<NQ_, MIX, BY>::NFX, NFY = FluxT<NQ_, MIX, BY>::NFY;
-    // wide: the owned cells' stage momenta, over the face pass
-    double mom[2][alias && !MIX ? B * BY : 1];
+    // the owned cells' stage momenta, over the face pass; 16 x 4: and drag factor
+    double mom[2][alias && MIX ? 1 : B * BY];
+    double im[alias ? 1 : B * BY];
     double red[STAGE_NT / 64];
     int tile, bx0, by0, bxa, bya, skip, cur, more, flat;
     int solids;              // some cell of the region has Hnpsi other than 0
@@ -976,6 +977,215 @@ __device__ __forceinline__ int split_item(int tid, int na, int nb, bool* second)
     return f < na ? f : -1;
 }
 
+// UpdateMaximum* of cell k on the pre-step state u at the time tn the step
+// reaches (src/TimeStepper.f90:1155-1303); m: its Hn, speed, erosion, deposit,
+// psi maxima and first inundation.  The second operator of a Strang step
+// would repeat the first one's update with the same state, which changes
+// nothing.
+template <bool ONED, class DevT>
+__device__ __forceinline__ void update_maxima(const DevT& d, const Params& p, unsigned k, const double (&m)[6],
+                                              const double (&u)[4], double b0, double bt, double gam, double bx,
+                                              double by, double tn) {
+    const size_t FS = (size_t)d.FS;
+    double* M = d.maxima + k;
+    if (bt < 0.0 && -bt > m[2]) { M[4 * FS] = -bt; M[5 * FS] = tn; }
+    if (bt > 0.0 && bt > m[3]) { M[6 * FS] = bt; M[7 * FS] = tn; }
+    double hn = compute_hn(u[0], b0, bt, gam);
+    if (hn < 0.0) hn = 0.0;
+    if (hn > p.hthr) {
+        double hp = u[3];
+        if (hp < 0.0) hp = 0.0;
+        const double eps = p.hthr;
+        const double den = hn * hn + dmax(hn * hn, eps * eps);
+        const double psi = dmin(2.0 * hn * hp / den, p.max_pack);
+        const double rho = density(p, psi);
+        const double uu = 2.0 * hn * u[1] / den / rho;
+        const double vv = ONED ? 0.0 : 2.0 * hn * u[2] / den / rho;
+        if (m[5] == -1) M[10 * FS] = tn;
+        if (hn > m[0]) { M[0] = hn; M[FS] = tn; }
+        const double spd = sqrt(speed2(p.geometric, uu, vv, bx, by));
+        if (spd > m[1]) { M[2 * FS] = spd; M[3 * FS] = tn; }
+        if (psi > m[4]) { M[8 * FS] = psi; M[9 * FS] = tn; }
+    }
+}
+
+// Activation flags of a wet cell near its tile's edges (CheckIfNearBoundaries,
+// src/TimeStepper.f90:946-1150): bit 0 N, 1 S, 2 E, 3 W; toward active
+// neighbours they would change nothing (tiles only become active): most steps
+// set none, and their activation ends at once.
+template <class DevT>
+__device__ __forceinline__ void flag_edges(const DevT& d, const Params& p, const Block& blk, int tx, int ty) {
+    const int i = blk.bx0 + tx, j = blk.by0 + ty, tb = p.tile_buffer;
+    unsigned f = 0;
+    if (j + 1 > p.ny - tb) f |= 1u;
+    if (j + 1 <= tb) f |= 2u;
+    if (i + 1 > p.nx - tb) f |= 4u;
+    if (i + 1 <= tb) f |= 8u;
+    const unsigned on = blk.nact;   // W, E, S, N
+    f &= ~(((on >> 3) & 1u) | ((on >> 1) & 2u) | ((on << 1) & 4u) | ((on << 3) & 8u));
+    if (f) {
+        atomicOr(&d.eflags[blk.t], f);
+        d.ctrl->edge = 1;
+    }
+}
+
+// Phase C of the 16 x 4 shape (FP64): wave C of the workgroup advances field C
+// (w, rhoHnu, rhoHnv, Hnpsi) of its 64 cells, so that the update's dependent
+// divisions are on the launch's critical path once, not four fields long, and
+// no wave idles.  Each wave loads what its field needs before the state.  A
+// launch of this shape is one dependent chain (launch 1.7 us, work item 0.7,
+// loads and derived variables 1.0, beds 0.7, faces 1.6, update 1.1): against
+// the four fields in one wave's chain cap release 256^2 38.8 from 39.7 us a
+// step, lake 51.9 from 52.9, hills 1024^2 246 from 254.
+struct FieldTopo {
+    double b0, bt, g;        // the cell's b0, bt, gamma
+    double pn;               // the field of u^n (stages 2, 3)
+    double pa, pb, bs;       // rhoHnu, rhoHnv: hydrostatic prefactors of the x and y faces, bed slope
+    double bx, by, m[6], u[4];   // last stage, wave 3: the maxima update's
+};
+
+template <int STAGE, bool VISC, typename Smem>
+struct FieldUpdate {
+    static constexpr int BY = Smem::by;
+    template <class DevT>
+    static __device__ __forceinline__ bool tracks(const DevT& d, const Params& p) {
+        return STAGE == 4 && p.track_maxima && !d.second;
+    }
+    static __device__ __forceinline__ int field(int tid) { return __builtin_amdgcn_readfirstlane(tid >> 6); }
+
+    template <class DevT>
+    __device__ __forceinline__ FieldTopo load(const DevT& d, const Params& p, const Block& blk, int bxa, int bya,
+                                              int tid) const {
+        FieldTopo f{};
+        const int C = field(tid), tx = tid & (B - 1), ty = (tid & 63) / B;
+        if (tx >= bxa || ty >= bya) return f;
+        const unsigned k = blk.t * p.NC + (blk.by0 + ty) * p.nx + blk.bx0 + tx;
+        f.b0 = ld(d.b0c, k);
+        f.bt = blk.flat ? 0.0 : ld(d.T.btc, k);
+        f.g = ld(d.T.cgam, k);
+        if (STAGE == 2 || STAGE == 3) f.pn = ld(C == 0 ? d.Uw : (C == 1 ? d.Uu : (C == 2 ? d.Uv : d.Uh)), k);
+        if (C == 1 || C == 2) {
+            f.pa = ld(C == 1 ? d.T.pxu : d.T.pxv, k);
+            f.pb = ld(C == 1 ? d.T.pxv : d.T.pyv, k);
+            f.bs = ld(C == 1 ? d.T.cbx : d.T.cby, k);
+        }
+        if (C == 3 && tracks(d, p)) {
+            f.bx = ld(d.T.cbx, k);
+            f.by = ld(d.T.cby, k);
+#pragma unroll
+            for (int q = 0; q < 6; ++q) f.m[q] = ld(d.maxima + 2 * q * (size_t)d.FS, k);   // fields 0, 2, ..., 10
+#pragma unroll
+            for (int q = 0; q < 4; ++q) f.u[q] = ld(d.S0 + q * (size_t)d.FS, k);
+        }
+        return f;
+    }
+
+    template <class DevT>
+    __device__ __forceinline__ void update(const DevT& d, const Params& p, const Smem& s, const Block& blk, int bxa,
+                                           int bya, int tid, double dt, const FieldTopo& f) const {
+        const int C = field(tid), cell = tid & 63, tx = cell & (B - 1), ty = cell / B;
+        if (tx >= bxa || ty >= bya) return;
+        const unsigned k = blk.t * p.NC + (blk.by0 + ty) * p.nx + blk.bx0 + tx;
+        const size_t FS = (size_t)d.FS;
+        const int r = rg(tx, ty), xs = ty * (B + 1) + tx, ys = ty * B + tx;
+        const double gam = f.g, ow = s.r.w[r], third = 1.0 / 3.0, twothird = 2.0 / 3.0;
+        double* Out = STAGE == 1 ? d.R : (STAGE == 2 ? d.S2 : (STAGE == 3 ? d.S3 : d.Sout));
+        if (C == 1 || C == 2) {
+            // ConstructHydraulicRHS (src/HydraulicRHS.f90:1228-1271; on a 1D grid
+            // :1276-1294, x fluxes only and the hydrostatic term divided by gamma)
+            const double* FXc = s.f.fx[C];
+            const double* FX4 = s.f.fx[4];
+            const double* FXv = s.f.fx[VISC ? C + 4 : 4];
+            Kahan kx;
+            kx.add(FXc[xs] - FXc[xs + 1]);
+            if constexpr (Smem::oned) kx.add((FX4[xs] - FX4[xs + 1]) / gam);
+            else kx.add((FX4[xs] - FX4[xs + 1]) * f.pa);
+            kx.add(VISC ? (FXv[xs + 1] - FXv[xs]) : 0.0);
+            double E = kx.s * p.dxr;
+            if constexpr (!Smem::oned) {
+                const double* FYc = s.f.fy[C];
+                const double* FY4 = s.f.fy[4];
+                const double* FYv = s.f.fy[VISC ? C + 4 : 4];
+                Kahan ky;
+                ky.add(FYc[ys] - FYc[ys + B]);
+                ky.add((FY4[ys] - FY4[ys + B]) * f.pb);
+                ky.add(VISC ? (FYv[ys + B] - FYv[ys]) : 0.0);
+                E = E + ky.s * p.dyr;
+            }
+            double hpg = -f.bt;
+            hpg = hpg + (ow - f.b0);
+            hpg = hpg / gam;
+            E = E + (0.0 - p.g * s.r.rho[r] * hpg * f.bs);
+            const double Im = s.im[cell], o = s.mom[C - 1][cell];
+            double v;
+            if (STAGE == 1) v = E;
+            else if (STAGE == 2) v = 0.75 * f.pn + 0.25 * (o + dt * E) / (1.0 - dt * Im);          // src/TimeStepper.f90:407-444
+            else if (STAGE == 3) v = third * f.pn + twothird * (o + dt * E) / (1.0 - dt * Im);     // src/TimeStepper.f90:466-498
+            else v = (o - dt * dt * E * Im) / (1.0 + dt * dt * Im * Im);                           // src/TimeStepper.f90:504-518
+            Out[C * FS + k] = v;
+            if (STAGE == 4 && d.last) d.UVo[(C - 1) * FS + k] = C == 1 ? s.r.u[r] : s.r.v[r];
+            return;
+        }
+        // w and Hnpsi
+        const double o = C == 0 ? ow : s.r.h[r];
+        if (STAGE == 4) {
+            Out[C * FS + k] = o;
+            if (C == 3) {
+                if (tracks(d, p))
+                    update_maxima<Smem::oned>(d, p, k, f.m, f.u, f.b0, f.bt, gam, f.bx, f.by, s.tgrid + dt);
+            } else if (d.last) {
+                double hn = compute_hn(ow, f.b0, f.bt, gam);
+                if (hn > p.hthr) flag_edges(d, p, blk, tx, ty);
+            }
+            return;
+        }
+        const double g = C == 0 ? gam * gam : gam;
+        const double* FXc = s.f.fx[C];
+        double E = (FXc[xs] - FXc[xs + 1]) * p.dxr / g;
+        if constexpr (!Smem::oned) {
+            const double* FYc = s.f.fy[C];
+            E = E + (FYc[ys] - FYc[ys + B]) * p.dyr / g;
+        }
+        // ExplicitSourceTerms (src/Equations.f90:456-620); with no source the
+        // flux terms are 0/(gam*gam) = 0 exactly
+        double src = 0.0;
+        if (p.n_sources > 0 && d.has_src[blk.t]) {
+            double Qt = 0.0, psiQt = 0.0;
+            const int ti = blk.t % p.ntx, tj = blk.t / p.ntx;
+            const int i = blk.bx0 + tx, j = blk.by0 + ty;
+            const double x = -0.5 * p.x_size + p.dx * (((ti + 1) - 1.0) * p.nx + ((i + 1) - 0.5));
+            const double y = -0.5 * p.y_size + p.dy * (((tj + 1) - 1.0) * p.ny + ((j + 1) - 0.5));
+            flux_sources(d, p, s.tstage, s.tgrid, x, y, Qt, psiQt);
+            src = 0.0 + (C == 0 ? Qt : psiQt) / g;
+        }
+        E = E + src;
+        double v = E;
+        if (STAGE != 1 && C == 0) {
+            double hpo = -f.bt;
+            hpo = hpo + (f.pn - f.b0);
+            double hpn = -f.bt;
+            hpn = hpn + (ow - f.b0);
+            v = f.bt;
+            if (STAGE == 2) {
+                v = v + 0.25 * hpn;
+                v = v + 0.75 * hpo;
+                v = v + 0.25 * dt * E;
+            } else {
+                v = v + third * hpo;
+                v = v + twothird * hpn;
+                v = v + twothird * dt * E;
+            }
+            v = v + f.b0;
+        } else if (STAGE == 2) {
+            v = 0.75 * f.pn + 0.25 * (o + dt * E);
+        } else if (STAGE == 3) {
+            v = third * f.pn + twothird * (o + dt * E);
+        }
+        Out[C * FS + k] = v;
+        if (STAGE == 1 && C == 3) Out[4 * FS + k] = s.im[cell];
+    }
+};
+
 // stage_body does one work item (one sub-block of an active tile): witem is
 // its index in the scenario's active-list order, or -1 to take the pass-th
 // item of the block in a one-scenario launch.  Returns whether the block has
@@ -1106,6 +1316,21 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             else bedv = face_bed<true>(d, p, t, blk.by0 + q % (BY + 3) - 1, blk.bx0 + q / (BY + 3));
         }
     }
+    // the small shape's loads of what phases B and C read, ahead of the state's
+    // too: its face's topography and its part of the update
+    FaceTopo pft{};
+    if (pre) {
+        bool yf;
+        const int f = split_item(tid, Smem::NFX, Smem::NFY, &yf);
+        if (f >= 0) {
+            if (!yf) pft = load_face_topo_at<false, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f % (B + 1), f / (B + 1), blk.flat);
+            else pft = load_face_topo_at<true, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f / B, f % B, blk.flat);
+        }
+    }
+    const FieldUpdate<STAGE, VISC, Smem> upd;
+    FieldTopo ftp{};
+    if constexpr (!Smem::alias) ftp = upd.load(d, p, blk, bxa, bya, tid);
+    double pbx = 0, pby = 0, pgxu = 0, pgxv = 0, pgyv = 0, pw0 = 0, pu0 = 0, pv0 = 0, ph0 = 0;
     bool solids = false;
     for (int round = 0; round < (one_round ? 1 : 2); ++round) {
         int rx, ry;
@@ -1223,20 +1448,6 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             Im = -(fric * hr / modu);
         }
     }
-    // the small shape's loads of what phases B and C read: its face's
-    // topography, its cell's bed slopes and prefactors (and u^n in stage 3);
-    // the 16 x 16 shape loads them as the face pass ends, so that they take
-    // no registers during it
-    FaceTopo pft{};
-    double pbx = 0, pby = 0, pgxu = 0, pgxv = 0, pgyv = 0, pw0 = 0, pu0 = 0, pv0 = 0, ph0 = 0;
-    if (pre) {
-        bool yf;
-        const int f = split_item(tid, Smem::NFX, Smem::NFY, &yf);
-        if (f >= 0) {
-            if (!yf) pft = load_face_topo_at<false, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f % (B + 1), f / (B + 1), blk.flat);
-            else pft = load_face_topo_at<true, STAGE != 4>(d, p, t, blk.bx0, blk.by0, f / B, f % B, blk.flat);
-        }
-    }
     // the last stage's maxima update reads u^n and six maxima fields of the
     // owned cell (each written only by its owner): loaded with them
     const bool trk = STAGE == 4 && p.track_maxima && !d.second;
@@ -1257,7 +1468,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             for (int k = 0; k < 4; ++k) mun[k] = ld(Un + k * (size_t)FS, oidx);
         }
     };
-    if (!Smem::alias) load_cell();
+    if (!Smem::alias && own) {
+        s.mom[0][tid] = oru;
+        s.mom[1][tid] = orv;
+        s.im[tid] = Im;
+    }
     // face beds: rows of x-faces -1..bxa+1 and columns of y-faces -1..bya+1
     if (pre) {
         bool yb;
@@ -1381,6 +1596,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     if (CFL) block_min_to(s, &d.ctrl->slot[(d.second ? 3 : 0) + STAGE - 1].bits);
 
     // ---- phase C: RHS of the owned cell and the stage update -------------
+    if constexpr (!Smem::alias) {
+        upd.update(d, p, s, blk, bxa, bya, tid, dt, ftp);
+        return more;
+    }
     if (!own) return more;
     const int xs = ty * (sw + 1) + tx, ys = ty * sw + tx;
 #define FX(q, o) fluxv<MIX, false>(s, q, xs + (o))
@@ -1394,46 +1613,30 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         ohn = compute_hn(ow, ob0, obt, gam);
         if (ohn < 0.0) ohn = 0.0;
     }
-    // ConstructHydraulicRHS (src/HydraulicRHS.f90:1228-1271; on a 1D grid
-    // :1276-1294, x fluxes only and the hydrostatic term divided by gamma)
+    // ConstructHydraulicRHS (src/HydraulicRHS.f90:1228-1271)
     double stw, sth, stu, stv;
-    if constexpr (Smem::oned) {
-        stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam);
-        sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam;
-        Kahan k1;
-        k1.add(FX(1, 0) - FX(1, 1));
-        k1.add((FX(4, 0) - FX(4, 1)) / gam);
-        k1.add(VISC ? (FX(5, 1) - FX(5, 0)) : 0.0);
-        stu = k1.s * p.dxr;
-        Kahan k3;
-        k3.add(FX(2, 0) - FX(2, 1));
-        k3.add((FX(4, 0) - FX(4, 1)) / gam);
-        k3.add(VISC ? (FX(6, 1) - FX(6, 0)) : 0.0);
-        stv = k3.s * p.dxr;
-    } else {
-        stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam) + (FY(0, 0) - FY(0, sw)) * p.dyr / (gam * gam);
-        sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, sw)) * p.dyr / gam;
-        Kahan k1;
-        k1.add(FX(1, 0) - FX(1, 1));
-        k1.add((FX(4, 0) - FX(4, 1)) * gxu);
-        k1.add(VISC ? (FX(5, 1) - FX(5, 0)) : 0.0);
-        stu = k1.s * p.dxr;
-        Kahan k2;
-        k2.add(FY(1, 0) - FY(1, sw));
-        k2.add((FY(4, 0) - FY(4, sw)) * gyu);
-        k2.add(VISC ? (FY(5, sw) - FY(5, 0)) : 0.0);
-        stu = stu + k2.s * p.dyr;
-        Kahan k3;
-        k3.add(FX(2, 0) - FX(2, 1));
-        k3.add((FX(4, 0) - FX(4, 1)) * gxv);
-        k3.add(VISC ? (FX(6, 1) - FX(6, 0)) : 0.0);
-        stv = k3.s * p.dxr;
-        Kahan k4;
-        k4.add(FY(2, 0) - FY(2, sw));
-        k4.add((FY(4, 0) - FY(4, sw)) * gyv);
-        k4.add(VISC ? (FY(6, sw) - FY(6, 0)) : 0.0);
-        stv = stv + k4.s * p.dyr;
-    }
+    stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam) + (FY(0, 0) - FY(0, sw)) * p.dyr / (gam * gam);
+    sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, sw)) * p.dyr / gam;
+    Kahan k1;
+    k1.add(FX(1, 0) - FX(1, 1));
+    k1.add((FX(4, 0) - FX(4, 1)) * gxu);
+    k1.add(VISC ? (FX(5, 1) - FX(5, 0)) : 0.0);
+    stu = k1.s * p.dxr;
+    Kahan k2;
+    k2.add(FY(1, 0) - FY(1, sw));
+    k2.add((FY(4, 0) - FY(4, sw)) * gyu);
+    k2.add(VISC ? (FY(5, sw) - FY(5, 0)) : 0.0);
+    stu = stu + k2.s * p.dyr;
+    Kahan k3;
+    k3.add(FX(2, 0) - FX(2, 1));
+    k3.add((FX(4, 0) - FX(4, 1)) * gxv);
+    k3.add(VISC ? (FX(6, 1) - FX(6, 0)) : 0.0);
+    stv = k3.s * p.dxr;
+    Kahan k4;
+    k4.add(FY(2, 0) - FY(2, sw));
+    k4.add((FY(4, 0) - FY(4, sw)) * gyv);
+    k4.add(VISC ? (FY(6, sw) - FY(6, 0)) : 0.0);
+    stv = stv + k4.s * p.dyr;
 #undef FX
 #undef FY
     // ExplicitSourceTerms (src/Equations.f90:456-620); with no source the
@@ -1515,54 +1718,11 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         // final implicit substep (src/TimeStepper.f90:504-518)
         const double un = (oru - dt * dt * Eu * Im) / (1.0 + dt * dt * Im * Im);
         const double vn = (orv - dt * dt * Ev * Im) / (1.0 + dt * dt * Im * Im);
-        if (trk) {
-            // UpdateMaximum* on the pre-step state at nextT (src/TimeStepper.f90:1155-1303);
-            // the second operator of a Strang step repeats the first one's
-            // update with the same state, which changes nothing
-            const double w0 = mun[0], u0 = mun[1], v0 = mun[2], h0 = mun[3];
-            const double tn = s.tgrid + dt;       // the step's t + dt
-            double* M = d.maxima;
-            if (obt < 0.0 && -obt > mxv[2]) { M[4 * FS + oidx] = -obt; M[5 * FS + oidx] = tn; }
-            if (obt > 0.0 && obt > mxv[3]) { M[6 * FS + oidx] = obt; M[7 * FS + oidx] = tn; }
-            double hn = compute_hn(w0, ob0, obt, gam);
-            if (hn < 0.0) hn = 0.0;
-            if (hn > p.hthr) {
-                double hp0 = h0;
-                if (hp0 < 0.0) hp0 = 0.0;
-                const double eps = p.hthr;
-                const double den = hn * hn + dmax(hn * hn, eps * eps);
-                const double psi = dmin(2.0 * hn * hp0 / den, p.max_pack);
-                const double rho = density(p, psi);
-                const double uu = 2.0 * hn * u0 / (hn * hn + dmax(hn * hn, eps * eps)) / rho;
-                const double vv = Smem::oned ? 0.0 : 2.0 * hn * v0 / (hn * hn + dmax(hn * hn, eps * eps)) / rho;
-                if (mxv[5] == -1) M[10 * FS + oidx] = tn;
-                if (hn > mxv[0]) { M[oidx] = hn; M[FS + oidx] = tn; }
-                const double spd = sqrt(speed2(p.geometric, uu, vv, bx, by));
-                if (spd > mxv[1]) { M[2 * FS + oidx] = spd; M[3 * FS + oidx] = tn; }
-                if (psi > mxv[4]) { M[8 * FS + oidx] = psi; M[9 * FS + oidx] = tn; }
-            }
-        }
+        if (trk) update_maxima<Smem::oned>(d, p, oidx, mxv, mun, ob0, obt, gam, bx, by, s.tgrid + dt);
         double* Out = MIX ? (s.cur ? d.S0 : d.S0b) : d.Sout;
         Out[oidx] = ow; Out[FS + oidx] = un; Out[2 * FS + oidx] = vn; Out[3 * FS + oidx] = oh;
         if (d.last) { d.UVo[oidx] = ou; d.UVo[FS + oidx] = ov; }
-        // activation flags from this state's Hn (CheckIfNearBoundaries,
-        // src/TimeStepper.f90:946-1150): bit 0 N, 1 S, 2 E, 3 W
-        // toward active neighbours they would change nothing (tiles only become
-        // active): most steps set none, and their activation ends at once
-        if (d.last && ohn > p.hthr) {
-            const int i = blk.bx0 + tx, j = blk.by0 + ty, tb = p.tile_buffer;
-            unsigned f = 0;
-            if (j + 1 > p.ny - tb) f |= 1u;
-            if (j + 1 <= tb) f |= 2u;
-            if (i + 1 > p.nx - tb) f |= 4u;
-            if (i + 1 <= tb) f |= 8u;
-            const unsigned on = blk.nact;   // W, E, S, N
-            f &= ~(((on >> 3) & 1u) | ((on >> 1) & 2u) | ((on << 1) & 4u) | ((on << 3) & 8u));
-            if (f) {
-                atomicOr(&d.eflags[t], f);
-                d.ctrl->edge = 1;
-            }
-        }
+        if (d.last && ohn > p.hthr) flag_edges(d, p, blk, tx, ty);
     }
     return more;
 }
