@@ -1616,7 +1616,8 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     // ConstructHydraulicRHS (src/HydraulicRHS.f90:1228-1271)
     double stw, sth, stu, stv;
     stw = (FX(0, 0) - FX(0, 1)) * p.dxr / (gam * gam) + (FY(0, 0) - FY(0, sw)) * p.dyr / (gam * gam);
-    sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, sw)) * p.dyr / gam;
+    sth = 0.0;               // (0 - 0) / gam + (0 - 0) / gam without solids
+    if (blk.solids) sth = (FX(3, 0) - FX(3, 1)) * p.dxr / gam + (FY(3, 0) - FY(3, sw)) * p.dyr / gam;
     Kahan k1;
     k1.add(FX(1, 0) - FX(1, 1));
     k1.add((FX(4, 0) - FX(4, 1)) * gxu);
