@@ -80,15 +80,15 @@ __device__ void morpho_work(const DevT& d, const Params& p, MWork& m, const Laun
 }
 
 // ExcessDeposition (src/Redistribute.f90:158-198) of cell gi, between
-// intermed0 = (SH, TA) and intermed3 = (SM[2], TB); also returns Hn_old,
-// deltaBt and psiold.
+// intermed0 = (stage 3's w and Hnpsi, TA) and intermed3 = (SM[2], TB); also
+// returns Hn_old, deltaBt and psiold.
 template <class DevT>
 __device__ __forceinline__ double excess_deposition(const DevT& d, const Params& p, size_t gi,
                                                     double btc3, double& ho, double& dbt,
                                                     double& psio) {
     const long long FS = d.FS;
     const double go = d.TA.cgam[gi], btc0 = d.TA.btc[gi];
-    const double w0 = d.SH[gi], h0 = d.SH[3 * FS + gi];
+    const double w0 = d.S3[gi], h0 = d.S3[3 * FS + gi];
     ho = compute_hn(w0, d.b0c[gi], btc0, go);
     dbt = btc3 - btc0;
     // intermed0's psi as ComputeDesingularisedVariables left it
@@ -135,10 +135,9 @@ __device__ __forceinline__ bool morpho_pass(const DevT& d, const Params& p, cons
     const long long FS = d.FS;
     const int t = m.tile, bx0 = m.bx0, by0 = m.by0, bxa = m.bxa, bya = m.bya;
     const double dtm = 2.0 * m.dt;
-    // intermed0's w and Hnpsi: stage 3's of the first operator, which its last
-    // stage copies to SH -- maybe beside this stage, so the first one reads
-    // stage 3's own
-    const double* W0 = (S == 1) ? d.S3 : d.SH;
+    // intermed0's w and Hnpsi are stage 3's of the first operator (its last
+    // stage, which comes beside or after M, copies them to SH)
+    const double* W0 = d.S3;
     const double* Win = (S == 1) ? W0 : d.SM[S - 2];
     const double* Hin = (S == 1) ? W0 + 3 * FS : d.SM[S - 2] + FS;
     const auto& Tin = (S == 1) ? d.TA : d.TM[S - 2];

@@ -1194,6 +1194,7 @@ template <int STAGE, bool VISC, int LIM, bool MIX, typename Smem, class DevT>
 __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem& s, int witem, int pass = 0,
                                            const Launch& l = {0, 8}) {
     constexpr int BY = Smem::by;       // sub-block height
+    constexpr bool REFUSED = STAGE == 4 && Smem::alias && !MIX;
     // the thread index as a fresh value per pass: in a block's loop over
     // items nothing derived from it is hoisted and held across items (which
     // would cost registers, and resident waves, for the common single pass).
@@ -1226,6 +1227,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
             const unsigned long long s2 = d.second ? c->slot[5].bits : c->slot[2].bits;
             if (STAGE >= 3 && advised_from_slot(p, s1, c->n_active) < dt) skip = 1;
             if (STAGE >= 4 && advised_from_slot(p, s2, c->n_active) < dt) skip = 1;
+            // the first operator's last stage where it follows the
+            // morphodynamic stages (the wide shape): of an attempt that their
+            // checks refused only the maxima are wanted
+            if (REFUSED && !skip && !d.second && c->mref) skip = p.track_maxima ? 2 : 1;
         }
         s.dt = dt;
         s.cur = c->cur;
@@ -1241,10 +1246,10 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         bool more = false;
         if (spec) w = pass == 0 ? wspec : nwork;
         else if (witem < 0) w = xcd_item(l, nwork, pass, &more);
-        if (!skip && w == 0)
+        if (skip != 1 && w == 0)
             atomicAdd((unsigned long long*)&d.ctrl->work[KW_STAGE + STAGE - 1 + (d.second ? 4 : 0)], 1ULL);
         if (w >= nwork) skip = 1;
-        if (!skip) {
+        if (skip != 1) {
             s.tile = spec ? tspec : d.active[w / spt];
             const int sub = w % spt;
             s.bx0 = (sub % sbx) * sw;
@@ -1260,7 +1265,8 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     __syncthreads();
     // read as wave-uniform values, so that the block's loop over items is a
     // uniform loop (a loop the compiler must treat as divergent costs far more)
-    if (__builtin_amdgcn_readfirstlane(s.skip)) return false;
+    const int skip = __builtin_amdgcn_readfirstlane(s.skip);
+    if (REFUSED ? skip == 1 : skip != 0) return false;
     const bool more = __builtin_amdgcn_readfirstlane(s.more) != 0;
     const int t = __builtin_amdgcn_readfirstlane(s.tile);
     const double dt = uniform(s.dt);   // in scalar registers
@@ -1289,6 +1295,20 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
     const int sw = blk.sw, sh = blk.sh, rw = sw + 4;
     const int ty = Smem::alias ? small_div(tid, p.dsw) : tid / B, tx = tid - ty * sw;
     const bool own = (tx < bxa) && (ty < bya);
+    if (REFUSED && skip == 2) {
+        if (own) {
+            const unsigned k = t * p.NC + (blk.by0 + ty) * p.nx + blk.bx0 + tx;
+            const double b0 = ld(d.b0c, k), bt = blk.flat ? 0.0 : ld(d.T.btc, k), gam = ld(d.T.cgam, k);
+            const double bx = ld(d.T.cbx, k), by = ld(d.T.cby, k);
+            double m[6], u[4];
+#pragma unroll
+            for (int q = 0; q < 6; ++q) m[q] = ld(d.maxima + 2 * q * (size_t)FS, k);   // fields 0, 2, ..., 10
+#pragma unroll
+            for (int q = 0; q < 4; ++q) u[q] = ld(Un + q * (size_t)FS, k);
+            update_maxima<false>(d, p, k, m, u, b0, bt, gam, bx, by, s.tgrid + dt);
+        }
+        return more;
+    }
     double ow = 0, oru = 0, orv = 0, oh = 0, ohn = 0, ou = 0, ov = 0, opsi = 0, orho = 0;
     double ob0 = 0, obt = 0, og = 1;
     double pw = 0, pru = 0, prv = 0, ph = 0;   // u^n of the owned cell (stage 2; mixed: 2..4)
@@ -3138,7 +3158,13 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
     // with its own launch while profiling, which times each kernel
     const bool side = d.morpho && sm && !E;
     const int ncommit = cap * TILE_PARTS;
-    for (int q = 0; q < 4; ++q)
+    // Wide, with morphodynamics: M reads stage 3 only, and its checks refuse
+    // many attempts of a flow that erodes (111 of 151 on the hills with 211
+    // active tiles), so the last stage comes after them and a refused attempt
+    // does without it: 1074 against 1136 us a step there, 2 to 5% from 32 to
+    // 653 active tiles.
+    const bool late = d.morpho && !sm;
+    for (int q = 0; q < (late ? 3 : 4); ++q)
         LAUNCH(KW_STAGE + q, (side && q == 3 ? k.side : k.fn[q]), dim3(nblk_stage * (side && q == 3 ? 2 : 1)), dim3(STAGE_NT), A, P, nblk_stage);
     if (d.morpho) {
         // M(2dt): three SSP stages, redistribution, face topography of the new bed
@@ -3157,6 +3183,7 @@ int launch_iteration(kst_handle* h, bool profiled, bool small, int cap, int grid
             LAUNCH(KW_MORPHO + 0, morpho_kernel<1>, dim3(nblk), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 1, morpho_kernel<2>, dim3(nblk), dim3(NT), A, P);
             LAUNCH(KW_MORPHO + 2, morpho_kernel<3>, dim3(nblk), dim3(NT), A, P);
+            LAUNCH(KW_STAGE + 3, k.fn[3], dim3(nblk_stage), dim3(STAGE_NT), A, P, nblk_stage);
         }
         LAUNCH(KW_REDIST, redistribute_kernel, dim3(1), dim3(RD_THREADS), A, P);
         LAUNCH(KW_FACETOPO, face_topo_kernel, dim3(cap * TILE_PARTS), dim3(256), A, P);
@@ -4125,13 +4152,14 @@ static int batch_launch_iteration(kst_batch* b, bool begins, bool ends) {
     const bool mo = b->morpho != 0;
     if (begins) hipLaunchKernelGGL((batch_control_kernel<false, true>), dim3(b->nslot), dim3(ACT_NT), 0, b->stream, bt);
     hipLaunchKernelGGL(batch_plan_kernel, dim3(1), dim3(BATCH_PLAN_THREADS), 0, b->stream, bt, mo ? 4 : 1);
-    for (int q = 0; q < 4; ++q)
+    for (int q = 0; q < (mo ? 3 : 4); ++q)      // the last one after M's checks (launch_iteration)
         hipLaunchKernelGGL(k.fn[q], dim3(b->grid), dim3(STAGE_NT), 0, b->stream, bt, 0);
     if (mo) {
         constexpr int NT = morpho_nt<B>();
         hipLaunchKernelGGL((batch_morpho_kernel<1>), dim3(b->mgrid), dim3(NT), 0, b->stream, bt);
         hipLaunchKernelGGL((batch_morpho_kernel<2>), dim3(b->mgrid), dim3(NT), 0, b->stream, bt);
         hipLaunchKernelGGL((batch_morpho_kernel<3>), dim3(b->mgrid), dim3(NT), 0, b->stream, bt);
+        hipLaunchKernelGGL(k.fn[3], dim3(b->grid), dim3(STAGE_NT), 0, b->stream, bt, 0);
         hipLaunchKernelGGL(batch_redistribute_kernel, dim3(b->nslot), dim3(RD_THREADS), 0, b->stream, bt);
         hipLaunchKernelGGL((batch_tile_part_kernel<0>), dim3(b->tgrid), dim3(256), 0, b->stream, bt);
         for (int q = 0; q < 4; ++q)
