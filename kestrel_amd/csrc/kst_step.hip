@@ -477,8 +477,8 @@ struct FaceTopo {
 
 // Element idx of an array whose address is uniform over the wave: base in
 // scalar registers, a 32-bit byte offset in a vector register (one
-// instruction instead of a 64-bit address computation per load; every array
-// of a handle that fits the device is shorter than 4 GB, checked in kst_create).
+// instruction instead of a 64-bit address computation per load; every cell and
+// face array is shorter than 4 GB, checked in kst_create).
 __device__ __forceinline__ double ld(const double* base, unsigned idx) {
     return *(const double*)((const char*)base + idx * 8u);
 }
@@ -3469,10 +3469,13 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
     // mixed precision covers the hydraulic operator only
     if (cfg->precision == KST_PREC_MIXED && cfg->morphodynamics) return KST_ERR_CONFIG;
     if (cfg->n_sources > 0 && !cfg->sources) return KST_ERR_CONFIG;
-    // 32-bit byte offsets into every per-tile array (a grid beyond them would
-    // need several times the device's memory)
-    const double per_tile = (double)(cfg->nx_per_tile + 1) * (cfg->ny_per_tile + 1) * 8.0;
-    if (per_tile * cfg->nx_tiles * cfg->ny_tiles >= 4294967296.0) return KST_ERR_CONFIG;
+    // 32-bit byte offsets into every cell and face array (ld): at least 4.3e8
+    // cells, from where on an int no longer holds an index into the five
+    // fields of a state
+    const double cells = (double)cfg->nx_per_tile * cfg->ny_per_tile;
+    double per_tile = cells + cfg->ny_per_tile;
+    if (!oned) per_tile = std::max(per_tile, cells + cfg->nx_per_tile);
+    if (8.0 * per_tile * cfg->nx_tiles * cfg->ny_tiles >= 4294967296.0) return KST_ERR_CONFIG;
     kst_handle* h = new kst_handle();
     h->cfg = *cfg;
     h->cfg.sources = nullptr;
