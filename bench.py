@@ -65,21 +65,21 @@ STEP_WORDS = {"hydraulic": 42, "morpho": 134}
 # profiles/stage_kernel_plain_cap_2048.md, profiles/kernels_morpho_hills_1024.md.
 PMC_FETCH_SCALE, PMC_WRITE_SCALE = 2.0, 1.0
 PMC_TRAFFIC = {
-    ("plain_cap_2048", "stage_kernel<2>"): (212956.2, 51263.5, 1634048.0),
-    ("plain_cap_2048", "stage_kernel<3>"): (202253.5, 51263.5, 1634048.0),
-    ("plain_cap_2048", "stage_kernel<4>"): (214820.1, 113545.8, 1634048.0),
-    ("morpho_hills_1024", "redistribute_kernel"): (92.3, 35.6, 5795.84),
-    ("morpho_hills_1024", "stage_kernel<2>"): (1111.6, 181.9, 5795.84),
-    ("morpho_hills_1024", "morpho_kernel<3>"): (645.8, 317.7, 5795.84),
+    ("plain_cap_2048", "stage_kernel<2>"): (247710.2, 83302.8, 1634048.0),
+    ("plain_cap_2048", "stage_kernel<3>"): (185655.0, 51263.5, 1634048.0),
+    ("plain_cap_2048", "stage_kernel<4>"): (197881.8, 112787.0, 1634048.0),
+    ("morpho_hills_1024", "redistribute_kernel"): (91.7, 35.6, 5795.84),
+    ("morpho_hills_1024", "stage_kernel<2>"): (1513.7, 181.9, 5795.84),
+    ("morpho_hills_1024", "morpho_kernel<3>"): (846.0, 317.9, 5795.84),
 }
 # VALU wave-instructions per productive dispatch (SQ_INSTS_VALU, active cells
 # per launch of that run): profiles/stage_kernel_plain_cap_2048_counters.md.
 # Issue peak: one wave64 VALU instruction per SIMD every 4 cycles, 1024
 # SIMDs at 2.4 GHz.
 PMC_VALU = {
-    ("plain_cap_2048", "stage_kernel<2>"): (3.365e7, 1634048.0),
-    ("plain_cap_2048", "stage_kernel<3>"): (3.286e7, 1634048.0),
-    ("plain_cap_2048", "stage_kernel<4>"): (3.201e7, 1634048.0),
+    ("plain_cap_2048", "stage_kernel<2>"): (2.691e7, 1634048.0),
+    ("plain_cap_2048", "stage_kernel<3>"): (2.598e7, 1634048.0),
+    ("plain_cap_2048", "stage_kernel<4>"): (2.599e7, 1634048.0),
 }
 VALU_PEAK = 1024 * 2.4e9 / 4   # wave-instructions/s
 
