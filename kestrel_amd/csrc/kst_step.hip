@@ -384,7 +384,7 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
 // The fluxes of a 16 x 16 sub-block take the place of what the face pass
 // reads (ALIAS: each thread holds its faces' fluxes over the barrier between
 // the two), which leaves room for four workgroups on a CU instead of three
-// (48 -> 26 KB a workgroup); the 16 x 4 shape keeps them apart, since its
+// (48 -> 28 KB a workgroup); the 16 x 4 shape keeps them apart, since its
 // launches never fill a CU and the extra barrier would lengthen each.
 constexpr int WIDE_REG = 432, WIDE_BED = 352, WIDE_EDGE = 32, WIDE_FACES = 288, WIDE_HALO = 160;
 template <int NQ, bool MIX, int BY, bool ONED>
@@ -1750,14 +1750,14 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 
 // The grid is sized for the active set the host last saw (with room to
 // grow); a block whose share of the list holds more items takes them in turn.
-// The 16 x 16 shape is bound by latency and VALU issue: it is held to 128
+// The wide shape is bound by HBM (3.0-4.0 TB/s, 60-78% of a large copy's
+// rate), VALU issue (45-57% busy) and latency together: it is held to 128
 // VGPRs (4 waves a SIMD) by what phase B does not hold in registers -- the
 // drag closures are evaluated before it, the owned cell is read again after
 // it -- and, where a region carries no solids, by what it does not compute.
-// Plain 2048^2 (1.66 M active cells, clear water), stages 1..4: 154, 164,
-// 160, 166 us at 3 waves a SIMD with every array read, 127, 151, 134, 140 us
-// now (stage 2 spills 15 registers; at 3 waves without the spills it takes
-// 160 us).  Not reading the face and cell bt of a flat bed (8 of 31 words a
+// Plain 2048^2 (1.63 M active cells, clear water), stages 1..4: 157, 161,
+// 159, 164 us at 3 waves a SIMD with every array read, 129, 148, 134, 136 us
+// now (stage 2 spills 9 registers; at 3 waves without spills it took 160 us).  Not reading the face and cell bt of a flat bed (8 of 31 words a
 // cell) by itself changed nothing at 3 waves.
 //
 // SIDE (16 x 4, STAGE 4): nstage workgroups do the stage.  The last stage of a
