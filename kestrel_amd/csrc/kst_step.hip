@@ -2855,7 +2855,8 @@ struct kst_handle {
         double us[4];                    // stage-1 launch time of each candidate (0: not tried)
     };
     std::map<int, Tune> tuned;           // bucket (active tiles, rounded up to a power of two)
-    double* vol_part = nullptr;          // volume partials (VOL_BLOCKS_MAX + 1 groups)
+    double* vol_part = nullptr;          // volume partials (VOL_BLOCKS_MAX groups)
+    double* vol_sum = nullptr;           // their sums, in pinned host memory
     double* io = nullptr;                // staging of the boundary's arrays (stage_buffer)
     double* out_buf = nullptr;           // kst_get_output staging, out_cap doubles
     size_t out_cap = 0;
@@ -2865,12 +2866,11 @@ struct kst_handle {
 };
 
 // Device scratch of kst_volume_noalloc: the partial sums of the volume
-// kernels (VOL_BLOCKS_MAX groups) and their merged result (one group), the
-// same layout as the handle's vol_part.  One copy per GPU, held until the
+// kernels (VOL_BLOCKS_MAX groups), the same layout as the handle's vol_part.  One copy per GPU, held until the
 // process ends; every call on that GPU shares it.  In host code the array's
 // name stands for no device address: its address on each device comes from
 // hipGetSymbolAddress (scratch_ptr), taken once per device in kst_create.
-constexpr size_t kScratchDoubles = (size_t)(VOL_BLOCKS_MAX + 1) * VOL_Q * 2;
+constexpr size_t kScratchDoubles = (size_t)VOL_BLOCKS_MAX * VOL_Q * 2;
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
 // A batch: a fixed table of slots, each holding a scenario handle whose
@@ -3514,7 +3514,8 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
     d.morpho = cfg->morphodynamics ? 1 : 0;
     d.mixed = cfg->precision == KST_PREC_MIXED ? 1 : 0;
     rc |= dalloc(h, &d.S0, 4 * FS);
-    rc |= dalloc(h, &h->vol_part, (size_t)(VOL_BLOCKS_MAX + 1) * VOL_Q * 2);
+    rc |= dalloc(h, &h->vol_part, kScratchDoubles);
+    rc |= hipHostMalloc(&h->vol_sum, VOL_Q * 2 * sizeof(double), hipHostMallocDefault) != hipSuccess;
     rc |= dalloc(h, &d.UVo, 2 * FS);
     if (d.mixed) {
         // S2, S3 (4 fields) and R (5 fields) hold floats
@@ -3835,20 +3836,19 @@ int kst_get_state(kst_handle* h, double* w, double* rhu, double* rhv, double* hn
 namespace {
 
 // CalculateVolume with the partial sums in `part`, which holds `cap` doubles
-// (VOL_BLOCKS_MAX + 1 groups of VOL_Q pairs suffice for any active set).
+// (VOL_BLOCKS_MAX groups of VOL_Q pairs suffice for any active set).  The last
+// kernel writes the sums to pinned host memory itself: a copy of 64 bytes
+// behind it took as long as both kernels' launches.
 int volume_into(kst_handle* h, double* part, size_t cap, double out[6]) {
     const int nb = volume_partials(h->ntiles);
-    if ((size_t)(VOL_BLOCKS_MAX + 1) * VOL_Q * 2 > cap)
+    if (kScratchDoubles > cap)
         return set_err(h, KST_ERR_CONFIG, "volume: the partial-sum buffer holds " + std::to_string(cap) +
-                                              " doubles; " + std::to_string((VOL_BLOCKS_MAX + 1) * VOL_Q * 2) +
-                                              " are needed");
-    double* fin = part + (size_t)VOL_BLOCKS_MAX * VOL_Q * 2;
+                                              " doubles; " + std::to_string(kScratchDoubles) + " are needed");
     hipLaunchKernelGGL(volume_kernel, dim3(nb), dim3(VOL_NT), 0, h->stream, h->d_args, h->d_par, part);
-    hipLaunchKernelGGL(volume_final_kernel, dim3(1), dim3(VOL_NT), 0, h->stream, h->d_args, part, fin);
+    hipLaunchKernelGGL(volume_final_kernel, dim3(1), dim3(VOL_NT), 0, h->stream, h->d_args, part, h->vol_sum);
     HIPCHK(h, hipGetLastError());
-    double r[VOL_Q * 2];
-    HIPCHK(h, hipMemcpyAsync(r, fin, sizeof r, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    const double* r = h->vol_sum;
     const kst_config& g = h->cfg;
     // each sum times dx dy, then the columns as CalculateVolume writes them
     // (src/Output.f90:709-730)
@@ -3870,7 +3870,7 @@ int volume_into(kst_handle* h, double* part, size_t cap, double out[6]) {
 int kst_volume(kst_handle* h, double out[6]) {
     if (!h || !out) return KST_ERR_CONFIG;
     if (!h->have_state) return set_err(h, KST_ERR_STATE, "kst_set_state must come first");
-    return volume_into(h, h->vol_part, (size_t)(VOL_BLOCKS_MAX + 1) * VOL_Q * 2, out);
+    return volume_into(h, h->vol_part, kScratchDoubles, out);
 }
 
 int kst_volume_noalloc(kst_handle* h, double out[6]) {
@@ -3882,9 +3882,8 @@ int kst_volume_noalloc(kst_handle* h, double out[6]) {
         return set_err(h, KST_ERR_CONFIG, "kst_volume_noalloc: the handle's device must be current");
     double* part = scratch_ptr(h->device);
     if (!part) return set_err(h, KST_ERR_STATE, "kst_volume_noalloc: no scratch address for this device");
-    // the volume kernels write at most VOL_BLOCKS_MAX partial groups and one
-    // merged group, which is what scratch holds; volume_into refuses a
-    // buffer smaller than that
+    // the volume kernels write at most VOL_BLOCKS_MAX partial groups, which is
+    // what scratch holds; volume_into refuses a buffer smaller than that
     return volume_into(h, part, kScratchDoubles, out);
 }
 
@@ -4389,6 +4388,7 @@ void kst_destroy(kst_handle* h) {
     for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (void* p : h->allocs) (void)hipFree(p);
+    if (h->vol_sum) (void)hipHostFree(h->vol_sum);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
 }
