@@ -69,8 +69,10 @@ struct Ctrl {
     int cur;                   // mixed precision: u^n is in S0 (0) or S0b (1)
     double next_t;             // NextFluxSeriesTime of t, kept with t
     // every vertex bt is +0 and stays so (no morphodynamics): bt of the cells
-    // and faces is 0 and a face's CorrectSlopes bed is its b0, and the stage
-    // kernels read neither
+    // and faces is 0 and a face's CorrectSlopes bed is its b0, the same on
+    // both sides of a tile edge, and the stage kernels read none of them.
+    // Not set where a periodic boundary joins vertices of different b0
+    // (kst_handle::b0_wraps): the tiles either side hold different beds there
     int flat;
     // CFL minima: first hydraulic operator stages 1..3, then the second
     // operator of a Strang step stages 1..3
@@ -2839,6 +2841,7 @@ struct kst_handle {
     std::string err;
     int nx, ny, ntx, nty, ntiles, NX, NY, NC;
     bool have_topo = false, have_state = false;
+    bool b0_wraps = true;   // the vertices that periodic boundaries join hold the same b0
     std::vector<std::vector<double>> src_times;   // flux-source knot times (host copy)
     std::vector<double> src_xyr;                  // flux sources' x, y, radius (host copy)
     double t = 0.0;
@@ -3612,6 +3615,20 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
     return KST_OK;
 }
 
+// Whether b0 is the same on the vertices that periodic boundaries join: the
+// last column and the first, the last row and the first (the columns of the
+// lower row on a 1D grid).  The boundary asks for it and nothing enforces it:
+// the tiles either side of the seam then each see their own bed there.
+static bool periodic_bed_wraps(const kst_handle* h, const double* b0v) {
+    if (h->cfg.bc != KST_BC_PERIODIC) return true;
+    const size_t GX = (size_t)h->NX + 1;
+    for (int J = 0; J <= (h->p.oned ? 0 : h->NY); ++J)
+        if (!(b0v[J * GX] == b0v[J * GX + h->NX])) return false;
+    for (size_t I = 0; !h->p.oned && I < GX; ++I)
+        if (!(b0v[I] == b0v[h->NY * GX + I])) return false;
+    return true;
+}
+
 int kst_set_topography(kst_handle* h, const double* b0v) {
     if (!h || !b0v) return KST_ERR_CONFIG;
     int rc = stage_buffer(h);
@@ -3623,6 +3640,15 @@ int kst_set_topography(kst_handle* h, const double* b0v) {
     rc = refresh_topography(h);
     if (rc) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    h->b0_wraps = periodic_bed_wraps(h, b0v);
+    if (h->have_state && !h->b0_wraps) {   // under a state that was set over another bed
+        Ctrl c;
+        rc = read_ctrl(h, &c);
+        if (rc) return rc;
+        c.flat = 0;
+        rc = write_ctrl(h, &c);
+        if (rc) return rc;
+    }
     h->have_topo = true;
     return KST_OK;
 }
@@ -3689,7 +3715,7 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
     // vertex bt: each active tile takes its own copy of the global values
     // (ghost tiles keep bt = 0, as AllocateTopographicData leaves them),
     // then the topography of every set follows
-    bool flat = true;
+    bool flat = true;   // Ctrl::flat, as far as bt goes
     {
         const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
         // all +0 to the last bit
@@ -3749,7 +3775,7 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
     c.status = ST_DONE;
     c.n_active = (int)act.size();
     c.n_ghost = (int)gh.size();
-    c.flat = h->d.morpho ? 0 : (int)flat;
+    c.flat = h->d.morpho || !h->b0_wraps ? 0 : (int)flat;
     rc = write_ctrl(h, &c);
     if (rc) return rc;
     if (!gh.empty())
