@@ -3745,7 +3745,8 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
     // containsSource: tiles holding a cell within a flux source's radius
     // (src/SetSources.f90:357-375)
     for (int q = 0; q < h->cfg.n_sources; ++q) {
-        const double sx = h->src_xyr[3 * q], sy = h->src_xyr[3 * q + 1], sr = h->src_xyr[3 * q + 2];
+        // (only the radius' square is compared: its sign means nothing)
+        const double sx = h->src_xyr[3 * q], sy = h->src_xyr[3 * q + 1], sr = std::fabs(h->src_xyr[3 * q + 2]);
         // the rows and columns that the circle can touch, and one more
         auto range = [&](double at, double size, double d, int n, int& lo, int& hi) {
             lo = (int)std::max(0.0, std::min((double)n, std::floor((at - sr + 0.5 * size) / d) - 1.0));
