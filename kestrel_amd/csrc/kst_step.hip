@@ -2047,15 +2047,16 @@ __device__ void tile_static_terms(const DevT& d, const Params& p, const TopoT& T
 
 // Ghost w slopes at the edge of tile g on side r (0..3: W, E, S, N) where it
 // faces an active tile (ReconstructwAtEdges, src/UpdateTiles.f90:669-750).
-// One wave's work; the loads leave whatever the neighbour's state (clamped
-// into the grid), with it.
+// One wave's work.  A 1D grid has no sides S and N: its tiles hold no second
+// row to read, and with periodic boundaries nb_tile gives the tile itself
+// there.
 template <class DevT>
 __device__ __forceinline__ void ghost_side_slopes(const DevT& d, const Params& p, int g, int r) {
+    if (p.oned && r >= 2) return;
     const int nx = p.nx, ny = p.ny, NC = p.NC;
     const double* w = (d.mixed && d.ctrl->cur) ? d.S0b : d.S0;
     const int nb = nb_tile(p, g, r == 0 ? -1 : (r == 1 ? 1 : 0), r == 2 ? -1 : (r == 3 ? 1 : 0));
-    if (nb < 0 || nb >= p.ntiles) return;
-    const bool on = d.tstate[nb] == KST_TILE_ACTIVE;
+    if (nb < 0 || nb >= p.ntiles || d.tstate[nb] != KST_TILE_ACTIVE) return;
     const bool X = r < 2;
     const int n = X ? ny : nx;
     const size_t base = (size_t)g * NC, nbase = (size_t)nb * NC;
@@ -2065,7 +2066,6 @@ __device__ __forceinline__ void ghost_side_slopes(const DevT& d, const Params& p
         const int in = X ? own + (r == 0 ? 1 : -1) : own + (r == 2 ? nx : -nx);
         const int ex = X ? k * nx + (r == 0 ? nx - 1 : 0) : k + (r == 2 ? (ny - 1) * nx : 0);
         const double c = w[base + own], i = w[base + in], e = w[nbase + ex];
-        if (!on) continue;
         const bool low = r == 0 || r == 2;
         const double up = low ? i - c : e - c, down = low ? c - e : c - i;
         (X ? d.gsx : d.gsy)[base + own] = (X ? p.dxr : p.dyr) * limiter(p.limiter, up, down);
