@@ -2860,7 +2860,7 @@ struct kst_handle {
     std::map<int, Tune> tuned;           // bucket (active tiles, rounded up to a power of two)
     double* vol_part = nullptr;          // volume partials (VOL_BLOCKS_MAX groups)
     double* vol_sum = nullptr;           // their sums, in pinned host memory
-    double* io = nullptr;                // staging of the boundary's arrays (stage_buffer)
+    struct Stage* stage = nullptr;       // the device's staging of the boundary's arrays
     double* out_buf = nullptr;           // kst_get_output staging, out_cap doubles
     size_t out_cap = 0;
     std::vector<hipEvent_t> ev;          // 8 per iteration of the current batch
@@ -2947,6 +2947,91 @@ int dalloc(kst_handle* h, T** ptr, size_t n) {
     *ptr = static_cast<T*>(p);
     return 0;
 }
+
+}  // namespace
+
+// The staging of the boundary's arrays (kst_io.hpp): one buffer per GPU for all
+// its handles, since a call needs it only while its arrays cross the link.  It
+// grows to what the largest grid asks for, at most kStageDoubles (64 MB; larger
+// arrays cross in chunks, 11 MB and more each, whose extra copies are lost in
+// the transfer), and is given back with the last handle.  A buffer for the
+// whole grid in each handle was 11% of a scenario's memory.
+constexpr size_t kStageDoubles = (size_t)8 << 20, kStageLeast = (size_t)8 << 10;
+struct Stage {
+    std::mutex m;
+    double* p = nullptr;
+    size_t n = 0;        // doubles it holds
+    int handles = 0;     // handles of the device
+};
+
+namespace {
+
+std::mutex g_stages_mutex;
+std::map<int, Stage>& stages() {
+    static std::map<int, Stage>* s = new std::map<int, Stage>();   // handles may outlive static objects
+    return *s;
+}
+
+void stage_join(kst_handle* h) {
+    {
+        std::lock_guard<std::mutex> lk(g_stages_mutex);
+        h->stage = &stages()[h->device];
+    }
+    std::lock_guard<std::mutex> lk(h->stage->m);
+    h->stage->handles += 1;
+}
+
+void stage_leave(kst_handle* h) {
+    if (!h->stage) return;
+    std::lock_guard<std::mutex> lk(h->stage->m);
+    if (--h->stage->handles > 0) return;
+    (void)hipFree(h->stage->p);
+    h->stage->p = nullptr;
+    h->stage->n = 0;
+}
+
+// The staging for the length of a call, which has it to itself (other handles'
+// calls, in other threads, wait): n >= kStageLeast doubles at p, `want` of them
+// if they fit.  On leaving, the handle's stream is done with it.
+class StageUse {
+    kst_handle* h;
+    std::unique_lock<std::mutex> lk;
+
+  public:
+    double* p = nullptr;
+    size_t n = 0;
+    int rc = 0;
+
+    StageUse(kst_handle* handle, size_t want) : h(handle), lk(handle->stage->m) {
+        Stage& s = *h->stage;
+        want = std::max(kStageLeast, std::min(want, kStageDoubles));
+        if (s.n < want) {
+            int cur = h->device;
+            (void)hipGetDevice(&cur);
+            if (cur != h->device) (void)hipSetDevice(h->device);
+            (void)hipFree(s.p);
+            s.p = nullptr;
+            s.n = 0;
+            // with little memory left, a smaller one
+            for (size_t k = want; !s.p && k >= kStageLeast; k /= 2) {
+                void* q = nullptr;
+                if (hipMalloc(&q, k * sizeof(double)) == hipSuccess) {
+                    s.p = static_cast<double*>(q);
+                    s.n = k;
+                } else {
+                    (void)hipGetLastError();
+                }
+            }
+            if (cur != h->device) (void)hipSetDevice(cur);
+        }
+        p = s.p;
+        n = s.n;
+        if (!p) rc = set_err(h, KST_ERR_HIP, "no device memory for the staging of the arrays");
+    }
+    ~StageUse() { (void)hipStreamSynchronize(h->stream); }
+    StageUse(const StageUse&) = delete;
+    StageUse& operator=(const StageUse&) = delete;
+};
 
 int alloc_topo(kst_handle* h, Topo& T) {
     const size_t FS = (size_t)h->ntiles * h->NC;
@@ -3052,36 +3137,47 @@ int write_ctrl(kst_handle* h, const Ctrl* c) {
     return 0;
 }
 
-// The handle's staging buffer for the boundary's arrays (kst_io.hpp): five
-// cell arrays, one vertex array and the time, allocated at the first call that
-// needs it.
-int stage_buffer(kst_handle* h) {
-    if (h->io) return 0;
-    const size_t cells = (size_t)h->NX * h->NY, verts = (size_t)(h->NX + 1) * (h->NY + 1);
-    void* p = nullptr;
-    HIPCHK(h, hipMalloc(&p, (5 * cells + verts + 1) * sizeof(double)));
-    h->allocs.push_back(p);
-    h->io = static_cast<double*>(p);
-    return 0;
-}
-
 // Blocks of a kernel that walks n elements (grid-stride).
 int io_blocks(size_t n) { return (int)std::min<size_t>((n + IO_NT - 1) / IO_NT, 65536); }
 
-// One cell array to the device and into tile order, or back (ts: 0 outside
-// allocated tiles); on the handle's stream.
-int put_cells(kst_handle* h, const double* host, double* dev) {
-    const size_t n = (size_t)h->NX * h->NY;
-    HIPCHK(h, hipMemcpyAsync(h->io, host, n * 8, hipMemcpyHostToDevice, h->stream));
-    hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, h->io,
-                       (const uint8_t*)nullptr, dev);
+// One cell array to the device and into tile order, or back, through the
+// staging; on the handle's stream.
+int put_cells(kst_handle* h, const StageUse& io, const double* host, double* dev) {
+    const size_t cells = (size_t)h->NX * h->NY;
+    for (size_t g0 = 0; g0 < cells; g0 += io.n) {
+        const size_t n = std::min(io.n, cells - g0);
+        HIPCHK(h, hipMemcpyAsync(io.p, host + g0, n * 8, hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, io.p,
+                           (const uint8_t*)nullptr, dev, g0, n);
+        HIPCHK(h, hipGetLastError());
+    }
     return 0;
 }
-int get_cells(kst_handle* h, const double* dev, const uint8_t* ts, double* host) {
-    const size_t n = (size_t)h->NX * h->NY;
-    hipLaunchKernelGGL(gather_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, dev, ts, h->io);
-    HIPCHK(h, hipGetLastError());
-    HIPCHK(h, hipMemcpyAsync(host, h->io, n * 8, hipMemcpyDeviceToHost, h->stream));
+int get_cells(kst_handle* h, const StageUse& io, const double* dev, double* host) {
+    const size_t cells = (size_t)h->NX * h->NY;
+    for (size_t g0 = 0; g0 < cells; g0 += io.n) {
+        const size_t n = std::min(io.n, cells - g0);
+        hipLaunchKernelGGL(gather_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, dev, io.p, g0, n);
+        HIPCHK(h, hipGetLastError());
+        HIPCHK(h, hipMemcpyAsync(host + g0, io.p, n * 8, hipMemcpyDeviceToHost, h->stream));
+    }
+    return 0;
+}
+
+// One vertex array (nullptr: 0 everywhere) into the tiles' copies
+// (scatter_vertices_kernel), each chunk by the rows of tiles that hold its rows
+// of vertices.
+int put_vertices(kst_handle* h, const StageUse& io, const double* host, const uint8_t* active, const VertexSets& sets) {
+    const size_t GX = (size_t)h->NX + 1, verts = GX * (h->NY + 1), step = host ? io.n : verts;
+    for (size_t g0 = 0; g0 < verts; g0 += step) {
+        const size_t n = std::min(step, verts - g0);
+        const int r0 = (int)(g0 / GX), r1 = (int)((g0 + n - 1) / GX);
+        const int first = r0 > 0 ? (r0 - 1) / h->ny : 0, last = std::min(r1 / h->ny, h->nty - 1);
+        if (host) HIPCHK(h, hipMemcpyAsync(io.p, host + g0, n * 8, hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(scatter_vertices_kernel, dim3((last - first + 1) * h->ntx), dim3(IO_NT), 0, h->stream, h->p,
+                           host ? io.p : (const double*)nullptr, active, sets, first * h->ntx, g0, n);
+        HIPCHK(h, hipGetLastError());
+    }
     return 0;
 }
 
@@ -3510,6 +3606,7 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
         delete h;
         return e;
     }
+    stage_join(h);
     Dev& d = h->d;
     const size_t FS = (size_t)h->ntiles * h->NC;
     const size_t NV = (size_t)(h->nx + 1) * (h->ny + 1);
@@ -3631,12 +3728,10 @@ static bool periodic_bed_wraps(const kst_handle* h, const double* b0v) {
 
 int kst_set_topography(kst_handle* h, const double* b0v) {
     if (!h || !b0v) return KST_ERR_CONFIG;
-    int rc = stage_buffer(h);
+    const StageUse io(h, (size_t)(h->NX + 1) * (h->NY + 1));
+    if (io.rc) return io.rc;
+    int rc = put_vertices(h, io, b0v, nullptr, VertexSets{{h->d.vb0}, 1});
     if (rc) return rc;
-    const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
-    HIPCHK(h, hipMemcpyAsync(h->io, b0v, verts * 8, hipMemcpyHostToDevice, h->stream));
-    hipLaunchKernelGGL(scatter_vertices_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->p, h->io,
-                       (const uint8_t*)nullptr, VertexSets{{h->d.vb0}, 1});
     rc = refresh_topography(h);
     if (rc) return rc;
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -3669,8 +3764,6 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                   const double* hnmax0) {
     if (!h || !w || !rhu || !rhv || !hnpsi || !ts) return KST_ERR_CONFIG;
     if (!h->have_topo) return set_err(h, KST_ERR_STATE, "kst_set_topography must come first");
-    int rc = stage_buffer(h);
-    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
     // tile lists: active sorted by id; ghosts = the non-active neighbours of
     // active tiles that AddGhostTiles takes (src/UpdateTiles.f90:389-481):
@@ -3711,29 +3804,28 @@ int kst_set_state(kst_handle* h, const double* w, const double* rhu, const doubl
                 if (st[n] == KST_TILE_OFF) { st[n] = KST_TILE_GHOST; gh.push_back(n); }
             }
     }
+    const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
+    const StageUse io(h, std::max(5 * FS, verts));
+    if (io.rc) return io.rc;
     HIPCHK(h, hipMemcpyAsync(h->d.tstate, st.data(), st.size(), hipMemcpyHostToDevice, h->stream));
     // vertex bt: each active tile takes its own copy of the global values
     // (ghost tiles keep bt = 0, as AllocateTopographicData leaves them),
     // then the topography of every set follows
-    bool flat = true;   // Ctrl::flat, as far as bt goes
-    {
-        const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1);
-        // all +0 to the last bit
-        for (size_t q = 0; btv && flat && q < verts; ++q) flat = btv[q] == 0.0 && !std::signbit(btv[q]);
-        if (btv) HIPCHK(h, hipMemcpyAsync(h->io, btv, verts * 8, hipMemcpyHostToDevice, h->stream));
-        VertexSets sets{{h->d.TA.vbt, h->d.TB.vbt, h->d.TM[0].vbt, h->d.TM[1].vbt}, h->d.morpho ? 4 : 1};
-        hipLaunchKernelGGL(scatter_vertices_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->p,
-                           btv ? h->io : (double*)nullptr, h->d.tstate, sets);
-        rc = refresh_topography(h);
-        if (rc) return rc;
-    }
+    bool flat = true;   // Ctrl::flat, as far as bt goes: all +0 to the last bit
+    for (size_t q = 0; btv && flat && q < verts; ++q) flat = btv[q] == 0.0 && !std::signbit(btv[q]);
+    int rc = put_vertices(h, io, btv, h->d.tstate,
+                          VertexSets{{h->d.TA.vbt, h->d.TB.vbt, h->d.TM[0].vbt, h->d.TM[1].vbt}, h->d.morpho ? 4 : 1});
+    if (rc) return rc;
+    rc = refresh_topography(h);
+    if (rc) return rc;
     // the fields, and all that starts from them
-    {
-        const double* in[5] = {w, rhu, rhv, hnpsi, hnmax0};
+    const double* in[5] = {w, rhu, rhv, hnpsi, hnmax0};
+    for (size_t g0 = 0, step = io.n / 5; g0 < FS; g0 += step) {
+        const size_t n = std::min(step, FS - g0);
         for (int q = 0; q < 5; ++q)
-            if (in[q]) HIPCHK(h, hipMemcpyAsync(h->io + q * FS, in[q], FS * 8, hipMemcpyHostToDevice, h->stream));
-        hipLaunchKernelGGL(scatter_state_kernel, dim3(h->ntiles), dim3(IO_NT), 0, h->stream, h->d, h->p, h->io,
-                           hnmax0 ? 1 : 0);
+            if (in[q]) HIPCHK(h, hipMemcpyAsync(io.p + q * n, in[q] + g0, n * 8, hipMemcpyHostToDevice, h->stream));
+        hipLaunchKernelGGL(scatter_state_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->d, h->p, io.p,
+                           hnmax0 ? 1 : 0, g0, n);
         HIPCHK(h, hipGetLastError());
     }
     std::vector<int> actp(act), ghp(gh);
@@ -3835,28 +3927,37 @@ int kst_step_n(kst_handle* h, int64_t n, kst_stats* st) {
 int kst_get_state(kst_handle* h, double* w, double* rhu, double* rhv, double* hnpsi, double* hn,
                   double* btv, uint8_t* ts, double* t) {
     if (!h) return KST_ERR_CONFIG;
-    int rc = stage_buffer(h);
-    if (rc) return rc;
-    const size_t FS = (size_t)h->ntiles * h->NC;
-    const size_t verts = (size_t)(h->NX + 1) * (h->NY + 1), total = 5 * FS + verts + 1;
-    hipLaunchKernelGGL(gather_state_kernel, dim3(io_blocks(verts)), dim3(IO_NT), 0, h->stream, h->d, h->p, h->io);
-    HIPCHK(h, hipGetLastError());
-    double* out[7] = {w, rhu, rhv, hnpsi, hn, btv, t};
-    const size_t at[8] = {0, FS, 2 * FS, 3 * FS, 4 * FS, 5 * FS, 5 * FS + verts, total};
+    const size_t FS = (size_t)h->ntiles * h->NC, verts = (size_t)(h->NX + 1) * (h->NY + 1);
+    const StageUse io(h, 6 * verts + 1);
+    if (io.rc) return io.rc;
+    double* out[6] = {w, rhu, rhv, hnpsi, hn, btv};
+    const size_t step = std::min(verts, (io.n - 1) / 6);
     // a small state in one copy (each costs about 15 us), a large one array by array
     std::vector<double> all;
-    if (total * 8 <= (1u << 20)) {
-        all.resize(total);
-        HIPCHK(h, hipMemcpyAsync(all.data(), h->io, total * 8, hipMemcpyDeviceToHost, h->stream));
-    } else {
-        for (int q = 0; q < 7; ++q)
-            if (out[q])
-                HIPCHK(h, hipMemcpyAsync(out[q], h->io + at[q], (at[q + 1] - at[q]) * 8, hipMemcpyDeviceToHost, h->stream));
+    if (step == verts && (6 * verts + 1) * 8 <= (1u << 20)) all.resize(6 * verts + 1);
+    for (size_t g0 = 0; g0 < verts; g0 += step) {
+        const size_t n = std::min(step, verts - g0);
+        hipLaunchKernelGGL(gather_state_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->d, h->p, io.p, g0, n);
+        HIPCHK(h, hipGetLastError());
+        if (!all.empty()) {
+            HIPCHK(h, hipMemcpyAsync(all.data(), io.p, all.size() * 8, hipMemcpyDeviceToHost, h->stream));
+            break;
+        }
+        for (int q = 0; q < 6; ++q) {
+            const size_t len = q < 5 ? FS : verts;
+            if (out[q] && g0 < len)
+                HIPCHK(h, hipMemcpyAsync(out[q] + g0, io.p + q * n, std::min(n, len - g0) * 8, hipMemcpyDeviceToHost,
+                                         h->stream));
+        }
+        if (t && g0 == 0) HIPCHK(h, hipMemcpyAsync(t, io.p + 6 * n, 8, hipMemcpyDeviceToHost, h->stream));
     }
     if (ts) HIPCHK(h, hipMemcpyAsync(ts, h->d.tstate, (size_t)h->ntiles, hipMemcpyDeviceToHost, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
-    for (int q = 0; q < 7 && !all.empty(); ++q)
-        if (out[q]) std::memcpy(out[q], all.data() + at[q], (at[q + 1] - at[q]) * 8);
+    if (!all.empty()) {
+        for (int q = 0; q < 6; ++q)
+            if (out[q]) std::memcpy(out[q], all.data() + q * verts, (q < 5 ? FS : verts) * 8);
+        if (t) *t = all.back();
+    }
     return KST_OK;
 }
 
@@ -3950,12 +4051,12 @@ int kst_get_output(kst_handle* h, int32_t max_tiles, double* fields, int32_t* ti
 
 int kst_get_maxima(kst_handle* h, double* const mx[11]) {
     if (!h || !mx) return KST_ERR_CONFIG;
-    int rc = stage_buffer(h);
-    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
+    const StageUse io(h, FS);
+    if (io.rc) return io.rc;
     for (int q = 0; q < 11; ++q)
         if (mx[q]) {
-            rc = get_cells(h, h->d.maxima + q * FS, nullptr, mx[q]);
+            const int rc = get_cells(h, io, h->d.maxima + q * FS, mx[q]);
             if (rc) return rc;
         }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -3964,15 +4065,14 @@ int kst_get_maxima(kst_handle* h, double* const mx[11]) {
 
 int kst_set_maxima(kst_handle* h, const double* const mx[11]) {
     if (!h || !mx) return KST_ERR_CONFIG;
-    int rc = stage_buffer(h);
-    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
+    const StageUse io(h, FS);
+    if (io.rc) return io.rc;
     for (int q = 0; q < 11; ++q)
         if (mx[q]) {
-            rc = put_cells(h, mx[q], h->d.maxima + q * FS);
+            const int rc = put_cells(h, io, mx[q], h->d.maxima + q * FS);
             if (rc) return rc;
         }
-    HIPCHK(h, hipGetLastError());
     HIPCHK(h, hipStreamSynchronize(h->stream));
     return KST_OK;
 }
@@ -3989,25 +4089,32 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
                             const uint8_t* cells) {
     if (!h || !btc || !dbdx || !dbdy || !cells) return KST_ERR_CONFIG;
     if (!h->have_state) return set_err(h, KST_ERR_STATE, "kst_set_state must come first");
-    int rc = stage_buffer(h);
-    if (rc) return rc;
     const size_t FS = (size_t)h->ntiles * h->NC;
+    // a chunk of a field, and behind it that of the mask
+    const StageUse io(h, FS + FS / 8 + 1);
+    if (io.rc) return io.rc;
     // every set takes the given cells of each field (all hold the same cell
-    // topography after kst_set_state); the mask after the field in the stage
+    // topography after kst_set_state)
     Topo* sets[4] = {&h->d.TA, &h->d.TB, &h->d.TM[0], &h->d.TM[1]};
     const int nsets = h->d.morpho ? 4 : 1;
     const double* src[3] = {btc, dbdx, dbdy};
-    uint8_t* mask = reinterpret_cast<uint8_t*>(h->io + FS);
-    HIPCHK(h, hipMemcpyAsync(mask, cells, FS, hipMemcpyHostToDevice, h->stream));
-    for (int f = 0; f < 3; ++f) {
-        double* from = f == 0 ? h->d.TA.btc : (f == 1 ? h->d.TA.cbx : h->d.TA.cby);
-        HIPCHK(h, hipMemcpyAsync(h->io, src[f], FS * 8, hipMemcpyHostToDevice, h->stream));
-        hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(FS)), dim3(IO_NT), 0, h->stream, h->p, h->io, mask, from);
-        for (int k = 1; k < nsets; ++k) {
-            double* to = f == 0 ? sets[k]->btc : (f == 1 ? sets[k]->cbx : sets[k]->cby);
-            HIPCHK(h, hipMemcpyAsync(to, from, FS * 8, hipMemcpyDeviceToDevice, h->stream));
+    double* const first[3] = {h->d.TA.btc, h->d.TA.cbx, h->d.TA.cby};
+    for (size_t g0 = 0, step = io.n / 9 * 8; g0 < FS; g0 += step) {
+        const size_t n = std::min(step, FS - g0);
+        uint8_t* mask = reinterpret_cast<uint8_t*>(io.p + n);
+        HIPCHK(h, hipMemcpyAsync(mask, cells + g0, n, hipMemcpyHostToDevice, h->stream));
+        for (int f = 0; f < 3; ++f) {
+            HIPCHK(h, hipMemcpyAsync(io.p, src[f] + g0, n * 8, hipMemcpyHostToDevice, h->stream));
+            hipLaunchKernelGGL(scatter_cells_kernel, dim3(io_blocks(n)), dim3(IO_NT), 0, h->stream, h->p, io.p, mask,
+                               first[f], g0, n);
+            HIPCHK(h, hipGetLastError());
         }
     }
+    for (int f = 0; f < 3; ++f)
+        for (int k = 1; k < nsets; ++k) {
+            double* to = f == 0 ? sets[k]->btc : (f == 1 ? sets[k]->cbx : sets[k]->cby);
+            HIPCHK(h, hipMemcpyAsync(to, first[f], FS * 8, hipMemcpyDeviceToDevice, h->stream));
+        }
     for (int k = 0; k < nsets; ++k)
         hipLaunchKernelGGL(cell_gamma_kernel, dim3(h->ntiles), dim3(256), 0, h->stream, h->d, h->p, *sets[k]);
     for (int k = 0; k < nsets; ++k)
@@ -4015,7 +4122,7 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
     // what kst_set_state derived from the cell topography: the activation
     // flags of the active tiles and tileContainer's velocities
     Ctrl c;
-    rc = read_ctrl(h, &c);
+    int rc = read_ctrl(h, &c);
     if (rc) return rc;
     if (c.flat) {   // the cells' bt may now differ from the vertices'
         c.flat = 0;
@@ -4036,13 +4143,13 @@ int kst_set_cell_topography(kst_handle* h, const double* btc, const double* dbdx
 
 int kst_get_cell_topography(kst_handle* h, double* b0c, double* btc, double* dbdx, double* dbdy) {
     if (!h) return KST_ERR_CONFIG;
-    int rc = stage_buffer(h);
-    if (rc) return rc;
+    const StageUse io(h, (size_t)h->NX * h->NY);
+    if (io.rc) return io.rc;
     double* outs[4] = {b0c, btc, dbdx, dbdy};
     const double* srcs[4] = {h->d.b0c, h->d.TA.btc, h->d.TA.cbx, h->d.TA.cby};
     for (int q = 0; q < 4; ++q)
         if (outs[q]) {
-            rc = get_cells(h, srcs[q], nullptr, outs[q]);
+            const int rc = get_cells(h, io, srcs[q], outs[q]);
             if (rc) return rc;
         }
     HIPCHK(h, hipStreamSynchronize(h->stream));
@@ -4415,6 +4522,7 @@ void kst_destroy(kst_handle* h) {
     for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (void* p : h->allocs) (void)hipFree(p);
+    stage_leave(h);
     if (h->vol_sum) (void)hipHostFree(h->vol_sum);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;

@@ -1,0 +1,98 @@
+"""Device memory: the staging of the boundary's arrays is one bounded buffer for
+all handles of the device, given back with the last of them."""
+import numpy as np
+import pytest
+
+from kestrel_amd import config as C
+from kestrel_amd import workloads
+from tests.helpers import stepper_for
+
+pytestmark = pytest.mark.gpu
+
+MB = 1 << 20
+STAGE = 64 * MB
+
+
+def _used():
+    import torch
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def _warm():
+    """Code objects, queues and scratch the first launches bring."""
+    g = stepper_for(workloads.plain_cap(128, 0, tile=32, cap_x=0.0, cap_radius=10.0))
+    g.step_n(2)
+    g.state()
+    g.close()
+
+
+def test_staging_is_shared_and_given_back(gpu):
+    from kestrel_amd.runtime import Stepper
+    _warm()
+    wl = workloads.plain_cap(2048, 0, tile=32, cap_x=0.0, cap_radius=100.0)
+    start = _used()
+    handles, grown = [], []
+    for _ in range(2):
+        g = Stepper(wl.cfg)
+        created = _used()
+        g.set_topography(wl.b0v)
+        g.set_state(wl.init)
+        g.state()
+        g.maxima()
+        g.cell_topography()
+        handles.append(g)
+        grown.append(_used() - created)
+    assert grown[0] <= STAGE + 2 * MB and grown[1] <= 2 * MB, grown
+    for g in handles:
+        g.close()
+    assert _used() - start <= 2 * MB
+
+
+@pytest.mark.parametrize("tiles", [(61, 53, 31, 29), (85000, 1, 100, 1)], ids=["2d", "1d"])
+def test_arrays_larger_than_the_staging(gpu, tiles):
+    """Round trip in chunks: a state, its topography and maxima whose arrays
+    do not fit the staging at once (1d: not even one of them)."""
+    from kestrel_amd import scenario as S
+    from kestrel_amd.runtime import Stepper
+    cfg = C.default_config(*tiles, dx=2.0)
+    C.hydraulic_only(cfg)
+    cfg.bc = C.BC_SPONGE
+    C.derive(cfg)
+    rng = np.random.default_rng(3)
+    shape, verts = (cfg.NY, cfg.NX), (cfg.NY + 1, cfg.NX + 1)
+    b0v = rng.standard_normal(verts)
+    btv = rng.standard_normal(verts)
+    on = np.zeros((tiles[1], tiles[0]), np.uint8)
+    on[(1 if tiles[1] > 1 else 0):(tiles[1] - 1 if tiles[1] > 1 else 1), 1:-1] = 1
+    f = [rng.standard_normal(shape) for _ in range(4)]
+    init = S.InitialState(*f, on.reshape(-1), np.abs(rng.standard_normal(shape)))
+    g = Stepper(cfg)
+    g.set_topography(b0v)
+    g.set_state(init, t=1.5, btv=btv)
+    active = init.tile_state[S._tile_of_cells(cfg)] == 1
+    b0c, btc, bx, by = S.cell_topography(cfg, b0v, btv)
+    st = g.state()
+    assert st["t"] == 1.5
+    for name, a in zip(("w", "rhoHnu", "rhoHnv", "Hnpsi"), f):
+        assert np.array_equal(st[name][active], a[active]), name
+    own = np.zeros(verts, bool)   # vertices read from an active tile's copy
+    own[:-1, :-1] |= active
+    own[-1, :-1] |= active[-1]
+    assert np.array_equal(st["btv"][own], btv[own])
+    topo = g.cell_topography()
+    assert np.array_equal(topo["b0c"], b0c)
+    assert np.array_equal(topo["btc"][active], btc[active])
+    mx = g.maxima()
+    assert np.array_equal(mx[0], init.hnmax0) and (mx[10] == -1.0).all()
+    mx[3] = rng.standard_normal(shape)
+    g.set_maxima(mx)
+    assert np.array_equal(g.maxima()[3], mx[3])
+    cells = rng.uniform(size=shape) < 0.5
+    new = [rng.standard_normal(shape) for _ in range(3)]
+    g.set_cell_topography(*new, cells)
+    topo2 = g.cell_topography()
+    for name, a in zip(("btc", "dbdx", "dbdy"), new):
+        assert np.array_equal(topo2[name], np.where(cells, a, topo[name])), name
+    g.close()
