@@ -28,15 +28,35 @@ from . import scenario as S
 from . import workloads
 from .runtime import SLOT_DONE, SLOT_ERROR, SLOT_RUNNING, Batch, KestrelError, Stepper
 
-# Device bytes per cell of a scenario (every tile of the grid), by precision:
-# the FP64 state, stages and RHS, the cell and face topography, ghost slopes,
-# maxima and tile lists (kst_create's allocations), and the staging of the
-# boundary's arrays.
-BYTES_PER_CELL = {C.PREC_FP64: 8 * 54, C.PREC_MIXED: 8 * 51}
+
+def _held(nbytes: float) -> float:
+    """Device memory an allocation takes: whole pieces of 2 MB; small ones
+    share a piece, of which packing leaves up to a fifth."""
+    piece = 1 << 21
+    return 1.25 * nbytes if nbytes <= piece // 2 else piece * math.ceil(nbytes / piece)
 
 
 def device_bytes(cfg) -> int:
-    return int(cfg.NX * cfg.NY * BYTES_PER_CELL[cfg.precision])
+    """Device memory that a scenario holds while it is resident: the arrays of
+    kst_create over every tile of the grid.  (The staging of the boundary's
+    arrays, at most 64 MB, belongs to the device, not to a scenario.)"""
+    nx, ny, tiles = cfg.nx_per_tile, cfg.ny_per_tile, cfg.nx_tiles * cfg.ny_tiles
+    c, v, fx, fy = nx * ny, (nx + 1) * (ny + 1), (nx + 1) * ny, nx * (ny + 1)
+    # words a tile of each array: b0 at cells, faces and vertices, one
+    # generation of the bed's topography, ghost slopes, velocities, maxima,
+    # u^n; then the stages and the RHS (mixed precision: u^n twice, the rest
+    # in 32 bits)
+    topo = [v] + 7 * [c] + 6 * [fx] + 6 * [fy]
+    arrays = [c, fx, fy, v] + topo + [c, c, 2 * c, 11 * c, 4 * c]
+    arrays += [4 * c, 2 * c, 2 * c, 2.5 * c] if cfg.precision == C.PREC_MIXED else [4 * c, 4 * c, 5 * c]
+    total = 1 << 21
+    if cfg.morphodynamics:
+        # three further beds, u after the first operator, w and Hnpsi of three
+        # stages, velocities, the second operator's RHS, candidate positions;
+        # the candidates' keys and excesses padded to a power of two
+        arrays += 3 * topo + [4 * c, 2 * c, 2 * c, 2 * c, 2 * c, 5 * c, 0.5 * c]
+        total += 2 * _held(8 << max(0, c * tiles - 1).bit_length())
+    return int(total + sum(_held(8 * a * tiles) for a in arrays))
 
 
 @dataclass

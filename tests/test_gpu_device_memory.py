@@ -1,10 +1,11 @@
 """Device memory: the staging of the boundary's arrays is one bounded buffer for
-all handles of the device, given back with the last of them."""
+all handles of the device, given back with the last of them; what a scenario
+holds lies within what the server's admission counts for it."""
 import numpy as np
 import pytest
 
 from kestrel_amd import config as C
-from kestrel_amd import workloads
+from kestrel_amd import serving, workloads
 from tests.helpers import stepper_for
 
 pytestmark = pytest.mark.gpu
@@ -96,3 +97,24 @@ def test_arrays_larger_than_the_staging(gpu, tiles):
     for name, a in zip(("btc", "dbdx", "dbdy"), new):
         assert np.array_equal(topo2[name], np.where(cells, a, topo[name])), name
     g.close()
+
+
+@pytest.mark.parametrize("kind,n,tile", [("fp64", 192, 16), ("fp64", 512, 32), ("fp64", 2048, 32), ("mixed", 256, 16),
+                                         ("mixed", 512, 50), ("morpho", 256, 32), ("morpho", 1024, 32)])
+def test_admission_counts_what_a_scenario_holds(gpu, kind, n, tile):
+    _warm()
+    keep = stepper_for(workloads.plain_cap(2048, 0, tile=32, cap_x=0.0, cap_radius=100.0))   # the staging at its largest
+    if kind == "morpho":
+        wl = workloads.morpho_cap(n, 0, tile=tile)
+    else:
+        wl = workloads.plain_cap(n // tile * tile, 0, tile=tile, cap_x=0.0, cap_radius=0.1 * n)
+        wl.cfg.precision = C.PREC_MIXED if kind == "mixed" else C.PREC_FP64
+    count = 4 if n <= 512 else 1
+    before = _used()
+    handles = [stepper_for(wl) for _ in range(count)]
+    handles[0].state()
+    held = (_used() - before) / count
+    for g in handles + [keep]:
+        g.close()
+    counted = serving.device_bytes(wl.cfg)
+    assert held <= counted <= 1.3 * held + 4 * MB, (held, counted)
