@@ -292,6 +292,12 @@ int kst_autotune_choices(const kst_handle* h, int max, int32_t* bucket, int32_t*
  * small candidate sets.  0 restores a default. */
 int kst_set_redistribution_chunk(kst_handle* h, int chunk, int lds_sort);
 
+/* The sub-block of cells that one workgroup of the wide stage kernels takes in
+ * tiles of nx_per_tile x ny_per_tile cells (at least 4 x 4; no counterpart in
+ * the reference): the shape of at most 256 cells that covers a tile in the
+ * fewest.  Needs no device. */
+int kst_stage_sub_block(int nx_per_tile, int ny_per_tile, int32_t* width, int32_t* height);
+
 /* Activation candidates (no counterpart in the reference, whose
  * CheckIfNearBoundaries walks the active list itself,
  * src/TimeStepper.f90:935-1150).  After an accepted step the device collects

@@ -3065,20 +3065,25 @@ int refresh_topography(kst_handle* h) {
 // The wide stage kernels' sub-block for tiles of nx x ny cells: of the shapes
 // whose cells, faces, halo and LDS arrays a 256-thread workgroup holds, one
 // that covers the tile in the fewest workgroups -- each costs about the same
-// whatever its share of cells -- and among those the one with the smallest
-// halo.  32 x 32 tiles: 16 x 16.  The 50 x 50 tiles of the reference's decks:
-// 25 x 10, ten workgroups a tile instead of sixteen of 16 x 16, seven of
-// which hold 2 columns or rows.
+// whatever its share of cells -- among those one with the smallest halo, and of
+// the two that mirror each other the wider (cells lie row by row: its rows and
+// the two-cell pieces of its W and E halo are fewer and longer).  32 x 32
+// tiles: 16 x 16.  The 50 x 50 tiles of the reference's decks: 25 x 10, ten
+// workgroups a tile instead of sixteen of 16 x 16, seven of which hold 2
+// columns or rows.  The wider of the two against the taller, us a step of a
+// cap over 70% of the grid: tiles of 50 270.4 / 274.4 (mixed precision 245.8 /
+// 254.8), 40 264.7 / 266.9, 25 276.5 / 286.5, 24 257.4 / 258.3, 20 246.2 /
+// 246.4, 21 225.6 / 224.2.
 void wide_shape(Params& p) {
     int best = INT_MAX, halo = INT_MAX;
-    for (int w = 4; w <= std::min(p.nx, WIDE_EDGE); ++w)
+    for (int w = 4; w <= std::min(p.nx, WIDE_EDGE); ++w)          // the last of equals: the widest
         for (int h = 4; h <= std::min(p.ny, WIDE_EDGE); ++h) {
             if (w * h > STAGE_NT || (w + 1) * h > WIDE_FACES || w * (h + 1) > WIDE_FACES ||
                 (w + 4) * (h + 4) > WIDE_REG || h * (w + 3) > WIDE_BED || w * (h + 3) > WIDE_BED ||
                 4 * (w + h) > WIDE_HALO)
                 continue;
             const int n = ((p.nx + w - 1) / w) * ((p.ny + h - 1) / h);
-            if (n < best || (n == best && w + h < halo)) { best = n; halo = w + h; p.sw = w; p.sh = h; }
+            if (n < best || (n == best && w + h <= halo)) { best = n; halo = w + h; p.sw = w; p.sh = h; }
         }
     if (p.oned) { p.sw = p.sh = 4; }   // 1D grids have no wide kernels
     p.sbx = (p.nx + p.sw - 1) / p.sw;
@@ -4204,6 +4209,17 @@ int kst_set_redistribution_chunk(kst_handle* h, int chunk, int lds_sort) {
     const Dev both[2] = {h->d, h->d2};
     HIPCHK(h, hipMemcpyAsync(h->d_args, both, sizeof both, hipMemcpyHostToDevice, h->stream));
     HIPCHK(h, hipStreamSynchronize(h->stream));
+    return KST_OK;
+}
+
+int kst_stage_sub_block(int nx_per_tile, int ny_per_tile, int32_t* width, int32_t* height) {
+    if (nx_per_tile < 4 || ny_per_tile < 4 || !width || !height) return KST_ERR_CONFIG;
+    Params p{};
+    p.nx = nx_per_tile;
+    p.ny = ny_per_tile;
+    wide_shape(p);
+    *width = p.sw;
+    *height = p.sh;
     return KST_OK;
 }
 

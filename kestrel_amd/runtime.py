@@ -36,7 +36,8 @@ EXPORTS = ["kst_config_defaults", "kst_config_derive", "kst_create", "kst_set_to
            "kst_batch_run", "kst_batch_stats", "kst_batch_last_error", "kst_batch_destroy",
            "kst_get_cell_topography", "kst_set_maxima", "kst_get_output", "kst_volume", "kst_set_grid_cap",
            "kst_set_redistribution_chunk", "kst_autotune", "kst_autotune_choices",
-           "kst_volume_noalloc", "kst_set_cell_topography", "kst_set_activation_candidates"]
+           "kst_volume_noalloc", "kst_set_cell_topography", "kst_set_activation_candidates",
+           "kst_stage_sub_block"]
 
 
 class KstStats(ctypes.Structure):
@@ -89,6 +90,8 @@ def lib():
         i32p = ctypes.POINTER(ctypes.c_int32)
         L.kst_autotune_choices.argtypes = [ctypes.c_void_p, ctypes.c_int, i32p, i32p, i32p, _dp]
         L.kst_autotune_choices.restype = ctypes.c_int
+        L.kst_stage_sub_block.argtypes = [ctypes.c_int, ctypes.c_int, i32p, i32p]
+        L.kst_stage_sub_block.restype = ctypes.c_int
         L.kst_volume.argtypes = [ctypes.c_void_p, _dp]
         L.kst_volume.restype = ctypes.c_int
         L.kst_volume_noalloc.argtypes = [ctypes.c_void_p, _dp]
