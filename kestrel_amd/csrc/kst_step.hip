@@ -2579,36 +2579,35 @@ struct Verdict {
 };
 template <class DevT>
 __device__ __forceinline__ Verdict verdict(const DevT& d, const Params& p, const CtrlSnap* c) {
-    Verdict v{false, (c->status == ST_NEW ? 1 : 0) + 1, step_dt(d, p, c), 0.0};
+    Verdict v{false, 0, step_dt(d, p, c), 0.0};
     const double dt = v.dt;
-    auto check = [&](unsigned long long bits) {      // a CFL re-check
+    // The checks passed, counted once each after its outcome is known.  (Counted
+    // in the branches, 1 behind one check and 1 more behind the next, the
+    // compiler of ROCm 7.2 made of it a select of 2 or 3 by a scalar condition
+    // that it never set from the comparison: 7 instead of 8 evaluations a step.)
+    int passed = 0;
+    auto check = [&](unsigned long long bits) {       // a CFL re-check
         const double adv = advised_from_slot(p, bits, c->n_active);
-        if (adv < dt) {
-            v.reject = true;
-            v.retry = 0.9 * adv;
-        } else {
-            v.evals += 1;
-        }
+        v.reject = adv < dt;
+        if (v.reject) v.retry = 0.9 * adv;
+        passed += !v.reject;
     };
     check(c->slot[1].bits);
     if (!v.reject) check(c->slot[2].bits);
     if (d.morpho && !v.reject) {
-        if (c->mref) {
-            v.reject = true;
-            v.retry = 0.5 * dt;
-        } else {
-            v.evals += 1;
+        v.reject = c->mref != 0;
+        if (v.reject) v.retry = 0.5 * dt;
+        passed += !v.reject;
+        if (!v.reject) {
             const double adv = 0.9 * advised_from_slot(p, c->slot[3].bits, c->n_active);
-            if (adv < dt) {
-                v.reject = true;
-                v.retry = ((dt - adv) / dt < 0.1) ? 0.9 * dt : adv;
-            } else {
-                v.evals += 1;
-                check(c->slot[4].bits);
-                if (!v.reject) check(c->slot[5].bits);
-            }
+            v.reject = adv < dt;
+            if (v.reject) v.retry = ((dt - adv) / dt < 0.1) ? 0.9 * dt : adv;
+            passed += !v.reject;
         }
+        if (!v.reject) check(c->slot[4].bits);
+        if (!v.reject) check(c->slot[5].bits);
     }
+    v.evals = (c->status == ST_NEW ? 1 : 0) + 1 + passed;
     return v;
 }
 
