@@ -225,7 +225,7 @@ int kst_volume(kst_handle* h, double out[6]);
  * tight serving loops, harnesses that forbid hipMalloc -- the same sums as
  * kst_volume (the same kernels and partition, so the same bits) with the
  * partial sums in a fixed device array of the library (VOL_BLOCKS_MAX = 2048
- * groups of 8 doubles plus one, 131 KB per GPU, held until the process ends)
+ * groups of 8 doubles, 131 KB per GPU, held until the process ends)
  * instead of the handle's buffer.  The number of partial groups is capped at
  * that capacity (workgroups take further tiles in turn), so every active set
  * fits.  Calls no hipMalloc/hipFree and no allocating library routine.  The

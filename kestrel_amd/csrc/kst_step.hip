@@ -1741,7 +1741,7 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
         // final implicit substep (src/TimeStepper.f90:504-518)
         const double un = (oru - dt * dt * Eu * Im) / (1.0 + dt * dt * Im * Im);
         const double vn = (orv - dt * dt * Ev * Im) / (1.0 + dt * dt * Im * Im);
-        if (trk) update_maxima<Smem::oned>(d, p, oidx, mxv, mun, ob0, obt, gam, bx, by, s.tgrid + dt);
+        if (trk) update_maxima<false>(d, p, oidx, mxv, mun, ob0, obt, gam, bx, by, s.tgrid + dt);   // (2D only)
         double* Out = MIX ? (s.cur ? d.S0 : d.S0b) : d.Sout;
         Out[oidx] = ow; Out[FS + oidx] = un; Out[2 * FS + oidx] = vn; Out[3 * FS + oidx] = oh;
         if (d.last) { d.UVo[oidx] = ou; d.UVo[FS + oidx] = ov; }
@@ -3967,15 +3967,13 @@ int kst_get_state(kst_handle* h, double* w, double* rhu, double* rhv, double* hn
 
 namespace {
 
-// CalculateVolume with the partial sums in `part`, which holds `cap` doubles
-// (VOL_BLOCKS_MAX groups of VOL_Q pairs suffice for any active set).  The last
-// kernel writes the sums to pinned host memory itself: a copy of 64 bytes
-// behind it took as long as both kernels' launches.
-int volume_into(kst_handle* h, double* part, size_t cap, double out[6]) {
+// CalculateVolume with the partial sums in `part`, which holds kScratchDoubles:
+// volume_partials is at most VOL_BLOCKS_MAX groups of VOL_Q pairs, whatever the
+// active set.  The last kernel writes the sums to pinned host memory itself: a
+// copy of 64 bytes behind it took as long as both kernels' launches.
+int volume_into(kst_handle* h, double* part, double out[6]) {
+    static_assert(kScratchDoubles == (size_t)VOL_BLOCKS_MAX * VOL_Q * 2, "the partials of the largest grid");
     const int nb = volume_partials(h->ntiles);
-    if (kScratchDoubles > cap)
-        return set_err(h, KST_ERR_CONFIG, "volume: the partial-sum buffer holds " + std::to_string(cap) +
-                                              " doubles; " + std::to_string(kScratchDoubles) + " are needed");
     hipLaunchKernelGGL(volume_kernel, dim3(nb), dim3(VOL_NT), 0, h->stream, h->d_args, h->d_par, part);
     hipLaunchKernelGGL(volume_final_kernel, dim3(1), dim3(VOL_NT), 0, h->stream, h->d_args, part, h->vol_sum);
     HIPCHK(h, hipGetLastError());
@@ -4002,7 +4000,7 @@ int volume_into(kst_handle* h, double* part, size_t cap, double out[6]) {
 int kst_volume(kst_handle* h, double out[6]) {
     if (!h || !out) return KST_ERR_CONFIG;
     if (!h->have_state) return set_err(h, KST_ERR_STATE, "kst_set_state must come first");
-    return volume_into(h, h->vol_part, kScratchDoubles, out);
+    return volume_into(h, h->vol_part, out);
 }
 
 int kst_volume_noalloc(kst_handle* h, double out[6]) {
@@ -4014,9 +4012,7 @@ int kst_volume_noalloc(kst_handle* h, double out[6]) {
         return set_err(h, KST_ERR_CONFIG, "kst_volume_noalloc: the handle's device must be current");
     double* part = scratch_ptr(h->device);
     if (!part) return set_err(h, KST_ERR_STATE, "kst_volume_noalloc: no scratch address for this device");
-    // the volume kernels write at most VOL_BLOCKS_MAX partial groups, which is
-    // what scratch holds; volume_into refuses a buffer smaller than that
-    return volume_into(h, part, kScratchDoubles, out);
+    return volume_into(h, part, out);
 }
 
 int kst_get_output(kst_handle* h, int32_t max_tiles, double* fields, int32_t* tiles, int32_t* n_tiles) {
