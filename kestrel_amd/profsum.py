@@ -14,7 +14,9 @@ in one pass; bench.py runs the same steps twice (timed, then profiled with HIP
 events), so the 2 x N longest dispatches (largest FETCH_SIZE for `pmc`) are
 the productive ones, and their mean is set beside bench.py's event mean.  The
 rest are launches that only checked the control block and returned (after a
-rejected check or at the end of a run).
+rejected check or at the end of a run).  `trace` sets the last stage's launches
+that take side work (the timed pass of a small morphodynamic run) apart from
+those without (the profiled pass).
 """
 from __future__ import annotations
 
@@ -25,8 +27,9 @@ import sqlite3
 import statistics
 
 
-def short_name(name: str) -> str:
-    """'void kst::stage_kernel<2, true, 1>(kst::Dev, kst::Params)' -> 'stage_kernel<2>'."""
+def short_name(name: str, sides: bool = False) -> str:
+    """'void kst::stage_kernel<2, true, 1>(kst::Dev, kst::Params)' -> 'stage_kernel<2>';
+    with `sides` a last stage's launch with side work -> 'stage_kernel<4> + side work'."""
     n = name.split("(")[0].replace("void ", "").strip()
     n = n.split("::")[-1]
     # the step control and the activation as bench.py's profiled pass launches
@@ -35,7 +38,11 @@ def short_name(name: str) -> str:
     if n in ctl:
         return ctl[n]
     m = re.match(r"(\w+)<(\d+)", n)
-    return f"{m.group(1)}<{m.group(2)}>" if m else n
+    if not m:
+        return n
+    args = n[n.index("<") + 1:].rstrip(">").split(", ")
+    side = sides and m.group(1) == "stage_kernel" and args[6:] == ["true"]
+    return f"{m.group(1)}<{m.group(2)}>" + (" + side work" if side else "")
 
 
 def bench_line(path: str) -> dict:
@@ -71,10 +78,14 @@ def trace_table(db: str, bench: dict | None = None) -> str:
     rows = con.execute("select name, start, end from kernels").fetchall()
     dur: dict = {}
     for n, s, e in rows:
-        dur.setdefault(short_name(n), []).append((e - s) / 1e3)
+        dur.setdefault(short_name(n, sides=True), []).append((e - s) / 1e3)
     total = sum(sum(v) for v in dur.values())
     prod = productive_counts(bench) if bench else {}
     ev = bench_means(bench) if bench else {}
+    for k in [k for k in dur if k.endswith(" + side work")]:   # one pass's launches each
+        base = k.split(" + ")[0]
+        if base in prod:
+            prod[k] = prod[base] = prod[base] // 2
     out = ["| kernel | dispatches | total ms | share | mean us (all) | productive | mean us (productive) | event mean us |",
            "|---|---|---|---|---|---|---|---|"]
     for k, v in sorted(dur.items(), key=lambda kv: -sum(kv[1])):
