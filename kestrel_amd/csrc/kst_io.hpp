@@ -4,10 +4,9 @@
 // are, once, through the device's staging (Stage), and these kernels rearrange
 // them and fill every buffer that starts from the state, a chunk of the
 // row-major arrays -- elements [g0, g0 + n), in the staging from 0 on -- at a
-// time.  They are
-// bound by HBM (a 2048 x 2048 set-up writes 1.1 GB in 0.3 ms); rearranged on
-// one host thread, with each buffer filled by a copy of its own, the same
-// set-up took 134 ms and reading the state 141 ms.  Included by
+// time.  They are bound by HBM (a 2048 x 2048 set-up writes 1.1 GB in 0.3 ms);
+// rearranged on one host thread, with each buffer filled by a copy of its own,
+// the same set-up took 134 ms and reading the state 141 ms.  Included by
 // kst_step.hip.
 #pragma once
 

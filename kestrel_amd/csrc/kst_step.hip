@@ -1,14 +1,16 @@
 // kst_step.hip -- gfx950 kernels of the finite-volume step.
 //
 // One RK stage of the hydraulic operator is ONE kernel: a workgroup takes a
-// 16x16 sub-block of an active tile, stages the stage state (plus a 2-cell
-// halo strip on each side) in LDS, and fuses in one pass what the reference
-// does in seven tile sweeps plus the stage update
+// sub-block of an active tile (up to 256 cells, or 16 x 4 where few tiles are
+// active), stages the stage state (plus a 2-cell halo strip on each side) in
+// LDS, and fuses in one pass what the reference does in seven tile sweeps plus
+// the stage update
 // (src/HydraulicRHS.f90:64-136 and src/TimeStepper.f90:333-527):
 //   limited slopes -> MUSCL faces -> CorrectSlopes -> desingularisation ->
 //   central-upwind fluxes + CFL -> flux divergence + sources -> SSP-RK stage.
 // Data in HBM is tile-major SoA: field f of cell (i,j) of tile t sits at
-// f*FS + t*NC + j*nx + i, so a sub-block row is 128 contiguous bytes.
+// f*FS + t*NC + j*nx + i, so a sub-block row is contiguous (128 bytes of 16
+// cells).
 //
 // Control (accept/reject, dt, tile activation) lives in device memory; the
 // host enqueues whole steps and only reads back status every few steps.
@@ -383,7 +385,7 @@ __device__ __forceinline__ T lim(int rt, T a, T b) {
 // BY = B/4: 16 x 4.  The region is the sub-block and 2 cells on every side.
 // ONED: a 1D grid (one row of cells), which also keeps the conserved rhoHnv
 // for its x-face reconstruction.
-// The fluxes of a 16 x 16 sub-block take the place of what the face pass
+// The fluxes of a wide sub-block take the place of what the face pass
 // reads (ALIAS: each thread holds its faces' fluxes over the barrier between
 // the two), which leaves room for four workgroups on a CU instead of three
 // (48 -> 28 KB a workgroup); the 16 x 4 shape keeps them apart, since its
@@ -1753,14 +1755,22 @@ __device__ __forceinline__ bool stage_body(const DevT& d, const Params& p, Smem&
 // The grid is sized for the active set the host last saw (with room to
 // grow); a block whose share of the list holds more items takes them in turn.
 // The wide shape is bound by HBM (3.0-4.0 TB/s, 60-78% of a large copy's
-// rate), VALU issue (45-57% busy) and latency together: it is held to 128
+// rate), VALU issue (45-47% busy) and latency together: it is held to 128
 // VGPRs (4 waves a SIMD) by what phase B does not hold in registers -- the
 // drag closures are evaluated before it, the owned cell is read again after
 // it -- and, where a region carries no solids, by what it does not compute.
 // Plain 2048^2 (1.63 M active cells, clear water), stages 1..4: 157, 161,
 // 159, 164 us at 3 waves a SIMD with every array read, 129, 148, 134, 136 us
-// now (stage 2 spills 9 registers; at 3 waves without spills it took 160 us).  Not reading the face and cell bt of a flat bed (8 of 31 words a
-// cell) by itself changed nothing at 3 waves.
+// now (stage 2 spills 9 registers; at 3 waves without spills it took 160 us).
+// Not reading the face and cell bt of a flat bed (8 of 31 words a cell) by
+// itself changed nothing at 3 waves.  Its price is a workgroup's latency (one
+// barrier more, the owned cell's topography read behind the face pass), which
+// shows where a launch holds no more workgroups than three waves a SIMD would
+// (768) over a changing bed with solids: 5 to 20% a launch, and 1 to 6% of a
+// morphodynamic step of 130 to 700 sub-blocks (32 x 32 tiles: 36 tiles 185
+// against 179 us an attempt, 100 tiles 231 against 224; from 196 tiles on 13%
+// faster).  Held to 3 waves a SIMD it would gain back 1 to 2% there and lose 3
+// to 13% from 800 sub-blocks on.
 //
 // SIDE (16 x 4, STAGE 4): nstage workgroups do the stage.  The last stage of a
 // Strang step's operators does not fill the chip then and nothing waits for it
@@ -2676,13 +2686,13 @@ struct Batch {
     const Dev* dev;
     const Params* par;
     const int* on;        // slot holds a scenario
-    int* off;             // [nslot + 1] first work item of each slot (16 x 16 sub-blocks)
+    int* off;             // [nslot + 1] first work item of each slot (wide sub-blocks, Params::spt a tile)
     int* status;          // [nslot] the scenario's status after each iteration
     int nslot;
     const Dev* dev2;      // the second hydraulic operator of each slot (morphodynamic slots)
-    int* off2;            // [nslot + 1] as off, morphodynamic slots only
+    int* off2;            // [nslot + 1] 16 x 16 sub-blocks of the morphodynamic slots (the M stages')
     int* off3;            // [nslot + 1] (tile, part) items of the morphodynamic slots
-    int* off4;            // [nslot + 1] as off (the stage kernels' sub-blocks), morphodynamic slots only
+    int* off4;            // [nslot + 1] as off, morphodynamic slots only (their second operator's stages)
 };
 
 constexpr int BATCH_PLAN_THREADS = 1024;
@@ -2706,11 +2716,10 @@ __global__ __launch_bounds__(ACT_NT) void batch_control_kernel(Batch bt) {
     if (threadIdx.x == 0) bt.status[s] = d.ctrl->status;
 }
 
-// Work list of the iteration: the running slots' active sub-blocks.
-// The iteration's work lists (exclusive prefix sums over the slots): off,
-// the running slots' sub-blocks; with morphodynamic slots (lists > 1) also
+// The iteration's work lists (exclusive prefix sums over the slots): off, the
+// running slots' wide sub-blocks; with morphodynamic slots (lists > 1) also
 // theirs alone for the morphodynamic kernels (off2, 16 x 16) and the second
-// operator's stages (off4), and off3, their (tile, part) items.
+// operator's stages (off4, wide), and off3, their (tile, part) items.
 __global__ __launch_bounds__(BATCH_PLAN_THREADS) void batch_plan_kernel(Batch bt, int lists) {
     __shared__ int sc[BATCH_PLAN_THREADS / 64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -2772,7 +2781,7 @@ __device__ __forceinline__ int batch_slot(const int* off, int nslot, int w) {
 // One RK stage over the work list.  The grid is a multiple of 8 blocks that
 // stay resident and walk the list; XCD x (blocks x, x+8, ...) takes the x-th
 // contiguous eighth of it, so neighbouring sub-blocks share an L2.
-// second: the second hydraulic operator of the morphodynamic slots (dev2, off2)
+// second: the second hydraulic operator of the morphodynamic slots (dev2, off4)
 template <int STAGE, bool VISC, int LIM, bool MIX>
 __global__ __launch_bounds__(STAGE_NT, 4) void batch_stage_kernel(Batch bt, int second) {
     __shared__ SmemT<VISC ? 7 : 5, MIX> s;
@@ -2849,11 +2858,11 @@ struct kst_handle {
     // kGraphIters whole iterations, per (grid cap, sub-block shape)
     std::vector<std::pair<long long, hipGraphExec_t>> graphs;
     int fixed_cap = 0;                   // kst_set_grid_cap (0: from the active set)
-    int resident = 0;                    // 16 x 16 stage-kernel blocks resident on the device at once
+    int resident = 0;                    // wide stage-kernel blocks resident on the device at once
     bool autotune = false;               // kst_autotune: choices per active-set bucket
     struct Tune {
         int small;                       // 16 x 4 sub-blocks
-        int grid;                        // launch-grid limit of the 16 x 16 shape (0: the cap's grid)
+        int grid;                        // launch-grid limit of the wide shape (0: the cap's grid)
         double us[4];                    // stage-1 launch time of each candidate (0: not tried)
     };
     std::map<int, Tune> tuned;           // bucket (active tiles, rounded up to a power of two)
@@ -2867,9 +2876,9 @@ struct kst_handle {
     long long prof_n[KW_N] = {};
 };
 
-// Device scratch of kst_volume_noalloc: the partial sums of the volume
-// kernels (VOL_BLOCKS_MAX groups), the same layout as the handle's vol_part.  One copy per GPU, held until the
-// process ends; every call on that GPU shares it.  In host code the array's
+// Device scratch of kst_volume_noalloc: the partial sums of the volume kernels
+// (VOL_BLOCKS_MAX groups), the same layout as the handle's vol_part.  One copy
+// per GPU, held until the process ends; every call on that GPU shares it.  In host code the array's
 // name stands for no device address: its address on each device comes from
 // hipGetSymbolAddress (scratch_ptr), taken once per device in kst_create.
 constexpr size_t kScratchDoubles = (size_t)VOL_BLOCKS_MAX * VOL_Q * 2;
@@ -3212,7 +3221,14 @@ const StageSet& stage_set_of(bool visc, int limiter) {
 // workgroups, each with one face per thread and its cells and halo loaded in
 // one round, so a stage that cannot fill the chip has a shorter critical
 // path (16 x 8 measured between the two); the morphodynamic kernels use the
-// same shape then.  FP64 only.
+// same shape then.  FP64 only.  The line, in sub-blocks of 16 x 16 (four of 16
+// x 4), lies where the small shape has lost most of its lead: us a step, wide
+// / small, at 100, 144 and 196 of them (periodic grids, every tile active):
+// flat beds in tiles of 32 61.5 / 54.8, 62.4 / 62.8, 64.3 / 85.7; over a
+// changed bed 70.7 / 59.8, 71.5 / 68.0, 73.7 / 95.3; morphodynamic 174 / 140,
+// 181 / 156, 191 / 232; in tiles of 50 at 64, 96, 144, 256: flat 61.3 / 49.6,
+// 60.4 / 53.3, 61.4 / 59.2, 63.9 / 97.5, morphodynamic 169 / 122, 167 / 133,
+// 170 / 147, 182 / 247.
 constexpr int BY_SMALL = B / 4;
 constexpr int SMALL_WORK = 128;       // sub-blocks of 16 x 16 below which the small shape is used
 
@@ -3352,9 +3368,9 @@ int ensure_graph(kst_handle* h, bool small, int cap, int grid_limit, hipGraphExe
 
 // Autotuner (kst_autotune).  For the active set of the coming launches it
 // times the first RK stage kernel -- a launch that reads u^n and writes only
-// the RHS buffer, the CFL minimum and the edge flags, all of which the
-// iteration's own stage 1 rewrites from the same u^n -- in each candidate
-// launch shape: 16 x 16 sub-blocks on the cap's grid, the same capped at the
+// the RHS buffer and the CFL minimum, which the iteration's own stage 1
+// rewrites from the same u^n -- in each candidate launch shape: the wide
+// sub-blocks (wide_shape) on the cap's grid, the same capped at the
 // resident blocks of the device (each block taking further items in turn),
 // at twice that, and (FP64) 16 x 4 sub-blocks.  The control block is saved
 // before the trials and restored after them, so the run is unchanged.  The
@@ -3593,7 +3609,7 @@ int kst_create(const kst_config* cfg, kst_handle** out) {
         return KST_ERR_HIP;
     }
     {
-        // blocks of the 16 x 16 stage kernel the device holds at once (the
+        // blocks of the wide stage kernel the device holds at once (the
         // autotuner's resident grid)
         int cus = 0, per = 0;
         if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess ||

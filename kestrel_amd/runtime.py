@@ -276,9 +276,13 @@ class Stepper:
                                         gr.ctypes.data_as(i32p), _ptr(us))
         if k < 0:
             raise KestrelError(k, "kst_autotune_choices")
-        names = ("16x16 default grid", "16x16 resident grid", "16x16 twice resident", "16x4")
+        w, h = ctypes.c_int32(), ctypes.c_int32()   # the wide sub-block in these tiles
+        self._check(self.L.kst_stage_sub_block(self.cfg.nx_per_tile, self.cfg.ny_per_tile, ctypes.byref(w),
+                                               ctypes.byref(h)) if k else 0)
+        wide = f"{w.value}x{h.value}"
+        names = (f"{wide} default grid", f"{wide} resident grid", f"{wide} twice resident", "16x4")
         return [{"active_tiles_bucket": int(b[q]),
-                 "shape": "16x4" if sm[q] else ("16x16" if gr[q] == 0 else f"16x16 grid {int(gr[q])}"),
+                 "shape": "16x4" if sm[q] else (wide if gr[q] == 0 else f"{wide} grid {int(gr[q])}"),
                  "stage1_us": {names[c]: round(float(us[q, c]), 2) for c in range(4) if us[q, c] > 0}}
                 for q in range(k)]
 
