@@ -118,3 +118,39 @@ def test_admission_counts_what_a_scenario_holds(gpu, kind, n, tile):
         g.close()
     counted = serving.device_bytes(wl.cfg)
     assert held <= counted <= 1.3 * held + 4 * MB, (held, counted)
+
+
+def test_staging_shared_by_threads(gpu):
+    """Two threads with a handle each, one of whose arrays make the shared
+    staging grow: each reads back what it set, whatever the other does."""
+    import threading
+
+    from kestrel_amd import scenario as S
+    from kestrel_amd.runtime import Stepper
+    failed = []
+
+    def work(tiles, tile, seed):
+        cfg = C.default_config(tiles, tiles, tile, tile)
+        C.hydraulic_only(cfg)
+        cfg.bc = C.BC_PERIODIC
+        C.derive(cfg)
+        rng = np.random.default_rng(seed)
+        shape = (cfg.NY, cfg.NX)
+        g = Stepper(cfg)
+        for k in range(12):
+            b0v = rng.standard_normal((cfg.NY + 1, cfg.NX + 1))
+            f = [rng.standard_normal(shape) for _ in range(5)]
+            g.set_topography(b0v)
+            g.set_state(S.InitialState(*f[:4], np.ones(cfg.ntiles, np.uint8), f[4]))
+            st = g.state()
+            ok = all(np.array_equal(st[n], a) for n, a in zip(("w", "rhoHnu", "rhoHnv", "Hnpsi"), f))
+            if not (ok and np.array_equal(g.maxima()[0], f[4])):
+                failed.append((tiles, k))
+        g.close()
+
+    threads = [threading.Thread(target=work, args=a) for a in ((5, 31, 1), (40, 37, 2))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
